@@ -34,19 +34,18 @@ extern "C" {
  * Forward: K = exp(-gamma * sqdist(X, Y)).
  * Replaces the pybind entry `rbf_forward(Tensor X, Tensor Y, double gamma)
  * -> Tensor` of the reference (cases/rbf/kernels/rbf_forward.cu:94-120),
- * which cases/rbf/op.py:30 calls.  N, M >= 0, D >= 1.  The fp32 MFMA path
- * runs for D == 64 with 16-byte aligned X, Y, K and M % 4 == 0; every other
- * shape uses a generic HIP kernel.
+ * which cases/rbf/op.py:30 calls.  N, M >= 0, D >= 1, any alignment.
+ * Distances come from norms and products, each product from three-term bf16
+ * splits of the fp32 rows; with D != 64, tiles holding a row with
+ * gamma |x|^2 > 4 (or a norm that is not finite, at any D) sum the squared
+ * differences directly.
  */
 int rbf_forward_f32(const float* X, const float* Y, float* K, int64_t N,
                     int64_t M, int64_t D, float gamma, hipStream_t stream);
 
 /*
- * Bytes of device workspace rbf_backward_f32 needs for these sizes: the
- * per-region partial sums of dX and dY of the tile kernels, or, for shapes
- * only the generic kernels take (D != 64, N or M past the tile limit), the
- * partial sums of the slices their walks are cut into.  0 means no
- * workspace is needed.
+ * Bytes of device workspace rbf_backward_f32 uses for these sizes: partial
+ * sums of dX and dY.  0 means no workspace is needed.
  */
 size_t rbf_backward_workspace_bytes(int64_t N, int64_t M, int64_t D);
 
@@ -56,9 +55,10 @@ size_t rbf_backward_workspace_bytes(int64_t N, int64_t M, int64_t D);
  * Tensor K, double gamma) -> [dX, dY]` of the reference
  * (cases/rbf/kernels/rbf_backward.cu:59-88), which cases/rbf/op.py:38 calls.
  * `workspace` must hold rbf_backward_workspace_bytes(N, M, D) bytes (it may
- * be NULL when that is 0).  A call that takes the generic kernels also runs
- * with a shorter or NULL workspace, its walks then unsliced (slower, and
- * rounded differently).  dX and dY are fully overwritten.
+ * be NULL when that is 0).  A call with D != 64, or with X, Y, dX or dY not
+ * 16-byte aligned, also runs with a shorter or NULL workspace, on generic
+ * kernels (slower, and rounded differently).  dX and dY are fully
+ * overwritten.
  */
 int rbf_backward_f32(const float* X, const float* Y, const float* dK,
                      const float* K, float* dX, float* dY, int64_t N,
@@ -66,20 +66,20 @@ int rbf_backward_f32(const float* X, const float* Y, const float* dK,
                      size_t workspace_bytes, hipStream_t stream);
 
 /*
- * Backward without a caller workspace and without any allocation: for the
- * tile kernels the same kernels and results as rbf_backward_f32 (bit for
- * bit), with the region
+ * Backward without a caller workspace and without any allocation: for calls
+ * that require a workspace the same kernels and results as rbf_backward_f32
+ * (bit for bit), with the
  * partials kept in a scratch array compiled into the library (64 MiB per
  * GPU, held from the first call on that GPU until the process ends).  No
  * counterpart in the reference: it is for callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops,
- * harnesses that forbid hipMalloc).  Calls that take the tile kernels
+ * harnesses that forbid hipMalloc).  Calls that require a workspace
  * (D = 64, 16-byte aligned X, Y, dX, dY) and whose
  * rbf_backward_workspace_bytes(N, M, D) exceeds
  * rbf_backward_noalloc_max_bytes() are rejected with NL2K_ERR_WORKSPACE
  * before any HIP call (N = M = 4096, D = 64 needs 34 MB and fits; 8192 does
- * not); calls that take the generic kernels use no scratch (their walks
- * unsliced) and run at any size.  Every call on one GPU shares that GPU's scratch, so calls that
+ * not); the others use no scratch (generic kernels, their walks unsliced)
+ * and run at any size.  Every call on one GPU shares that GPU's scratch, so calls that
  * overlap in time on one GPU (different streams, or threads) race and must
  * be serialised by the caller; a call needs no initial scratch contents.
  */

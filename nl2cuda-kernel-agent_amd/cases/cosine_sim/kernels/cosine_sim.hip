@@ -12,21 +12,21 @@
 // cosine_sim.cu:63-102, uses s_a in place of 1/|a| in the second term; the
 // two agree to within eps / |a|.)
 //
-// Design (D == 64 fast path), on the RBF tile engines of
-// csrc/pairwise_d64.h:
-//  * Forward: the inverse norms are folded into the MFMA operands -- each
-//    wave scales its X rows in registers when it loads them, and Y rows are
-//    scaled as they are staged into LDS -- so the epilogue is a plain store
-//    of the accumulators (no VALU work beside the matrix cores).  The same
-//    launch writes inv_a / inv_b for the backward.
-//  * Backward: one pass over dS (W = dS, no product), both contractions
-//    dS . bh and dS^T . ah as region partials (the staged X / Y rows scaled
-//    by inv_a / inv_b); cos_bwd_reduce_kernel sums the partials and applies
-//    the projection, one 16-lane group per row.
-//  * Other feature widths and misaligned pointers use the tiled SIMT kernels
-//    of csrc/pairwise_generic.h (rows scaled by their inverse norms as they
+// Design:
+//  * Forward: on bf16 splits of the fp32 rows (csrc/pairwise_split.h), at any
+//    D and alignment.  A tile's rows are read once for their norms and again,
+//    from L2, to be scaled by their inverse norms, split and multiplied, so
+//    the epilogue is a plain store of the accumulators.  The same launch
+//    writes inv_a / inv_b for the backward.
+//  * Backward: one pass over dS (W = dS, no product) per 64 features, both
+//    contractions dS . bh and dS^T . ah as region partials (the staged X / Y
+//    rows scaled by inv_a / inv_b), on the bf16 splits or, for small shapes
+//    at D = 64, on fp32 MFMA (csrc/pairwise_d64.h); cos_bwd_reduce_kernel sums
+//    the partials and applies the projection.
+//  * Past those kernels' index ranges the tiled SIMT kernels of
+//    csrc/pairwise_generic.h run (rows scaled by their inverse norms as they
 //    are staged), the backward's walks in slices whose partial rows the
-//    projection kernel adds in order.
+//    same reduce adds in order.
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
@@ -34,13 +34,9 @@
 #include "../../../csrc/common.h"
 #include "../../../csrc/pairwise_d64.h"
 #include "../../../csrc/pairwise_generic.h"
+#include "../../../csrc/pairwise_split.h"
 #include "cosine_sim.h"
 
-using nl2k::f32x4;
-using nl2k::load4;
-using nl2k::store4;
-using nl2k::zero4;
-using nl2k::pairwise::kD;
 
 namespace {
 
@@ -48,24 +44,12 @@ __device__ __forceinline__ float inv_norm(float sumsq, float eps) {
   return 1.f / (sqrtf(sumsq) + eps);
 }
 
-// Forward policy: rows scaled by their inverse norms before the contraction;
-// the row / column terms written out are those inverse norms.
+// Forward policy: rows scaled by their inverse norms before the contraction,
+// the inverse norms written out.
 struct CosFwdOp {
   float eps;
-  static constexpr bool kSideOut = true;
-  static constexpr bool kRowScales = true;
-  __device__ __forceinline__ float row(f32x4 (&x)[4], float sx) const {
-    const float s = inv_norm(sx, eps);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) x[q] *= s;
-    return s;
-  }
-  __device__ __forceinline__ float col(f32x4& y, float sy) const {
-    const float s = inv_norm(sy, eps);
-    y *= s;
-    return s;
-  }
-  __device__ __forceinline__ float out(float dot, float, float) const { return dot; }
+  static constexpr bool kScale = true, kDirect = false;
+  __device__ __forceinline__ float inv(float nsq) const { return inv_norm(nsq, eps); }
 };
 
 // Backward policy: W = dS, X / Y rows scaled by inv_a / inv_b, no sums.
@@ -73,54 +57,91 @@ struct CosBwdOp {
   static constexpr bool kProduct = false, kScale = true, kSums = false;
 };
 
-// Both outputs in one launch: block b < bx handles dA, the rest dB.  One
-// thread per float4 of the output, 16 threads per row (a 16-aligned lane
-// group): acc = sum of the slots, then
-//   out = s acc - (ah . acc) / |a| ah,  ah = s a.
-__global__ __launch_bounds__(256) void cos_bwd_reduce_kernel(
-    const float* __restrict__ Px, const float* __restrict__ A,
-    const float* __restrict__ inv_a, float* __restrict__ dA, int N, int sx,
-    const float* __restrict__ Py, const float* __restrict__ B,
-    const float* __restrict__ inv_b, float* __restrict__ dB, int M, int sy, int bx) {
-  const bool is_a = (int)blockIdx.x < bx;
-  const float* __restrict__ Pt = is_a ? Px : Py;
-  const float* __restrict__ V = is_a ? A : B;
-  const float* __restrict__ inv = is_a ? inv_a : inv_b;
-  float* __restrict__ out = is_a ? dA : dB;
-  const int rows = is_a ? N : M;
-  const int slots = is_a ? sx : sy;
-  const int b0 = is_a ? 0 : bx;
-  const int nb = is_a ? bx : (int)gridDim.x - bx;
-  const size_t n4 = (size_t)rows * (kD / 4);
-  const size_t stride = (size_t)rows * kD;
-  // The stride is a multiple of 16 and rows start at multiples of 16, so the
-  // 16 threads of a row are always active together.
-  for (size_t e = (size_t)(blockIdx.x - b0) * blockDim.x + threadIdx.x; e < n4;
-       e += (size_t)nb * blockDim.x) {
-    const size_t r = e / (kD / 4);
-    f32x4 a0 = zero4(), a1 = zero4(), a2 = zero4(), a3 = zero4();
+// One row: acc = sum of its partial rows, in slot order, then
+//   out = s acc - (ah . acc) / |a| ah,  ah = s a,
+// by L lanes of V features each (the sums over the row's lanes leave every
+// lane the same bits).  The first kKeep groups of a lane stay in registers
+// between the two passes; wider rows add their partials up again.
+constexpr int kKeep = 4;
+template <int V, int L>
+__device__ __forceinline__ void project_row(const float* __restrict__ P, const float* __restrict__ A,
+                                            const float* __restrict__ inv, float* __restrict__ out,
+                                            int64_t rows, int64_t r, int D, int slots, int lane) {
+  typedef float vec __attribute__((ext_vector_type(V), aligned(4)));
+  const int per = D / V;
+  const int64_t stride = rows * (int64_t)D;
+  const float* p = P + r * D;
+  const float* a = A + r * D;
+  const float sc = inv[r];
+  auto partial = [&](int e) {
+    auto at = [&](int s) { return *reinterpret_cast<const vec*>(p + s * stride + (int64_t)e * V); };
+    vec a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
     int s = 0;
     for (; s + 4 <= slots; s += 4) {
-      a0 += load4(Pt + (size_t)s * stride + 4 * e);
-      a1 += load4(Pt + (size_t)(s + 1) * stride + 4 * e);
-      a2 += load4(Pt + (size_t)(s + 2) * stride + 4 * e);
-      a3 += load4(Pt + (size_t)(s + 3) * stride + 4 * e);
+      a0 += at(s);
+      a1 += at(s + 1);
+      a2 += at(s + 2);
+      a3 += at(s + 3);
     }
-    for (; s < slots; ++s) a0 += load4(Pt + (size_t)s * stride + 4 * e);
-    const f32x4 acc = (a0 + a1) + (a2 + a3);
-    const f32x4 a = load4(V + 4 * e);
-    const float sc = inv[r];
-    const f32x4 ah = a * sc;
-    float dot = (ah[0] * acc[0] + ah[1] * acc[1]) + (ah[2] * acc[2] + ah[3] * acc[3]);
-    float nn = (a[0] * a[0] + a[1] * a[1]) + (a[2] * a[2] + a[3] * a[3]);
+    for (; s < slots; ++s) a0 += at(s);
+    return (a0 + a1) + (a2 + a3);
+  };
+  float dot = 0.f, nn = 0.f;
+  vec keep[kKeep], row[kKeep];
+  auto add = [&](const vec& acc, const vec& av) {
+    const vec ah = av * sc;
 #pragma unroll
-    for (int off = 1; off < 16; off <<= 1) {
-      dot += __shfl_xor(dot, off, 64);
-      nn += __shfl_xor(nn, off, 64);
+    for (int v = 0; v < V; ++v) {
+      dot = fmaf(ah[v], acc[v], dot);
+      nn = fmaf(av[v], av[v], nn);
     }
-    const float nrm = sqrtf(nn);
-    const float coef = nrm > 0.f ? dot / nrm : 0.f;
-    store4(out + 4 * e, sc * acc - coef * ah);
+  };
+#pragma unroll
+  for (int k = 0; k < kKeep; ++k) {
+    const int e = lane + L * k;
+    if (e < per) {
+      keep[k] = partial(e);
+      row[k] = *reinterpret_cast<const vec*>(a + (int64_t)e * V);
+      add(keep[k], row[k]);
+    }
+  }
+  for (int e = lane + L * kKeep; e < per; e += L)
+    add(partial(e), *reinterpret_cast<const vec*>(a + (int64_t)e * V));
+#pragma unroll
+  for (int off = 1; off < L; off <<= 1) {
+    dot += __shfl_xor(dot, off, 64);
+    nn += __shfl_xor(nn, off, 64);
+  }
+  const float nrm = sqrtf(nn);
+  const float coef = nrm > 0.f ? dot / nrm : 0.f;
+  auto store = [&](int e, const vec& acc, const vec& av) {
+    *reinterpret_cast<vec*>(out + r * D + (int64_t)e * V) = sc * acc - coef * (av * sc);
+  };
+#pragma unroll
+  for (int k = 0; k < kKeep; ++k)
+    if (lane + L * k < per) store(lane + L * k, keep[k], row[k]);
+  for (int e = lane + L * kKeep; e < per; e += L)
+    store(e, partial(e), *reinterpret_cast<const vec*>(a + (int64_t)e * V));
+}
+
+// Both outputs in one launch: block b < bx handles dA, the rest dB.  A row's
+// lanes stay together: every lane of a group has the same row.
+template <int V, int L>
+__global__ __launch_bounds__(256) void cos_bwd_reduce_kernel(
+    const float* __restrict__ Px, const float* __restrict__ A,
+    const float* __restrict__ inv_a, float* __restrict__ dA, int64_t N, int sx,
+    const float* __restrict__ Py, const float* __restrict__ B,
+    const float* __restrict__ inv_b, float* __restrict__ dB, int64_t M, int sy, int D, int bx) {
+  constexpr int kRows = 256 / L;
+  const int b = (int)blockIdx.x;
+  const int lane = threadIdx.x % L, g = threadIdx.x / L;
+  if (b < bx) {
+    for (int64_t r = (int64_t)b * kRows + g; r < N; r += (int64_t)bx * kRows)
+      project_row<V, L>(Px, A, inv_a, dA, N, r, D, sx, lane);
+  } else {
+    const int64_t nb = (int)gridDim.x - bx;
+    for (int64_t r = (int64_t)(b - bx) * kRows + g; r < M; r += nb * kRows)
+      project_row<V, L>(Py, B, inv_b, dB, M, r, D, sy, lane);
   }
 }
 
@@ -166,37 +187,6 @@ struct CosGenBwd {
   }
   __device__ __forceinline__ float finish(float, float, float acc) const { return acc; }
 };
-
-// out_r = s dvh_r - (vh_r . dvh_r) / |v_r| vh_r, one wave per row; dvh is
-// the sum, in slice order, of the S partial rows part[s][r][:].
-__device__ __forceinline__ float slice_sum(const float* __restrict__ part, int64_t S,
-                                           int64_t plane, int64_t e) {
-  float v = 0.f;
-  for (int64_t sl = 0; sl < S; ++sl) v += part[sl * plane + e];
-  return v;
-}
-__global__ __launch_bounds__(256) void cos_project_generic_kernel(
-    const float* __restrict__ V, const float* __restrict__ inv, const float* __restrict__ part,
-    int64_t S, float* __restrict__ out, int64_t rows, int64_t D) {
-  const int lane = threadIdx.x & 63;
-  const int64_t waves = (int64_t)gridDim.x * (blockDim.x / 64);
-  for (int64_t r = (int64_t)blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6); r < rows;
-       r += waves) {
-    const float sc = inv[r];
-    float dot = 0.f, nn = 0.f;
-    for (int64_t d = lane; d < D; d += 64) {
-      const float v = V[r * D + d];
-      dot = fmaf(v * sc, slice_sum(part, S, rows * D, r * D + d), dot);
-      nn = fmaf(v, v, nn);
-    }
-    dot = nl2k::wave_sum(dot);
-    nn = nl2k::wave_sum(nn);
-    const float nrm = sqrtf(nn);
-    const float coef = nrm > 0.f ? dot / nrm : 0.f;
-    for (int64_t d = lane; d < D; d += 64)
-      out[r * D + d] = sc * slice_sum(part, S, rows * D, r * D + d) - coef * (V[r * D + d] * sc);
-  }
-}
 
 // Floats of the generic backward's partial rows: S slices a side when
 // `sliced`, one otherwise.
@@ -245,9 +235,31 @@ int fill_zero(float* p, size_t count, hipStream_t stream) {
   return nl2k::check_launch("cosine_sim fill");
 }
 
-bool fast_backward(int64_t D, const void* A, const void* B, const void* dA, const void* dB) {
-  return D == kD && nl2k::aligned16(A) && nl2k::aligned16(B) && nl2k::aligned16(dA) &&
-         nl2k::aligned16(dB);
+// Sums the partial rows (sx of each row of A, sy of B) into dA and dB.
+int reduce(const float* px, const float* py, int64_t sx, int64_t sy, const float* A,
+           const float* B, const float* inv_a, const float* inv_b, float* dA, float* dB,
+           int64_t N, int64_t M, int64_t D, hipStream_t stream, const char* who) {
+  const bool vec = D % 4 == 0;
+  const bool wide = D > (vec ? 64 : 16);  // a wave per row, else 16 lanes
+  auto* kernel = vec ? (wide ? &cos_bwd_reduce_kernel<4, 64> : &cos_bwd_reduce_kernel<4, 16>)
+                     : (wide ? &cos_bwd_reduce_kernel<1, 64> : &cos_bwd_reduce_kernel<1, 16>);
+  const int bx = grid_for(N, wide ? 4 : 16, 2048), by = grid_for(M, wide ? 4 : 16, 2048);
+  hipLaunchKernelGGL(kernel, dim3(bx + by), dim3(256), 0, stream, px, A, inv_a, dA, N, (int)sx,
+                     py, B, inv_b, dB, M, (int)sy, (int)D, bx);
+  return nl2k::check_launch(who);
+}
+
+// What cosine_sim_backward_workspace_bytes reports, in floats: callers hold
+// buffers of this size, and the split backward is cut so that its partials
+// fit.  At D = 64 it is the fp32 regions' (pairwise_d64.h) or one partial row
+// for each row, else what the generic kernels' slices or the split backward
+// use.
+size_t workspace_floats(int64_t N, int64_t M, int64_t D) {
+  if (N == 0 || M == 0) return 0;
+  const nl2k::pairwise::BwdPlan p = nl2k::pairwise::plan_backward(N, M, D, false);
+  if (p.fast) return std::max(p.ws_floats, generic_ws_floats(N, M, D, false));
+  return std::max(generic_ws_floats(N, M, D, true),
+                  nl2k::pairwise::split_floats(N, M, D, false));
 }
 
 }  // namespace
@@ -271,16 +283,10 @@ int cosine_sim_forward_f32(const float* A, const float* B, float* S, float* inv_
     if (st) return st;
     return launch_norms(B, inv_b, M, D, eps, stream);
   }
-  nl2k::pairwise::FwdPlan fp;
-  if (D == kD && nl2k::aligned16(A) && nl2k::aligned16(B) &&
-      nl2k::pairwise::plan_forward(N, M, fp)) {
-    const int vec_store = (M % 4 == 0) && nl2k::aligned16(S);
-    auto* kernel = fp.ib == 2 ? &nl2k::pairwise::pair_fwd_d64_kernel<CosFwdOp, 2>
-                              : &nl2k::pairwise::pair_fwd_d64_kernel<CosFwdOp, 4>;
-    hipLaunchKernelGGL(kernel, dim3(fp.n_wg), dim3(256), 0, stream, A, B, S, (int)N, (int)M,
-                       CosFwdOp{eps}, fp.n_jt, fp.n_units, fp.upw, vec_store, inv_a, inv_b);
-    return nl2k::check_launch(who);
-  }
+  const nl2k::pairwise::SplitFwdPlan fp = nl2k::pairwise::plan_split_forward(N, M, D);
+  if (fp.n_jt > 0)
+    return nl2k::pairwise::launch_fwd_split(fp, A, B, S, N, M, D, CosFwdOp{eps}, inv_a, inv_b,
+                                            stream, who);
   st = launch_norms(A, inv_a, N, D, eps, stream);
   if (st) return st;
   st = launch_norms(B, inv_b, M, D, eps, stream);
@@ -295,13 +301,7 @@ int cosine_sim_forward_f32(const float* A, const float* B, float* S, float* inv_
 
 size_t cosine_sim_backward_workspace_bytes(int64_t N, int64_t M, int64_t D) {
   if (validate_sizes(N, M, D, "cosine_sim_backward_workspace_bytes")) return 0;
-  if (N == 0 || M == 0) return 0;
-  const nl2k::pairwise::BwdPlan p = nl2k::pairwise::plan_backward(N, M, D, false);
-  const size_t fast = p.fast ? p.ws_floats * sizeof(float) : 0;
-  // The generic kernels' partial rows: [S][N][D] and [S][M][D] for the
-  // slices of shapes the tile path never takes; one slice a side (the
-  // walks whole) otherwise, which a misaligned call of a tile shape uses.
-  return std::max(fast, generic_ws_floats(N, M, D, !p.fast) * sizeof(float));
+  return workspace_floats(N, M, D) * sizeof(float);
 }
 
 int cosine_sim_backward_f32(const float* A, const float* B, const float* inv_a,
@@ -318,7 +318,7 @@ int cosine_sim_backward_f32(const float* A, const float* B, const float* inv_a,
   if (M == 0) return fill_zero(dA, (size_t)(N * D), stream);
   if (N == 0) return fill_zero(dB, (size_t)(M * D), stream);
   if (!dS) return nl2k::fail(NL2K_ERR_NULL, "%s: dS must be non-null", who);
-  const size_t need = cosine_sim_backward_workspace_bytes(N, M, D);
+  const size_t floats = workspace_floats(N, M, D), need = floats * sizeof(float);
   if (workspace == nullptr || workspace_bytes < need)
     return nl2k::fail(NL2K_ERR_WORKSPACE, "%s: workspace of %zu bytes required, got %zu", who,
                       need, workspace ? workspace_bytes : (size_t)0);
@@ -326,18 +326,20 @@ int cosine_sim_backward_f32(const float* A, const float* B, const float* inv_a,
     return nl2k::fail(NL2K_ERR_ALIGN, "%s: workspace must be 16-byte aligned", who);
   float* ws = static_cast<float*>(workspace);
 
-  const nl2k::pairwise::BwdPlan p = nl2k::pairwise::plan_backward(N, M, D, false);
-  if (p.fast && fast_backward(D, A, B, dA, dB)) {
-    const bool vec_nm = (M % 4 == 0) && nl2k::aligned16(dS);
-    nl2k::pairwise::launch_bwd_tiles<CosBwdOp>(p, A, B, dS, nullptr, ws, (int)N, (int)M, vec_nm,
-                                               inv_a, inv_b, stream);
-    st = nl2k::check_launch(who);
-    if (st) return st;
-    const int bx = grid_for(N * (kD / 4), 256, 2048);
-    const int by = grid_for(M * (kD / 4), 256, 2048);
-    hipLaunchKernelGGL(cos_bwd_reduce_kernel, dim3(bx + by), dim3(256), 0, stream, ws + p.px, A,
-                       inv_a, dA, (int)N, p.nRJ, ws + p.py, B, inv_b, dB, (int)M, p.nRI, bx);
-    return nl2k::check_launch("cosine_sim_backward_f32 (reduce)");
+  const nl2k::pairwise::BwdPlan rp = nl2k::pairwise::plan_backward(N, M, D, false);
+  if (nl2k::pairwise::takes_regions(rp, M, A, B, dS, dS)) {
+    st = nl2k::pairwise::launch_bwd_regions<CosBwdOp>(rp, A, B, dS, nullptr, ws, N, M, inv_a,
+                                                      inv_b, stream, who);
+    return st ? st : reduce(ws + rp.px, ws + rp.py, rp.nRJ, rp.nRI, A, B, inv_a, inv_b, dA, dB, N,
+                            M, D, stream, who);
+  }
+  const nl2k::pairwise::SplitBwdPlan p =
+      nl2k::pairwise::plan_split_backward(N, M, D, false, floats);
+  if (p.ok) {
+    st = nl2k::pairwise::launch_bwd_split<CosBwdOp>(p, A, B, dS, nullptr, ws, N, M, D, inv_a,
+                                                    inv_b, stream, who);
+    return st ? st : reduce(ws + p.px, ws + p.py, p.nRJ, p.nRI, A, B, inv_a, inv_b, dA, dB, N, M,
+                            D, stream, who);
   }
 
   // generic kernels: the walks in slices when the workspace holds their
@@ -367,13 +369,8 @@ int cosine_sim_backward_f32(const float* A, const float* B, const float* inv_a,
                      gy.chunk, op);
   st = nl2k::check_launch("cosine_sim_backward_f32 (generic dB)");
   if (st) return st;
-  hipLaunchKernelGGL(cos_project_generic_kernel, dim3(grid_for(N, 4, 1 << 16)), dim3(256), 0,
-                     stream, A, inv_a, dah, gx.s, dA, N, D);
-  st = nl2k::check_launch("cosine_sim_backward_f32 (generic project A)");
-  if (st) return st;
-  hipLaunchKernelGGL(cos_project_generic_kernel, dim3(grid_for(M, 4, 1 << 16)), dim3(256), 0,
-                     stream, B, inv_b, dbh, gy.s, dB, M, D);
-  return nl2k::check_launch("cosine_sim_backward_f32 (generic project B)");
+  return reduce(dah, dbh, gx.s, gy.s, A, B, inv_a, inv_b, dA, dB, N, M, D, stream,
+                "cosine_sim_backward_f32 (generic reduce)");
 }
 
 }  // extern "C"

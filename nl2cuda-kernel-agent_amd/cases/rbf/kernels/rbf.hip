@@ -7,35 +7,22 @@
 //   dX[i] = -2 gamma * sum_j W[i,j] (X[i] - Y[j])
 //   dY[j] = -2 gamma * sum_i W[i,j] (Y[j] - X[i])
 //
-// Design (D == 64 fast path):
+// Design:
 //  * Forward: K[i,j] = exp2(min(2 kappa x_i.y_j - kappa (|x_i|^2 + |y_j|^2), 0))
-//    with kappa = gamma log2(e).  The cross term runs on fp32 MFMA
-//    (v_mfma_f32_16x16x4_f32).  Work unit = 256 rows x 64 columns of K; a
-//    workgroup of four waves walks a contiguous range of units.  Each wave
-//    keeps its 64 X rows in MFMA operand registers (with their norms) for as
-//    long as the row block lasts, and the unit's 64 Y rows are staged once
-//    per workgroup in LDS (double buffered, norms alongside) while the
-//    previous unit runs on the matrix cores.  The contraction index is
-//    permuted identically for both operands so every lane moves 16
-//    contiguous bytes per load.  The exp epilogue runs from the accumulators
-//    and each lane writes 4 consecutive K entries of a row (16-byte stores).
-//  * Backward: one pass over dK and K.  A workgroup (8 waves) owns a region
-//    of R x R entries of W = dK o K (R = 256 at N = M = 4096, one region per
-//    CU) and walks it in 64x64 tiles.  Waves 4-7 only stage: they load dK and
-//    K three tiles ahead into registers, form W into the LDS tile buffer of
-//    the next tile, and stage the next 64-row X chunk (transposed).  Waves
-//    0-3 only compute: per tile both contractions W . Y (rows, accumulated
-//    over the region's columns and flushed per 64-row chunk) and W^T . X
-//    (columns, accumulated over the whole region) on fp32 MFMA, with the row
-//    and column sums of W taken from the same operand registers.  Each region
-//    writes raw partial contractions and partial sums to its workspace slot;
-//    rbf_bwd_reduce_kernel sums the slots and applies
+//    with kappa = gamma log2(e), on bf16 splits of the fp32 rows
+//    (csrc/pairwise_split.h), at any D and alignment.  Tiles whose distances
+//    that form would round too coarsely (norm_max below) sum the squared
+//    differences directly, on SIMT tiles.
+//  * Backward: one pass over dK and K per 64 features.  Workgroups own
+//    regions of W = dK o K and write raw partial contractions W . Y and
+//    W^T . X and partial row and column sums of W to workspace slots, on the
+//    bf16 splits or, for small shapes at D = 64, on fp32 MFMA
+//    (csrc/pairwise_d64.h); rbf_bwd_reduce_kernel sums the slots and applies
 //    dX = -2 gamma (rowsum(W) X - W Y), dY = -2 gamma (colsum(W) Y - W^T X).
-//  * Other feature widths and misaligned pointers use tiled SIMT kernels:
-//    64 x 64 tiles staged through LDS, the forward summing the squared
-//    differences directly, the backward forming W in LDS and walking it in
-//    slices whose partial sums a reduce kernel adds in order (unsplit when
-//    the caller passes no workspace for them).
+//  * Without a workspace, or past the kernels' index ranges, tiled SIMT
+//    kernels run: W formed in LDS and walked in slices whose partial sums a
+//    reduce kernel adds in order (unsplit when the caller passes no workspace
+//    for them).
 #include <algorithm>
 #include <atomic>
 #include <cmath>
@@ -44,32 +31,44 @@
 #include "../../../csrc/common.h"
 #include "../../../csrc/pairwise_d64.h"
 #include "../../../csrc/pairwise_generic.h"
+#include "../../../csrc/pairwise_split.h"
 #include "rbf.h"
 
-using nl2k::f32x4;
-using nl2k::load4;
-using nl2k::store4;
-using nl2k::zero4;
 using nl2k::pairwise::kD;
 
 namespace {
 
 constexpr float kLog2e = 1.4426950408889634f;
 
+// Forward policy of the SIMT tiles: the squared differences summed directly,
+// as the reference kernel does.
+struct RbfGenFwd {
+  float gamma;
+  __device__ __forceinline__ float x_in(float v, int64_t) const { return v; }
+  __device__ __forceinline__ float y_in(float v, int64_t) const { return v; }
+  __device__ __forceinline__ float step(float s, float x, float y) const {
+    const float t = x - y;
+    return fmaf(t, t, s);
+  }
+  __device__ __forceinline__ float out(float s) const { return expf(-gamma * s); }
+};
+
 // Forward policy: the row term is -kappa |x|^2, the column term |y|^2, and
 // K = exp2(min(2 kappa x.y - kappa (|x|^2 + |y|^2), 0)); the clamp keeps
 // K <= 1 when the distance cancels to a tiny negative value.
 struct RbfFwdOp {
   float neg_kappa;  // -gamma log2(e)
-  static constexpr bool kSideOut = false;
-  static constexpr bool kRowScales = false;
-  __device__ __forceinline__ float row(f32x4 (&)[4], float sx) const { return neg_kappa * sx; }
-  __device__ __forceinline__ float col(f32x4&, float sy) const { return sy; }
+  float gamma;
+  float norm_max;
+  static constexpr bool kScale = false, kDirect = true;
+  __device__ __forceinline__ float row(float sx) const { return neg_kappa * sx; }
+  __device__ __forceinline__ float col(float sy) const { return sy; }
   __device__ __forceinline__ float out(float dot, float rt, float ct) const {
     float t = fmaf(-2.f * neg_kappa, dot, fmaf(neg_kappa, ct, rt));
     t = t > 0.f ? 0.f : t;  // squared distance >= 0; NaN passes through
     return __builtin_amdgcn_exp2f(t);
   }
+  __device__ __forceinline__ RbfGenFwd direct() const { return RbfGenFwd{gamma}; }
 };
 
 // Backward policy: W = dK o K, raw X / Y rows, row and column sums of W.
@@ -77,67 +76,67 @@ struct RbfBwdOp {
   static constexpr bool kProduct = true, kScale = false, kSums = true;
 };
 
-// ------------------------------------------------------------------ forward
+// ------------------------------------------------------------------ backward
+// out[r][:] = neg2g (sum_s S[s][r] A[r][:] - sum_s P[s][r][:]), one thread
+// per V features (V = 4 when D is a multiple of 4: rows then hold whole
+// groups); the slot loop is unrolled by 4 so that the loads of several slots
+// are in flight together.
+template <int V, typename I>
+__device__ __forceinline__ void reduce_side(const float* __restrict__ P,
+                                            const float* __restrict__ S,
+                                            const float* __restrict__ A, float* __restrict__ out,
+                                            int64_t rows, int D, int slots, float neg2g, I first,
+                                            I step) {
+  typedef float vec __attribute__((ext_vector_type(V), aligned(4)));
+  const I per = (I)(D / V), groups = (I)(rows * per);
+  const size_t stride = (size_t)rows * D;
+  for (I e = first; e < groups; e += step) {
+    const I r = e / per;
+    const float* p = P + (size_t)e * V;
+    const float* q = S + r;
+    auto at = [&](int s) { return *reinterpret_cast<const vec*>(p + (size_t)s * stride); };
+    vec a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
+    float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
+    int s = 0;
+    for (; s + 4 <= slots; s += 4) {
+      a0 += at(s);
+      a1 += at(s + 1);
+      a2 += at(s + 2);
+      a3 += at(s + 3);
+      s0 += q[(size_t)s * rows];
+      s1 += q[(size_t)(s + 1) * rows];
+      s2 += q[(size_t)(s + 2) * rows];
+      s3 += q[(size_t)(s + 3) * rows];
+    }
+    for (; s < slots; ++s) {
+      a0 += at(s);
+      s0 += q[(size_t)s * rows];
+    }
+    const vec acc = (a0 + a1) + (a2 + a3);
+    const float sum = (s0 + s1) + (s2 + s3);
+    const vec a = *reinterpret_cast<const vec*>(A + (size_t)e * V);
+    *reinterpret_cast<vec*>(out + (size_t)e * V) = neg2g * (sum * a - acc);
+  }
+}
+
 // Both outputs in one launch: block b < bx handles dX, the rest dY.
-// out[r][:] = neg2g * (sum_s S[s][r] * A[r][:] - sum_s Pt[s][r][:]), D = 64,
-// one thread per float4 of the output; the slot loop is unrolled by 4 so
-// the loads of several slots are in flight together.
+template <int V, typename I>
 __global__ __launch_bounds__(256) void rbf_bwd_reduce_kernel(
     const float* __restrict__ Px, const float* __restrict__ Rx,
     const float* __restrict__ X, float* __restrict__ dX, int N, int sx,
     const float* __restrict__ Py, const float* __restrict__ Ry,
-    const float* __restrict__ Y, float* __restrict__ dY, int M, int sy,
+    const float* __restrict__ Y, float* __restrict__ dY, int M, int sy, int D,
     int bx, float neg2g) {
-  const bool is_x = (int)blockIdx.x < bx;
-  const float* __restrict__ Pt = is_x ? Px : Py;
-  const float* __restrict__ S = is_x ? Rx : Ry;
-  const float* __restrict__ A = is_x ? X : Y;
-  float* __restrict__ out = is_x ? dX : dY;
-  const int rows = is_x ? N : M;
-  const int slots = is_x ? sx : sy;
-  const int b0 = is_x ? 0 : bx;
-  const int nb = is_x ? bx : (int)gridDim.x - bx;
-  const size_t n4 = (size_t)rows * (kD / 4);
-  const size_t stride = (size_t)rows * kD;
-  for (size_t e = (size_t)(blockIdx.x - b0) * blockDim.x + threadIdx.x; e < n4;
-       e += (size_t)nb * blockDim.x) {
-    const size_t r = e / (kD / 4);
-    f32x4 a0 = zero4(), a1 = zero4(), a2 = zero4(), a3 = zero4();
-    float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
-    int s = 0;
-    for (; s + 4 <= slots; s += 4) {
-      a0 += load4(Pt + (size_t)s * stride + 4 * e);
-      a1 += load4(Pt + (size_t)(s + 1) * stride + 4 * e);
-      a2 += load4(Pt + (size_t)(s + 2) * stride + 4 * e);
-      a3 += load4(Pt + (size_t)(s + 3) * stride + 4 * e);
-      s0 += S[(size_t)s * rows + r];
-      s1 += S[(size_t)(s + 1) * rows + r];
-      s2 += S[(size_t)(s + 2) * rows + r];
-      s3 += S[(size_t)(s + 3) * rows + r];
-    }
-    for (; s < slots; ++s) {
-      a0 += load4(Pt + (size_t)s * stride + 4 * e);
-      s0 += S[(size_t)s * rows + r];
-    }
-    const f32x4 acc = (a0 + a1) + (a2 + a3);
-    const float sum = (s0 + s1) + (s2 + s3);
-    store4(out + 4 * e, neg2g * (sum * load4(A + 4 * e) - acc));
-  }
+  const int b = (int)blockIdx.x;
+  if (b < bx)
+    reduce_side<V, I>(Px, Rx, X, dX, N, D, sx, neg2g, (I)b * 256 + threadIdx.x, (I)bx * 256);
+  else
+    reduce_side<V, I>(Py, Ry, Y, dY, M, D, sy, neg2g, (I)(b - bx) * 256 + threadIdx.x,
+                      (I)((int)gridDim.x - bx) * 256);
 }
 
 // ------------------------------------------------------- generic (any D)
 // Policies of the tiled SIMT kernels (csrc/pairwise_generic.h).
-struct RbfGenFwd {
-  float gamma;
-  __device__ __forceinline__ float x_in(float v, int64_t) const { return v; }
-  __device__ __forceinline__ float y_in(float v, int64_t) const { return v; }
-  // the squared differences summed directly, as the reference kernel does
-  __device__ __forceinline__ float step(float s, float x, float y) const {
-    const float t = x - y;
-    return fmaf(t, t, s);
-  }
-  __device__ __forceinline__ float out(float s) const { return expf(-gamma * s); }
-};
 struct RbfGenBwd {
   float neg2g;
   static constexpr bool kSums = true;
@@ -211,6 +210,30 @@ inline size_t generic_ws_floats(int64_t N, int64_t M, int64_t D) {
   return (size_t)(gx.s * N * (D + 1) + gy.s * M * (D + 1));
 }
 
+// What rbf_backward_workspace_bytes reports, in floats: callers hold buffers
+// of this size, and the split backward is cut so that its partials fit.  At
+// D = 64 it is the fp32 regions' (pairwise_d64.h).
+inline size_t workspace_floats(int64_t N, int64_t M, int64_t D) {
+  if (N <= 0 || M <= 0) return 0;
+  const nl2k::pairwise::BwdPlan p = nl2k::pairwise::plan_backward(N, M, D, true);
+  if (p.fast) return p.ws_floats;
+  return std::max(generic_ws_floats(N, M, D), nl2k::pairwise::split_floats(N, M, D, true));
+}
+
+// Largest squared row norm whose distances the forward forms from norms and
+// products (|x|^2 + |y|^2 - 2 x.y); a tile with a larger one (or with a norm
+// that is not finite) sums the squared differences directly.  The former
+// leaves an error of about 2^-24 (|x|^2 + |y|^2) in the distance whatever the
+// distance is, which gamma carries into K: at gamma (|x|^2 + |y|^2) <= 8 the
+// error of K stays within a few 1e-7, as small as the direct sum's.  D = 64
+// takes the products for every finite norm, as it always has.  A negative or
+// NaN gamma always sums directly.
+inline float norm_max(float gamma, int64_t D) {
+  if (!(gamma >= 0.f)) return -1.f;
+  const float cap = gamma > 1e7f ? 1e37f / gamma : 1e30f;  // gamma times it stays finite
+  return D == kD || gamma == 0.f ? cap : std::min(cap, 4.f / gamma);
+}
+
 int launch_fill_zero(float* p, size_t count, hipStream_t stream) {
   if (count == 0) return NL2K_SUCCESS;
   const int blocks = (int)std::min<size_t>((count + 255) / 256, 4096);
@@ -218,12 +241,32 @@ int launch_fill_zero(float* p, size_t count, hipStream_t stream) {
   return nl2k::check_launch("rbf fill");
 }
 
-// The backward's tile kernels (which need the workspace) run for D == 64 and
-// 16-byte aligned X, Y, dX and dY; everything else takes the generic kernels.
-bool takes_tile_path(const nl2k::pairwise::BwdPlan& p, const float* X, const float* Y,
+// D == 64 and 16-byte aligned X, Y, dX and dY: the workspace is required.
+// Any other call runs without one (or with a shorter one) on the generic
+// kernels, their walks whole.
+bool needs_workspace(int64_t N, int64_t M, int64_t D, const float* X, const float* Y,
                      const float* dX, const float* dY) {
-  return p.fast && nl2k::aligned16(X) && nl2k::aligned16(Y) && nl2k::aligned16(dX) &&
-         nl2k::aligned16(dY);
+  using nl2k::pairwise::kMaxTileDim;
+  return D == kD && N <= kMaxTileDim && M <= kMaxTileDim && nl2k::aligned16(X) && nl2k::aligned16(Y) &&
+         nl2k::aligned16(dX) && nl2k::aligned16(dY);
+}
+
+template <class Plan>
+int reduce(const Plan& p, const float* ws, const float* X, const float* Y, float* dX,
+           float* dY, int64_t N, int64_t M, int64_t D, float neg2g, hipStream_t stream,
+           const char* who) {
+  const int64_t v = D % 4 == 0 ? 4 : 1;
+  const int64_t gx = N * (D / v), gy = M * (D / v);
+  const int bx = (int)std::min<int64_t>(nl2k::ceil_div(gx, (int64_t)256), 2048);
+  const int by = (int)std::min<int64_t>(nl2k::ceil_div(gy, (int64_t)256), 2048);
+  const bool small = std::max(gx, gy) < (int64_t(1) << 31);  // the strides fit 32 bits beside it
+  auto* kernel = v == 4 ? (small ? &rbf_bwd_reduce_kernel<4, uint32_t>
+                                 : &rbf_bwd_reduce_kernel<4, uint64_t>)
+                        : (small ? &rbf_bwd_reduce_kernel<1, uint32_t>
+                                 : &rbf_bwd_reduce_kernel<1, uint64_t>);
+  hipLaunchKernelGGL(kernel, dim3(bx + by), dim3(256), 0, stream, ws + p.px, ws + p.rx, X, dX,
+                     (int)N, p.nRJ, ws + p.py, ws + p.ry, Y, dY, (int)M, p.nRI, (int)D, bx, neg2g);
+  return nl2k::check_launch(who);
 }
 
 // Both backward entry points: the caller's workspace, or the scratch array
@@ -242,26 +285,31 @@ int backward_impl(const float* X, const float* Y, const float* dK, const float* 
   if (!dK || !K) return nl2k::fail(NL2K_ERR_NULL, "%s: dK and K must be non-null", who);
 
   const float neg2g = -2.f * gamma;
-  const nl2k::pairwise::BwdPlan p = nl2k::pairwise::plan_backward(N, M, D, true);
-  if (takes_tile_path(p, X, Y, dX, dY)) {
-    const size_t need = p.ws_floats * sizeof(float);
-    if (workspace == nullptr || workspace_bytes < need)
+  const size_t floats = workspace_floats(N, M, D), need = floats * sizeof(float);
+  const bool have = workspace != nullptr && workspace_bytes >= need;
+  if (needs_workspace(N, M, D, X, Y, dX, dY)) {
+    if (!have)
       return nl2k::fail(NL2K_ERR_WORKSPACE, "%s: workspace of %zu bytes required, got %zu", who,
                         need, workspace ? workspace_bytes : (size_t)0);
     if (!nl2k::aligned16(workspace))
       return nl2k::fail(NL2K_ERR_ALIGN, "%s: workspace must be 16-byte aligned", who);
+  }
+  if (have && reinterpret_cast<uintptr_t>(workspace) % 4 == 0) {
     float* ws = static_cast<float*>(workspace);
-    const bool vec_nm = (M % 4 == 0) && nl2k::aligned16(dK) && nl2k::aligned16(K);
-    nl2k::pairwise::launch_bwd_tiles<RbfBwdOp>(p, X, Y, dK, K, ws, (int)N, (int)M, vec_nm,
-                                               nullptr, nullptr, stream);
-    st = nl2k::check_launch(who);
-    if (st) return st;
-    const int bx = (int)std::min<int64_t>((N * (kD / 4) + 255) / 256, 2048);
-    const int by = (int)std::min<int64_t>((M * (kD / 4) + 255) / 256, 2048);
-    hipLaunchKernelGGL(rbf_bwd_reduce_kernel, dim3(bx + by), dim3(256), 0, stream,
-                       ws + p.px, ws + p.rx, X, dX, (int)N, p.nRJ, ws + p.py, ws + p.ry,
-                       Y, dY, (int)M, p.nRI, bx, neg2g);
-    return nl2k::check_launch(who);
+    const nl2k::pairwise::BwdPlan rp = nl2k::pairwise::plan_backward(N, M, D, true);
+    if (needs_workspace(N, M, D, X, Y, dX, dY) &&
+        nl2k::pairwise::takes_regions(rp, M, X, Y, dK, K)) {
+      st = nl2k::pairwise::launch_bwd_regions<RbfBwdOp>(rp, X, Y, dK, K, ws, N, M, nullptr,
+                                                        nullptr, stream, who);
+      return st ? st : reduce(rp, ws, X, Y, dX, dY, N, M, D, neg2g, stream, who);
+    }
+    const nl2k::pairwise::SplitBwdPlan p =
+        nl2k::pairwise::plan_split_backward(N, M, D, true, floats);
+    if (p.ok) {
+      st = nl2k::pairwise::launch_bwd_split<RbfBwdOp>(p, X, Y, dK, K, ws, N, M, D, nullptr,
+                                                      nullptr, stream, who);
+      return st ? st : reduce(p, ws, X, Y, dX, dY, N, M, D, neg2g, stream, who);
+    }
   }
 
   // Generic kernels: the walks split into slices when the workspace holds
@@ -357,17 +405,11 @@ int rbf_forward_f32(const float* X, const float* Y, float* K, int64_t N,
   if (!X || !Y || !K)
     return nl2k::fail(NL2K_ERR_NULL, "rbf_forward_f32: X, Y and K must be non-null");
 
-  nl2k::pairwise::FwdPlan fp;
-  if (D == kD && nl2k::aligned16(X) && nl2k::aligned16(Y) &&
-      nl2k::pairwise::plan_forward(N, M, fp)) {
-    const int vec_store = (M % 4 == 0) && nl2k::aligned16(K);
-    auto* kernel = fp.ib == 2 ? &nl2k::pairwise::pair_fwd_d64_kernel<RbfFwdOp, 2>
-                              : &nl2k::pairwise::pair_fwd_d64_kernel<RbfFwdOp, 4>;
-    hipLaunchKernelGGL(kernel, dim3(fp.n_wg), dim3(256), 0, stream, X, Y, K, (int)N, (int)M,
-                       RbfFwdOp{-gamma * kLog2e}, fp.n_jt, fp.n_units, fp.upw, vec_store, nullptr,
-                       nullptr);
-    return nl2k::check_launch("rbf_forward_f32");
-  }
+  const nl2k::pairwise::SplitFwdPlan fp = nl2k::pairwise::plan_split_forward(N, M, D);
+  if (fp.n_jt > 0)
+    return nl2k::pairwise::launch_fwd_split(fp, X, Y, K, N, M, D,
+                                            RbfFwdOp{-gamma * kLog2e, gamma, norm_max(gamma, D)},
+                                            nullptr, nullptr, stream, "rbf_forward_f32");
   const int64_t ntiles = nl2k::ceil_div(N, (int64_t)nl2k::pairwise::kGT) *
                          nl2k::ceil_div(M, (int64_t)nl2k::pairwise::kGT);
   hipLaunchKernelGGL(nl2k::pairwise::pair_fwd_generic_kernel<RbfGenFwd>,
@@ -378,11 +420,7 @@ int rbf_forward_f32(const float* X, const float* Y, float* K, int64_t N,
 
 size_t rbf_backward_workspace_bytes(int64_t N, int64_t M, int64_t D) {
   if (validate_sizes(N, M, D)) return 0;
-  const nl2k::pairwise::BwdPlan p = nl2k::pairwise::plan_backward(N, M, D, true);
-  // Shapes the tile path takes (when aligned) report its need; the others
-  // the generic kernels' slices.  A misaligned call of a tile-path shape
-  // runs the generic kernels unsplit within that workspace.
-  return (p.fast ? p.ws_floats : generic_ws_floats(N, M, D)) * sizeof(float);
+  return workspace_floats(N, M, D) * sizeof(float);
 }
 
 int rbf_backward_f32(const float* X, const float* Y, const float* dK,
@@ -401,10 +439,11 @@ int rbf_backward_f32_noalloc(const float* X, const float* Y, const float* dK, co
   const char* who = "rbf_backward_f32_noalloc";
   int st = validate_sizes(N, M, D);
   if (st) return st;
-  // Only the tile path uses scratch; shapes and alignments that take the
-  // generic kernels run whatever their size.
-  const nl2k::pairwise::BwdPlan p = nl2k::pairwise::plan_backward(N, M, D, true);
-  const size_t need = takes_tile_path(p, X, Y, dX, dY) ? p.ws_floats * sizeof(float) : 0;
+  // Only calls that require a workspace use scratch; the others run whatever
+  // their size, on the generic kernels.
+  const size_t need = needs_workspace(N, M, D, X, Y, dX, dY)
+                          ? workspace_floats(N, M, D) * sizeof(float)
+                          : 0;
   if (need > kScratchBytes)
     return nl2k::fail(NL2K_ERR_WORKSPACE,
                       "%s: N=%lld M=%lld D=%lld needs %zu bytes of scratch; the library's static "

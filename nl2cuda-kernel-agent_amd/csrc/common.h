@@ -118,6 +118,7 @@ inline int resident_blocks(const void* kernel, int threads, int* out) {
 }
 
 // -------------------------------------------------------------- device side
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef double f64x2 __attribute__((ext_vector_type(2)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
@@ -149,6 +150,10 @@ __device__ __forceinline__ buffer_rsrc make_rsrc(const void* base, uint32_t byte
 
 __device__ __forceinline__ f32x4 buffer_load4(buffer_rsrc r, uint32_t lane_off, int wave_off) {
   return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, lane_off, wave_off, 0));
+}
+
+__device__ __forceinline__ f32x2 buffer_load2(buffer_rsrc r, uint32_t lane_off, int wave_off) {
+  return __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(r, lane_off, wave_off, 0));
 }
 
 // Store through a raw buffer resource: a lane whose offset is at or past the

@@ -53,54 +53,67 @@ inline GenericSplit generic_whole(int64_t others) {
   return GenericSplit{1, ceil_div(others, (int64_t)kGT) * kGT};
 }
 
+struct SimtTile {
+  float xs[kGK][kGT + 4];
+  float ys[kGK][kGT + 4];
+};
+
+// out[i0 .. i0 + 63][j0 .. j0 + 63], by 256 threads (every thread of the
+// workgroup calls it; t may hold anything, and is free on return).
+template <class Op>
+__device__ __forceinline__ void simt_fwd_tile(SimtTile& t, const float* __restrict__ X,
+                                              const float* __restrict__ Y,
+                                              float* __restrict__ out, int64_t N, int64_t M,
+                                              int64_t D, int64_t i0, int64_t j0, const Op& op) {
+  const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
+  float s[4][4] = {};
+  __syncthreads();
+  for (int64_t k0 = 0; k0 < D; k0 += kGK) {
+    // 64 rows x 16 features of X and of Y: four of each per thread
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int e = threadIdx.x + 256 * q;  // 0 .. 1023
+      const int r = e / kGK, k = e % kGK;
+      const int64_t gi = i0 + r, gj = j0 + r, gk = k0 + k;
+      const bool kin = gk < D;
+      const int64_t ci = min(gi, N - 1), cj = min(gj, M - 1);
+      const float xv = X[ci * D + min(gk, D - 1)];
+      const float yv = Y[cj * D + min(gk, D - 1)];
+      t.xs[k][r] = (kin && gi < N) ? op.x_in(xv, ci) : 0.f;
+      t.ys[k][r] = (kin && gj < M) ? op.y_in(yv, cj) : 0.f;
+    }
+    __syncthreads();
+#pragma unroll 4
+    for (int k = 0; k < kGK; ++k) {
+      const f32x4 xa = *reinterpret_cast<const f32x4*>(&t.xs[k][4 * ty]);
+      const f32x4 yb = *reinterpret_cast<const f32x4*>(&t.ys[k][4 * tx]);
+#pragma unroll
+      for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) s[a][b] = op.step(s[a][b], xa[a], yb[b]);
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    const int64_t i = i0 + 4 * ty + a;
+    if (i >= N) continue;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      const int64_t j = j0 + 4 * tx + b;
+      if (j < M) out[i * M + j] = op.out(s[a][b]);
+    }
+  }
+}
+
 template <class Op>
 __global__ __launch_bounds__(256) void pair_fwd_generic_kernel(
     const float* __restrict__ X, const float* __restrict__ Y, float* __restrict__ out,
     int64_t N, int64_t M, int64_t D, Op op) {
-  __shared__ float xs[kGK][kGT + 4];
-  __shared__ float ys[kGK][kGT + 4];
-  const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
+  __shared__ __attribute__((aligned(16))) SimtTile t;
   const int64_t ntj = (M + kGT - 1) / kGT, ntiles = (N + kGT - 1) / kGT * ntj;
-  for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const int64_t i0 = tile / ntj * kGT, j0 = tile % ntj * kGT;
-    float s[4][4] = {};
-    for (int64_t k0 = 0; k0 < D; k0 += kGK) {
-      // 64 rows x 16 features of X and of Y: four of each per thread
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int e = threadIdx.x + 256 * q;  // 0 .. 1023
-        const int r = e / kGK, k = e % kGK;
-        const int64_t gi = i0 + r, gj = j0 + r, gk = k0 + k;
-        const bool kin = gk < D;
-        const int64_t ci = min(gi, N - 1), cj = min(gj, M - 1);
-        const float xv = X[ci * D + min(gk, D - 1)];
-        const float yv = Y[cj * D + min(gk, D - 1)];
-        xs[k][r] = (kin && gi < N) ? op.x_in(xv, ci) : 0.f;
-        ys[k][r] = (kin && gj < M) ? op.y_in(yv, cj) : 0.f;
-      }
-      __syncthreads();
-#pragma unroll 4
-      for (int k = 0; k < kGK; ++k) {
-        const f32x4 xa = *reinterpret_cast<const f32x4*>(&xs[k][4 * ty]);
-        const f32x4 yb = *reinterpret_cast<const f32x4*>(&ys[k][4 * tx]);
-#pragma unroll
-        for (int a = 0; a < 4; ++a)
-#pragma unroll
-          for (int b = 0; b < 4; ++b) s[a][b] = op.step(s[a][b], xa[a], yb[b]);
-      }
-      __syncthreads();
-    }
-#pragma unroll
-    for (int a = 0; a < 4; ++a) {
-      const int64_t i = i0 + 4 * ty + a;
-      if (i >= N) continue;
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const int64_t j = j0 + 4 * tx + b;
-        if (j < M) out[i * M + j] = op.out(s[a][b]);
-      }
-    }
-  }
+  for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x)
+    simt_fwd_tile(t, X, Y, out, N, M, D, tile / ntj * kGT, tile % ntj * kGT, op);
 }
 
 // TRANS = false: rows are X's (N), the walk is over Y's rows (M), W[i][j];
