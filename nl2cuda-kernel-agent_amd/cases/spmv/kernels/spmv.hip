@@ -39,11 +39,11 @@
 //    column varies between runs, as with the reference's atomics.  Column
 //    counts too large for 1024 buckets of 16384 columns fall back to
 //    zero-fill plus fp32 atomics from the walk.
-//  * D > 1 (SpMM): groups of L lanes cover a row's columns (L = 4, 16 or
-//    64), float4 columns when D % 4 == 0 and X / Y are 16-byte aligned; the
-//    lanes of a group share each (col, val) load and read the X row
-//    coalesced, and G groups split a long row's nonzeros (their sums added
-//    by an xor butterfly).  Backward, deterministic and without atomics:
+//  * D > 1 (SpMM): groups of L lanes cover a row's columns (L = 4 .. 64),
+//    four a lane from D = 4 on, at any alignment; the lanes of a group share
+//    each (col, val) load and read the X row coalesced, G groups split a
+//    row's nonzeros (their sums added by an xor butterfly), and the whole
+//    workgroup shares its longest rows.  Backward, deterministic and without atomics:
 //    with D % 4 == 0, D <= 64, 128 to 256 blocks of 256 / L columns
 //    (K = 4096 at the reference default) and 16-byte aligned X / dY / dX,
 //    two launches: each 1024-position chunk sorts its entries by column
@@ -52,8 +52,10 @@
 //    up to K = 16384, a stable column-major copy of A built in the workspace
 //    (chunk histograms, column offsets, an in-order scatter), then the same
 //    lane-group gather per column (the spmm_t_* kernels); dvals from the
-//    gather pass either way.  Beyond 16384 columns: per nonzero a group
-//    reduction for dvals and per-element atomics for dX.
+//    gather pass either way.  Beyond 16384 columns, with room for the entries
+//    in the workspace: grouped by bucket of columns and summed per bucket in
+//    LDS (the spmm_c_* kernels); without it per nonzero a group reduction for
+//    dvals and per-element atomics for dX.
 #include <algorithm>
 #include <cstdint>
 #include <type_traits>
@@ -706,14 +708,17 @@ __global__ __launch_bounds__(kSumThreads) void spmv_bucket_sum_kernel(
 }
 
 // ------------------------------------------------------------------ D > 1
+// 16 bytes at any 4-byte boundary.
+typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
+
 template <bool VEC>
 struct Lanes;
 template <>
 struct Lanes<true> {
   using T = f32x4;
   static constexpr int W = 4;
-  __device__ static T load(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
-  __device__ static void store(float* p, T v) { *reinterpret_cast<f32x4*>(p) = v; }
+  __device__ static T load(const float* p) { return *reinterpret_cast<const f32x4_u*>(p); }
+  __device__ static void store(float* p, T v) { *reinterpret_cast<f32x4_u*>(p) = v; }
   __device__ static T zero() { return f32x4{0.f, 0.f, 0.f, 0.f}; }
   __device__ static float dot(T a, T b) { return (a[0] * b[0] + a[1] * b[1]) + (a[2] * b[2] + a[3] * b[3]); }
 };
@@ -771,6 +776,16 @@ __device__ __forceinline__ void spmm_chunk(const I* __restrict__ col,
   for (int u = 0; u < U; ++u) acc += vv[u] * xs[u];
 }
 
+// Rows of more than kLongRow * G entries are left to the whole workgroup,
+// after its other rows: every group takes a share of the row, added in a
+// fixed order, so a long row costs a few round trips instead of a chain of
+// them.  D >= 4: a lane owns four columns, at any alignment; the last lane of
+// a D that is no multiple of 4 owns the row's last four, some of them with
+// its neighbour (both sum and store the same bits).
+// Bound by the gather of X rows (D floats per nonzero, from L2 and MALL).
+// 100000 rows of 1 to 516 entries, 1.6 M in all, D = 32: 120 -> 59 us (eight
+// lanes a row instead of sixteen half idle, long rows shared).
+constexpr int kLongRow = 64;
 template <typename I, int L, int G, bool VEC>
 __global__ __launch_bounds__(kThreads) void spmm_fwd_kernel(
     const I* __restrict__ ptr, const I* __restrict__ col, const float* __restrict__ vals,
@@ -779,40 +794,78 @@ __global__ __launch_bounds__(kThreads) void spmm_fwd_kernel(
   using V = Lanes<VEC>;
   constexpr int kRowLanes = L * G;
   static_assert(kRowLanes <= 64 && (kRowLanes & (kRowLanes - 1)) == 0, "rows inside a wave");
-  const int64_t row = (int64_t)blockIdx.x * (kThreads / kRowLanes) + threadIdx.x / kRowLanes;
+  constexpr int kRows = kThreads / kRowLanes;  // rows per workgroup
+  constexpr int kWaves = kThreads / 64;
+  __shared__ int s_n, s_long[kRows];
+  __shared__ typename V::T s_sum[kWaves][L];
+  const int64_t row0 = (int64_t)blockIdx.x * kRows;
+  const int64_t row = row0 + threadIdx.x / kRowLanes;
   const int gl = threadIdx.x % L;
   const int grp = (threadIdx.x % kRowLanes) / L;
   const bool live = row < M;
   const int64_t s = live ? ld_ptr(ptr, row, nnz) : 0;
   const int64_t e = live ? max(s, ld_ptr(ptr, row + 1, nnz)) : 0;
+  const bool is_long = e - s > kLongRow * G;
+  if (threadIdx.x == 0) s_n = 0;
+  __syncthreads();
+  if (is_long && gl == 0 && grp == 0) s_long[atomicAdd(&s_n, 1)] = threadIdx.x / kRowLanes;
+  const int64_t own_e = is_long ? s : e;
   for (int64_t d0 = 0; d0 < D; d0 += (int64_t)L * V::W) {
     const int64_t d = d0 + (int64_t)gl * V::W;
     const bool active = d < D;
-    const int64_t dc = active ? d : 0;
+    const int64_t dc = active ? min(d, D - V::W) : 0;
     typename V::T acc = V::zero();
     // chunks of 16 entries per group (the whole group's share of a
     // reference-default row: 11.6 against 12.4 us with chunks of 4), then 4
     int64_t p = s + grp;
-    for (; p + 15 * G < e; p += 16 * G) spmm_chunk<16, G, V>(col, vals, X, p, K, D, dc, acc);
-    for (; p + 3 * G < e; p += 4 * G) spmm_chunk<4, G, V>(col, vals, X, p, K, D, dc, acc);
-    for (; p < e; p += G) acc += vals[p] * V::load(X + ld_col(col, p, K) * D + dc);
+    for (; p + 15 * G < own_e; p += 16 * G) spmm_chunk<16, G, V>(col, vals, X, p, K, D, dc, acc);
+    for (; p + 3 * G < own_e; p += 4 * G) spmm_chunk<4, G, V>(col, vals, X, p, K, D, dc, acc);
+    for (; p < own_e; p += G) acc += vals[p] * V::load(X + ld_col(col, p, K) * D + dc);
     if constexpr (G > 1) acc = groups_sum<L, G>(acc);
-    if (live && active && grp == 0) V::store(Y + row * D + d, acc);
+    if (live && !is_long && active && grp == 0) V::store(Y + row * D + dc, acc);
+  }
+  __syncthreads();
+  const int n_long = s_n;
+  constexpr int kGroups = kThreads / L;  // of the workgroup
+  const int wave = threadIdx.x >> 6, wg = threadIdx.x / L;
+  for (int k = 0; k < n_long; ++k) {
+    const int64_t r = row0 + s_long[k];
+    const int64_t ls = ld_ptr(ptr, r, nnz), le = max(ls, ld_ptr(ptr, r + 1, nnz));
+    for (int64_t d0 = 0; d0 < D; d0 += (int64_t)L * V::W) {
+      const int64_t d = d0 + (int64_t)gl * V::W;
+      const bool active = d < D;
+      const int64_t dc = active ? min(d, D - V::W) : 0;
+      typename V::T acc = V::zero();
+      int64_t p = ls + wg;
+      for (; p + 7 * kGroups < le; p += 8 * kGroups)
+        spmm_chunk<8, kGroups, V>(col, vals, X, p, K, D, dc, acc);
+      for (; p + kGroups < le; p += 2 * kGroups)
+        spmm_chunk<2, kGroups, V>(col, vals, X, p, K, D, dc, acc);
+      if (p < le) acc += vals[p] * V::load(X + ld_col(col, p, K) * D + dc);
+      acc = groups_sum<L, 64 / L>(acc);
+      if ((threadIdx.x & 63) < L) s_sum[wave][gl] = acc;
+      __syncthreads();
+      if (threadIdx.x < L && active) {
+        typename V::T t = s_sum[0][gl];
+#pragma unroll
+        for (int w = 1; w < kWaves; ++w) t += s_sum[w][gl];
+        V::store(Y + r * D + dc, t);
+      }
+      __syncthreads();
+    }
   }
 }
 
 // Sum over each aligned group of L lanes (every lane of a group active).
-// L = 4 and 16 stay inside a DPP row: quad_perm [1,0,3,2] and [2,3,0,1],
-// then row_half_mirror and row_mirror; L = 64 uses cross-row shuffles.
+// L = 4, 8 and 16 stay inside a DPP row: quad_perm [1,0,3,2] and [2,3,0,1],
+// then row_half_mirror and row_mirror; L = 32 and 64 use cross-row shuffles.
 template <int L>
 __device__ __forceinline__ float group_sum(float v) {
-  if constexpr (L == 4 || L == 16) {
+  if constexpr (L <= 16) {
     v += nl2k::dpp_mov<0xB1>(v);
     v += nl2k::dpp_mov<0x4E>(v);
-    if constexpr (L == 16) {
-      v += nl2k::dpp_mov<0x141>(v);
-      v += nl2k::dpp_mov<0x140>(v);
-    }
+    if constexpr (L >= 8) v += nl2k::dpp_mov<0x141>(v);
+    if constexpr (L >= 16) v += nl2k::dpp_mov<0x140>(v);
     return v;
   } else {
 #pragma unroll
@@ -1689,6 +1742,351 @@ __global__ __launch_bounds__(kBktThreads) void spmm_b_gather_kernel(
   if (half == 0 && live && active) nl2k::store4(dX + c * D + d, acc + s_half[tl]);
 }
 
+// ------------------ SpMM backward dX by column buckets (D > 1, K > 16384)
+// dX = A^T dY where a count per column and chunk (the column-major copy) no
+// longer fits: entries are grouped by bucket of `cols` columns, then each
+// bucket's columns are summed by one workgroup.
+//  B1 spmm_c_hist_kernel:    entries per bucket (LDS counts, one integer
+//                            atomic per bucket and tile).
+//  B2 spmm_c_scan_kernel:    one workgroup: each bucket's first record, and
+//                            the list of parts, kCbPart entries of a bucket
+//                            each (a bucket without entries has one part).
+//  B3 spmm_c_scatter_kernel: each tile finds its positions' rows, reserves
+//                            its share of every bucket, and writes one
+//                            16-byte record {row, position, value, column}
+//                            per entry.  It also zeroes the dX rows of
+//                            buckets of several parts.
+//  B4 spmm_c_gather_kernel:  a part, up to kCbCap records a round: sorted by
+//                            column in LDS (integer counts), then cut evenly
+//                            between groups of L lanes whatever the columns'
+//                            lengths; a group sums vals * dY[row] in
+//                            registers and adds a finished column's sum to
+//                            the part's LDS copy of its dX rows (by compare
+//                            and swap only where a column crosses from one
+//                            group to the next); dvals[p] = dY[row] . X[c] on
+//                            the way.  A bucket of one part is stored, the
+//                            parts of a longer one are added to dX with
+//                            atomics.
+// The order of the additions within a column varies between runs, as with the
+// atomics a call without the workspace takes.
+// Bound by the gather of dY rows (D floats per entry, from L2 and MALL).  1.6 M
+// entries, 100000 columns, D = 32: 90 us (2 + 10 + 4 + 28 + 45) against 981 with
+// atomics.
+constexpr int kCbThreads = 512;
+constexpr int kCbHistTile = 8192;   // positions per workgroup, B1
+constexpr int kCbCap = 2048;        // records per round, B4
+constexpr int kCbPart = 4 * kCbCap; // records per part
+constexpr int kCbMaxBuckets = 8192; // LDS counts of a tile
+constexpr int kCbMaxCols = 1024;    // columns per bucket
+constexpr int kCbFloats = 8192;     // LDS floats of a bucket's dX (and X) rows
+
+__global__ __launch_bounds__(kThreads) void spmm_c_zero_kernel(int* __restrict__ count, int n) {
+  const int i = (int)blockIdx.x * kThreads + threadIdx.x;
+  if (i < n) count[i] = 0;
+}
+
+template <typename I>
+__global__ __launch_bounds__(kCbThreads) void spmm_c_hist_kernel(const I* __restrict__ col,
+                                                                 int* __restrict__ count,
+                                                                 int64_t K, int64_t nnz,
+                                                                 int shift, int nb) {
+  extern __shared__ int lds_i[];
+  for (int b = threadIdx.x; b < nb; b += kCbThreads) lds_i[b] = 0;
+  __syncthreads();
+  const int64_t p0 = (int64_t)blockIdx.x * kCbHistTile, p1 = min(nnz, p0 + kCbHistTile);
+  constexpr int B = kCbHistTile / kCbThreads;  // loads in flight per thread
+  I cv[B];
+#pragma unroll
+  for (int u = 0; u < B; ++u) cv[u] = col[min(p0 + (int64_t)u * kCbThreads + threadIdx.x, p1 - 1)];
+#pragma unroll
+  for (int u = 0; u < B; ++u) {
+    const int64_t c = (int64_t)cv[u];
+    if (p0 + (int64_t)u * kCbThreads + threadIdx.x < p1)
+      atomicAdd(&lds_i[(int)((c < 0 ? 0 : (c >= K ? K - 1 : c)) >> shift)], 1);
+  }
+  __syncthreads();
+  for (int b = threadIdx.x; b < nb; b += kCbThreads) {
+    const int v = lds_i[b];
+    if (v) atomicAdd(&count[b], v);
+  }
+}
+
+// count[b] -> base[b] (first record), base[nb]; cursor[b] = base[b];
+// part_of[i] = {bucket, first record, one past the last, parts of the bucket},
+// n_parts[0] of them.
+constexpr int kCbScanThreads = 1024;
+constexpr int kCbScanPer = kCbMaxBuckets / kCbScanThreads;
+__global__ __launch_bounds__(kCbScanThreads) void spmm_c_scan_kernel(
+    const int* __restrict__ count, int* __restrict__ cursor, i32x4_t* __restrict__ part_of,
+    int* __restrict__ n_parts, int nb) {
+  __shared__ int s_rec[kCbScanThreads / 64], s_part[kCbScanThreads / 64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int n[kCbScanPer], rec = 0, parts = 0;
+#pragma unroll
+  for (int u = 0; u < kCbScanPer; ++u) {
+    const int b = (int)threadIdx.x * kCbScanPer + u;
+    n[u] = b < nb ? count[b] : 0;
+    rec += n[u];
+    parts += b < nb ? max(1, (n[u] + kCbPart - 1) / kCbPart) : 0;
+  }
+  const int irec = wave_incl_scan<int>(rec, lane), ipart = wave_incl_scan<int>(parts, lane);
+  if (lane == 63) {
+    s_rec[wave] = irec;
+    s_part[wave] = ipart;
+  }
+  __syncthreads();
+  int r0 = irec - rec, q0 = ipart - parts;
+  for (int w = 0; w < wave; ++w) {
+    r0 += s_rec[w];
+    q0 += s_part[w];
+  }
+#pragma unroll
+  for (int u = 0; u < kCbScanPer; ++u) {
+    const int b = (int)threadIdx.x * kCbScanPer + u;
+    if (b >= nb) continue;
+    cursor[b] = r0;
+    const int np = max(1, (n[u] + kCbPart - 1) / kCbPart);
+    for (int k = 0; k < np; ++k)
+      part_of[q0 + k] = i32x4_t{b, r0 + k * kCbPart, r0 + min(n[u], (k + 1) * kCbPart), np};
+    r0 += n[u];
+    q0 += np;
+    if (b == nb - 1) n_parts[0] = q0;
+  }
+}
+
+// NT threads, kPerT positions each: 512 x 4, or 1024 x 8 from kCbLongNnz
+// entries on.  A tile makes one atomic per bucket it meets, all tiles on the
+// same cursors, and writes its entries of a bucket side by side, so larger
+// tiles make fewer of the one and longer runs of the other: 49 against 28 us
+// at 1.6 M entries in 782 buckets.
+constexpr int64_t kCbLongNnz = 1 << 19;
+template <typename I, int NT, int kPerT>
+__global__ __launch_bounds__(NT) void spmm_c_scatter_kernel(
+    const I* __restrict__ ptr, const I* __restrict__ col, const float* __restrict__ vals,
+    int* __restrict__ cursor, i32x4_t* __restrict__ crec, const i32x4_t* __restrict__ part_of,
+    const int* __restrict__ n_parts, float* __restrict__ dX, int64_t M, int64_t K, int64_t D,
+    int64_t nnz, int shift, int nb) {
+  extern __shared__ int lds_i[];  // counts, then first records, of the tile's buckets
+  __shared__ int s_win[kScatterRowWin];  // row_ptr[ra + 1 .. rb]
+  __shared__ long long s_rows[2];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t p0 = (int64_t)blockIdx.x * (NT * kPerT), p1 = min(nnz, p0 + NT * kPerT);
+  // the row searches first: a wave's loads complete in order
+  if (wave < 2) {
+    const int64_t r = rows_lower_bound(ptr, M, nnz, wave == 0 ? p0 + 1 : p1, lane, 0) - 1;
+    if (lane == 0) s_rows[wave] = max((int64_t)0, min(r, M - 1));
+  }
+  I craw[kPerT];
+  float vv[kPerT];
+#pragma unroll
+  for (int k = 0; k < kPerT; ++k) {
+    const int64_t q = min(p0 + (int64_t)k * NT + threadIdx.x, p1 - 1);
+    craw[k] = col[q];
+    vv[k] = vals[q];
+  }
+  for (int b = threadIdx.x; b < nb; b += NT) lds_i[b] = 0;
+  // dX rows of the buckets that several workgroups will add to
+  for (int i = blockIdx.x; i < n_parts[0]; i += gridDim.x) {
+    const i32x4_t pt = part_of[i];
+    if (pt[3] == 1) continue;
+    const int64_t c0 = (int64_t)pt[0] << shift;
+    const int64_t n = min(K - c0, (int64_t)1 << shift) * D;
+    for (int64_t e = threadIdx.x; e < n; e += NT) dX[c0 * D + e] = 0.f;
+  }
+  __syncthreads();
+  const int64_t ra = s_rows[0], rb = max(s_rows[0], s_rows[1]);
+  const int nw = (int)min(rb - ra, (int64_t)kScatterRowWin + 1);
+  const bool windowed = rb - ra <= kScatterRowWin;
+  if (windowed && rb > ra && threadIdx.x < kThreads) load_to_lds(ptr + ra + 1, s_win, rb - ra);
+  int bk[kPerT], rank[kPerT], cl[kPerT];
+#pragma unroll
+  for (int k = 0; k < kPerT; ++k) {
+    const int64_t c = (int64_t)craw[k];
+    cl[k] = (int)(c < 0 ? 0 : (c >= K ? K - 1 : c));
+    bk[k] = cl[k] >> shift;
+    rank[k] = p0 + (int64_t)k * NT + threadIdx.x < p1 ? atomicAdd(&lds_i[bk[k]], 1) : -1;
+  }
+  __syncthreads();
+  for (int b = threadIdx.x; b < nb; b += NT) {
+    const int v = lds_i[b];
+    if (v) lds_i[b] = atomicAdd(&cursor[b], v);
+  }
+  __syncthreads();
+  int top = 1;
+  while (top * 2 <= nw) top *= 2;
+#pragma unroll
+  for (int k = 0; k < kPerT; ++k) {
+    const int64_t q = p0 + (int64_t)k * NT + threadIdx.x;
+    const int64_t qr = min(q, p1 - 1);
+    int64_t row;
+    if (windowed) {  // row ra + m with s_win[m - 1] = row_ptr[ra + m] <= qr
+      int m = 0;
+      for (int step = top; step > 0; step >>= 1)
+        if (m + step <= nw && s_win[m + step - 1] <= qr) m += step;
+      row = ra + m;
+    } else {
+      row = row_of(ptr, ra, rb, qr, nnz);
+    }
+    if (rank[k] >= 0)
+      crec[min((int64_t)lds_i[bk[k]] + rank[k], nnz - 1)] =
+          i32x4_t{(int)row, (int)q, __float_as_int(vv[k]), cl[k]};
+  }
+}
+
+// MODE: kCbScalar one column per lane (D < 4); kCbVec four, D % 4 == 0;
+// kCbTail four, the row's last lane holding its last D % 4 columns: it reads
+// the row's last four and keeps its own (rows then start at any 4-byte
+// boundary, which is all the loads need).
+constexpr int kCbScalar = 0, kCbVec = 1, kCbTail = 2;
+template <int L, int MODE, bool DV>
+__global__ __launch_bounds__(kCbThreads) void spmm_c_gather_kernel(
+    const i32x4_t* __restrict__ crec, const i32x4_t* __restrict__ part_of,
+    const int* __restrict__ n_parts, const float* __restrict__ X, const float* __restrict__ dY,
+    float* __restrict__ dX, float* __restrict__ dvals, int64_t M, int64_t K, int64_t D,
+    int64_t nnz, int shift) {
+  using V = Lanes<MODE != kCbScalar>;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int cols = 1 << shift;
+  i32x4_t* list = reinterpret_cast<i32x4_t*>(smem);                    // [kCbCap]
+  float* acc = reinterpret_cast<float*>(smem + kCbCap * sizeof(i32x4_t));  // [cols][D]
+  float* xs = acc + (size_t)cols * D;                                  // [cols][D], DV
+  __shared__ int cnt[kCbMaxCols];
+  __shared__ int s_wsum[kCbThreads / 64];
+  if ((int)blockIdx.x >= n_parts[0]) return;
+  const i32x4_t pt = part_of[blockIdx.x];
+  const int64_t c0 = (int64_t)pt[0] << shift;
+  const int n_cols = (int)min(K - c0, (int64_t)cols);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int gl = tid % L, g = tid / L;
+  constexpr int kGroups = kCbThreads / L;
+  constexpr int U = 4;  // entries whose rows are in flight together, per group
+  for (int e = tid; e < n_cols * (int)D; e += kCbThreads) {
+    acc[e] = 0.f;
+    if constexpr (DV) xs[e] = X[c0 * D + e];
+  }
+  for (int r0 = pt[1]; r0 < pt[2]; r0 += kCbCap) {
+    const int n = min(kCbCap, pt[2] - r0);
+    for (int i = tid; i < cols; i += kCbThreads) cnt[i] = 0;
+    __syncthreads();  // (the last round's list has been read, too)
+    constexpr int kPerT = kCbCap / kCbThreads;
+    i32x4_t rec[kPerT];
+    int lc[kPerT], rank[kPerT];
+#pragma unroll
+    for (int k = 0; k < kPerT; ++k) rec[k] = crec[r0 + min(k * kCbThreads + tid, n - 1)];
+#pragma unroll
+    for (int k = 0; k < kPerT; ++k) {
+      lc[k] = min(max((int)(rec[k][3] - c0), 0), n_cols - 1);
+      rank[k] = k * kCbThreads + tid < n ? atomicAdd(&cnt[lc[k]], 1) : -1;
+    }
+    __syncthreads();
+    // exclusive scan of the counts, two a thread
+    const int a0 = 2 * tid < cols ? cnt[2 * tid] : 0, a1 = 2 * tid + 1 < cols ? cnt[2 * tid + 1] : 0;
+    const int incl = wave_incl_scan<int>(a0 + a1, lane);
+    if (lane == 63) s_wsum[wave] = incl;
+    __syncthreads();
+    int start = incl - a0 - a1;
+    for (int w = 0; w < wave; ++w) start += s_wsum[w];
+    if (2 * tid < cols) cnt[2 * tid] = start;
+    if (2 * tid + 1 < cols) cnt[2 * tid + 1] = start + a0;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kPerT; ++k)
+      if (rank[k] >= 0) {
+        rec[k][3] = lc[k];
+        list[cnt[lc[k]] + rank[k]] = rec[k];
+      }
+    __syncthreads();
+    // group g's run of the sorted list
+    const int per = (n + kGroups - 1) / kGroups;
+    const int q0 = min(n, g * per), q1 = min(n, q0 + per);
+    if (q0 < q1) {  // whole groups
+      const int first = q0 > 0 && list[q0 - 1][3] == list[q0][3] ? list[q0][3] : -1;
+      const int last = q1 < n && list[q1][3] == list[q1 - 1][3] ? list[q1][3] : -1;
+      for (int64_t d0 = 0; d0 < D; d0 += (int64_t)L * V::W) {
+        const int d = (int)d0 + gl * V::W;
+        const bool active = d < D;
+        const int dc = active ? (MODE == kCbTail ? min(d, (int)D - 4) : d) : 0;
+        const int skip = active ? d - dc : V::W;  // columns of the load that are another lane's
+        typename V::T sum = V::zero();
+        int cur = list[q0][3];
+        auto flush = [&] {
+          float* a = acc + cur * (int)D + dc;
+          const bool shared = cur == first || cur == last;
+          if constexpr (MODE == kCbVec) {
+            if (!active) return;
+            if (shared) {
+#pragma unroll
+              for (int u = 0; u < 4; ++u) lds_add_f32(a + u, sum[u]);
+            } else {
+              *reinterpret_cast<f32x4*>(a) += sum;
+            }
+          } else {
+#pragma unroll
+            for (int u = 0; u < V::W; ++u) {
+              float v;
+              if constexpr (MODE == kCbScalar) v = sum;
+              else v = sum[u];
+              if (u < skip) continue;
+              if (shared) lds_add_f32(a + u, v);
+              else a[u] += v;
+            }
+          }
+        };
+        // a lane's own columns of row r (of dY or of the LDS copy of X)
+        auto own = [&](typename V::T v) {
+          if constexpr (MODE == kCbTail) {
+#pragma unroll
+            for (int u = 0; u < 3; ++u) v[u] = u < skip ? 0.f : v[u];
+          }
+          return v;
+        };
+        auto lds_row = [&](const float* x) {
+          if constexpr (MODE == kCbVec) return *reinterpret_cast<const f32x4*>(x);
+          else if constexpr (MODE == kCbTail) return f32x4{x[0], x[1], x[2], x[3]};
+          else return *x;
+        };
+        for (int q = q0; q < q1; q += U) {
+          i32x4_t r[U];
+          typename V::T gy[U];
+#pragma unroll
+          for (int u = 0; u < U; ++u) r[u] = list[min(q + u, q1 - 1)];
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            const int64_t row = min(max((int64_t)r[u][0], (int64_t)0), M - 1);
+            gy[u] = own(V::load(dY + row * D + dc));
+          }
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            const bool in = q + u < q1;  // the same over the group
+            if (in && r[u][3] != cur) {
+              flush();
+              cur = r[u][3];
+              sum = V::zero();
+            }
+            if (in) sum += __int_as_float(r[u][2]) * gy[u];
+            if constexpr (DV) {
+              const float dt =
+                  group_sum<L>(active ? V::dot(gy[u], lds_row(xs + r[u][3] * (int)D + dc)) : 0.f);
+              const int64_t p = min(max((int64_t)r[u][1], (int64_t)0), nnz - 1);
+              if (in && gl == 0) dvals[p] = dt;
+            }
+          }
+        }
+        flush();
+      }
+    }
+    __syncthreads();
+  }
+  __syncthreads();
+  float* out = dX + c0 * D;
+  if (pt[3] == 1) {
+    for (int e = tid; e < n_cols * (int)D; e += kCbThreads) out[e] = acc[e];
+  } else {
+    for (int e = tid; e < n_cols * (int)D; e += kCbThreads)
+      __hip_atomic_fetch_add(out + e, acc[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
 // ------------------------------ D == 1 dX: contributions formed in the sort
 // tile_rows[t] for t in [0, n_tiles]: the last row r with row_ptr[r] <=
 // min(t * kSortTile, nnz - 1), clamped into [0, M - 1] -- the row holding
@@ -2039,6 +2437,12 @@ int lanes_for(int64_t D, bool vec) {
   return units <= 4 ? 4 : (units <= 16 ? 16 : 64);
 }
 
+// Lanes for a row of `units` (four columns each, or one where D < 4): the
+// smallest group that covers it, or a whole wave in several passes.
+int row_lanes(int64_t units) {
+  return units <= 4 ? 4 : units <= 8 ? 8 : units <= 16 ? 16 : units <= 32 ? 32 : 64;
+}
+
 // Groups of L lanes that share a column in the SpMM backward's gather: 2
 // when L * 2 <= 64 and an average column has two 16-entry steps or more,
 // else 1.  At the reference default (64 entries per column, L = 16, 159
@@ -2104,35 +2508,39 @@ int forward(const I* ptr, const I* col, const float* vals, const float* X, float
                        X, Y, Xg, M, K, nnz, n_waves);
     return nl2k::check_launch(who);
   }
-  const bool vec = D % 4 == 0 && nl2k::aligned16(X) && nl2k::aligned16(Y);
-  const int L = lanes_for(D, vec);
+  const int L = row_lanes(D < 4 ? D : nl2k::ceil_div(D, (int64_t)4));
   const int G = spmm_row_groups(L, M, nnz);
   const int64_t blocks = nl2k::ceil_div(M, kThreads / (L * G));
   const dim3 grid((unsigned)blocks), block(kThreads);
 #define SPMM_FWD(LL, GG, VV)                                                                    \
   hipLaunchKernelGGL((spmm_fwd_kernel<I, LL, GG, VV>), grid, block, 0, stream, ptr, col, vals, X, \
                      Y, M, K, D, nnz)
-#define SPMM_FWD_L16(VV)              \
-  if (G == 1) SPMM_FWD(16, 1, VV);    \
-  else if (G == 2) SPMM_FWD(16, 2, VV); \
-  else SPMM_FWD(16, 4, VV)
-#define SPMM_FWD_L4(VV)               \
-  if (G == 1) SPMM_FWD(4, 1, VV);     \
+#define SPMM_FWD_L4(VV)                 \
+  if (G == 1) SPMM_FWD(4, 1, VV);       \
   else if (G == 2) SPMM_FWD(4, 2, VV);  \
   else if (G == 4) SPMM_FWD(4, 4, VV);  \
   else if (G == 8) SPMM_FWD(4, 8, VV);  \
   else SPMM_FWD(4, 16, VV)
-  if (vec) {
-    if (L == 4) { SPMM_FWD_L4(true); }
-    else if (L == 16) { SPMM_FWD_L16(true); }
-    else SPMM_FWD(64, 1, true);
+  if (D < 4) {
+    SPMM_FWD_L4(false);
+  } else if (L == 4) {
+    SPMM_FWD_L4(true);
+  } else if (L == 8) {
+    if (G == 1) SPMM_FWD(8, 1, true);
+    else if (G == 2) SPMM_FWD(8, 2, true);
+    else if (G == 4) SPMM_FWD(8, 4, true);
+    else SPMM_FWD(8, 8, true);
+  } else if (L == 16) {
+    if (G == 1) SPMM_FWD(16, 1, true);
+    else if (G == 2) SPMM_FWD(16, 2, true);
+    else SPMM_FWD(16, 4, true);
+  } else if (L == 32) {
+    if (G == 1) SPMM_FWD(32, 1, true);
+    else SPMM_FWD(32, 2, true);
   } else {
-    if (L == 4) { SPMM_FWD_L4(false); }
-    else if (L == 16) { SPMM_FWD_L16(false); }
-    else SPMM_FWD(64, 1, false);
+    SPMM_FWD(64, 1, true);
   }
 #undef SPMM_FWD_L4
-#undef SPMM_FWD_L16
 #undef SPMM_FWD
   return nl2k::check_launch(who);
 }
@@ -2305,6 +2713,30 @@ int col_block_backward(const ColBlockPlan& cp, const I* ptr, const I* col, const
   return nl2k::check_launch(who);
 }
 
+// dvals for D beyond one gather pass: the row-wise kernel, without dX.
+template <typename I>
+int row_dvals(const I* ptr, const I* col, const float* vals, const float* X, const float* dY,
+              float* dvals, int64_t M, int64_t K, int64_t D, int64_t nnz, hipStream_t stream,
+              const char* who) {
+  const bool vr = D % 4 == 0 && nl2k::aligned16(X) && nl2k::aligned16(dY);
+  const int Lr = lanes_for(D, vr);
+  const dim3 rgrid((unsigned)nl2k::ceil_div(M, kThreads / Lr));
+#define SPMM_DV(LL, VV)                                                                        \
+  hipLaunchKernelGGL((spmm_bwd_kernel<I, LL, VV>), rgrid, dim3(kThreads), 0, stream, ptr, col, vals, X, \
+                     dY, dvals, (float*)nullptr, M, K, D, nnz)
+  if (vr) {
+    if (Lr == 4) SPMM_DV(4, true);
+    else if (Lr == 16) SPMM_DV(16, true);
+    else SPMM_DV(64, true);
+  } else {
+    if (Lr == 4) SPMM_DV(4, false);
+    else if (Lr == 16) SPMM_DV(16, false);
+    else SPMM_DV(64, false);
+  }
+#undef SPMM_DV
+  return nl2k::check_launch(who);
+}
+
 template <typename I>
 int transpose_backward(const TransposePlan& tp, const I* ptr, const I* col, const float* vals,
                        const float* X, const float* dY, float* dvals, float* dX, int64_t M,
@@ -2367,24 +2799,105 @@ int transpose_backward(const TransposePlan& tp, const I* ptr, const I* col, cons
 #undef SPMM_T
   st = nl2k::check_launch(who);
   if (st || dvals == nullptr || dv) return st;
-  // dvals for D beyond one gather pass: the row-wise kernel, without dX
-  const bool vr = D % 4 == 0 && nl2k::aligned16(X) && nl2k::aligned16(dY);
-  const int Lr = lanes_for(D, vr);
-  const dim3 rgrid((unsigned)nl2k::ceil_div(M, kThreads / Lr));
-#define SPMM_DV(LL, VV)                                                                        \
-  hipLaunchKernelGGL((spmm_bwd_kernel<I, LL, VV>), rgrid, block, 0, stream, ptr, col, vals, X, \
-                     dY, dvals, (float*)nullptr, M, K, D, nnz)
-  if (vr) {
-    if (Lr == 4) SPMM_DV(4, true);
-    else if (Lr == 16) SPMM_DV(16, true);
-    else SPMM_DV(64, true);
-  } else {
-    if (Lr == 4) SPMM_DV(4, false);
-    else if (Lr == 16) SPMM_DV(16, false);
-    else SPMM_DV(64, false);
-  }
-#undef SPMM_DV
-  return nl2k::check_launch(who);
+  return row_dvals<I>(ptr, col, vals, X, dY, dvals, M, K, D, nnz, stream, who);
+}
+
+// dX by column buckets (spmm_c_* kernels): D > 1, K past the column-major
+// copy's limit.  Buckets of a power of two of columns, as many as keep an
+// average bucket's entries within one round of the gather and its rows within
+// kCbFloats.  Workspace: counts [nb], cursors [nb], the number of parts, parts
+// (16 B each), records [nnz] (16 B).
+struct ColBucketPlan {
+  bool use = false;
+  int shift = 0, nb = 0;
+  int64_t n_parts = 0;  // at most
+  size_t off_cursor = 0, off_n = 0, off_parts = 0, off_rec = 0, bytes = 0;
+};
+
+ColBucketPlan col_bucket_plan(int64_t M, int64_t K, int64_t D, int64_t nnz) {
+  ColBucketPlan p;
+  if (D <= 1 || M <= 0 || M > INT32_MAX || nnz <= 0 || nnz > INT32_MAX / 2 ||
+      K <= kTransposeMaxCols || 2 * D > kCbFloats)
+    return p;
+  const double avg = (double)nnz / (double)K;
+  int shift = 1;
+  while ((2 << shift) <= kCbMaxCols && ((int64_t)2 << shift) * D <= kCbFloats &&
+         (double)(2 << shift) * avg <= 0.9 * kCbCap)
+    ++shift;
+  const int64_t nb = nl2k::ceil_div(K, (int64_t)1 << shift);
+  if (nb > kCbMaxBuckets) return p;
+  p.use = true;
+  p.shift = shift;
+  p.nb = (int)nb;
+  p.n_parts = nb + nnz / kCbPart;
+  p.off_cursor = align256((size_t)nb * sizeof(int));
+  p.off_n = p.off_cursor + align256((size_t)nb * sizeof(int));
+  p.off_parts = p.off_n + 256;
+  p.off_rec = p.off_parts + align256((size_t)p.n_parts * 16);
+  p.bytes = p.off_rec + align256((size_t)nnz * 16);
+  return p;
+}
+
+template <typename I>
+int col_bucket_backward(const ColBucketPlan& bp, const I* ptr, const I* col, const float* vals,
+                        const float* X, const float* dY, float* dvals, float* dX, int64_t M,
+                        int64_t K, int64_t D, int64_t nnz, char* ws, hipStream_t stream,
+                        const char* who) {
+  int* count = reinterpret_cast<int*>(ws);
+  int* cursor = reinterpret_cast<int*>(ws + bp.off_cursor);
+  int* n_parts = reinterpret_cast<int*>(ws + bp.off_n);
+  i32x4_t* part_of = reinterpret_cast<i32x4_t*>(ws + bp.off_parts);
+  i32x4_t* crec = reinterpret_cast<i32x4_t*>(ws + bp.off_rec);
+  hipLaunchKernelGGL(spmm_c_zero_kernel, dim3((unsigned)nl2k::ceil_div(bp.nb, kThreads)),
+                     dim3(kThreads), 0, stream, count, bp.nb);
+  int st = nl2k::check_launch(who);
+  if (st) return st;
+  const size_t lds = (size_t)bp.nb * sizeof(int);
+  hipLaunchKernelGGL((spmm_c_hist_kernel<I>), dim3((unsigned)nl2k::ceil_div(nnz, kCbHistTile)),
+                     dim3(kCbThreads), lds, stream, col, count, K, nnz, bp.shift, bp.nb);
+  st = nl2k::check_launch(who);
+  if (st) return st;
+  hipLaunchKernelGGL(spmm_c_scan_kernel, dim3(1), dim3(kCbScanThreads), 0, stream, count, cursor,
+                     part_of, n_parts, bp.nb);
+  st = nl2k::check_launch(who);
+  if (st) return st;
+  const int nt = nnz >= kCbLongNnz ? 1024 : 512;
+  auto* scatter = nt == 1024 ? &spmm_c_scatter_kernel<I, 1024, 8> : &spmm_c_scatter_kernel<I, 512, 4>;
+  const int64_t tile = nt == 1024 ? 1024 * 8 : 512 * 4;
+  hipLaunchKernelGGL(scatter, dim3((unsigned)nl2k::ceil_div(nnz, tile)), dim3(nt), lds, stream,
+                     ptr, col, vals, cursor, crec, part_of, n_parts, dX, M, K, D, nnz, bp.shift,
+                     bp.nb);
+  st = nl2k::check_launch(who);
+  if (st) return st;
+  const int mode = D < 4 ? kCbScalar : D % 4 == 0 ? kCbVec : kCbTail;
+  const int64_t units = D < 4 ? D : nl2k::ceil_div(D, (int64_t)4);
+  const int L = row_lanes(units);
+  const bool dv = dvals != nullptr && units <= L;
+  auto pick = [&](auto m, auto w) {
+    constexpr int MM = decltype(m)::value;
+    constexpr bool DD = decltype(w)::value;
+    return L == 4    ? &spmm_c_gather_kernel<4, MM, DD>
+           : L == 8  ? &spmm_c_gather_kernel<8, MM, DD>
+           : L == 16 ? &spmm_c_gather_kernel<16, MM, DD>
+           : L == 32 ? &spmm_c_gather_kernel<32, MM, DD>
+                     : &spmm_c_gather_kernel<64, MM, DD>;
+  };
+  auto pick_dv = [&](auto m) {
+    return dv ? pick(m, std::true_type{}) : pick(m, std::false_type{});
+  };
+  auto* kernel = mode == kCbVec    ? pick_dv(std::integral_constant<int, kCbVec>{})
+                 : mode == kCbTail ? pick_dv(std::integral_constant<int, kCbTail>{})
+                 : dv              ? &spmm_c_gather_kernel<4, kCbScalar, true>
+                                   : &spmm_c_gather_kernel<4, kCbScalar, false>;
+  const size_t rows = ((size_t)1 << bp.shift) * (size_t)D * sizeof(float);
+  const size_t glds = kCbCap * sizeof(i32x4_t) + (dv ? 2 : 1) * rows;
+  st = nl2k::raise_dynamic_lds(reinterpret_cast<const void*>(kernel), (int)glds);
+  if (st) return st;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)bp.n_parts), dim3(kCbThreads), glds, stream, crec,
+                     part_of, n_parts, X, dY, dX, dvals, M, K, D, nnz, bp.shift);
+  st = nl2k::check_launch(who);
+  if (st || dvals == nullptr || dv) return st;
+  return row_dvals<I>(ptr, col, vals, X, dY, dvals, M, K, D, nnz, stream, who);
 }
 
 // Xg != nullptr (D == 1 only): dvals reads the forward's gathered copy of X
@@ -2469,6 +2982,13 @@ int backward(const I* ptr, const I* col, const float* vals, const float* X, cons
     return transpose_backward<I>(tp, ptr, col, vals, X, dY, dvals, dX, M, K, D, nnz,
                                  static_cast<char*>(workspace), stream, who);
   }
+  // Column buckets when the caller's workspace holds their records, else
+  // atomics (which need none).
+  const ColBucketPlan kp = col_bucket_plan(M, K, D, nnz);
+  if (dX && kp.use && workspace != nullptr && ws_bytes >= kp.bytes &&
+      (reinterpret_cast<uintptr_t>(workspace) & 255u) == 0)
+    return col_bucket_backward<I>(kp, ptr, col, vals, X, dY, dvals, dX, M, K, D, nnz,
+                                  static_cast<char*>(workspace), stream, who);
   if (dX) {
     const int64_t n = K * D;
     const unsigned fb = (unsigned)std::min<int64_t>(nl2k::ceil_div(n, kThreads), 4096);
@@ -2579,6 +3099,12 @@ size_t spmv_backward_workspace_bytes(int64_t M, int64_t K, int64_t D, int64_t nn
   if (validate(M, K, D, nnz, INT64_MAX / 2, "spmv_backward_workspace_bytes")) return 0;
   // the int64-index layout, which also serves int32 indices
   return workspace_bytes_for<int64_t>(M, K, D, nnz);
+}
+
+size_t spmv_backward_best_workspace_bytes(int64_t M, int64_t K, int64_t D, int64_t nnz) {
+  if (validate(M, K, D, nnz, INT64_MAX / 2, "spmv_backward_best_workspace_bytes")) return 0;
+  const ColBucketPlan kp = col_bucket_plan(M, K, D, nnz);
+  return kp.use ? kp.bytes : workspace_bytes_for<int64_t>(M, K, D, nnz);
 }
 
 size_t spmv_status_offset(int64_t M, int64_t K, int64_t D, int64_t nnz) {

@@ -48,6 +48,8 @@ def bind_library(lib):
                   [V, V, V, V, V, V, V, V, I64, I64, I64, I64, V, capi.c_size_t, V])
         capi.bind(lib, f"spmv_check_structure_{t}", [V, V, I64, I64, I64, V, V])
     capi.bind(lib, "spmv_backward_workspace_bytes", [I64, I64, I64, I64], restype=capi.c_size_t)
+    capi.bind(lib, "spmv_backward_best_workspace_bytes", [I64, I64, I64, I64],
+              restype=capi.c_size_t)
     capi.bind(lib, "spmv_status_offset", [I64, I64, I64, I64], restype=capi.c_size_t)
     capi.bind_last_error(lib, "spmv_last_error")
     return lib
@@ -158,7 +160,7 @@ def spmv_backward(row_ptr, col_idx, vals, X, grad_Y, need_vals=True, need_X=True
         check_structure(row_ptr, col_idx, K)
     grad_vals = torch.empty_like(vals) if need_vals else None
     grad_X = torch.empty_like(X) if need_X else None
-    ws_bytes = lib.spmv_backward_workspace_bytes(M, K, D, vals.numel()) if need_X else 0
+    ws_bytes = lib.spmv_backward_best_workspace_bytes(M, K, D, vals.numel()) if need_X else 0
     ws = torch.empty(max(ws_bytes, 8), dtype=torch.uint8, device=X.device)  # scratch
     status = None
     if need_X and capi.checking() and not torch.cuda.is_current_stream_capturing():

@@ -1,0 +1,103 @@
+"""SpMM where a row or column crosses the edges of its kernels: the backward's
+column buckets (more than 16384 columns: bucket and part edges, columns that
+hold most of the entries, widths with a ragged last lane) and the forward's
+rows shared by a workgroup (more than 64 entries per lane group).  Against
+float64, at a 2-norm error of 2^-24 sqrt(n) / sqrt(3) of the result (n
+roundings of a sum of n independent terms), n the longest row or column, and
+three roundings more."""
+
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from conftest import announce
+
+pytestmark = pytest.mark.gpu
+
+
+def _csr(lens, k, seed, hub):
+    g = np.random.default_rng(seed)
+    ptr = np.concatenate([[0], np.cumsum(lens)])
+    col = g.integers(0, k, ptr[-1])
+    if hub:  # half of the entries in three columns, one of them the last
+        at = g.random(ptr[-1]) < 0.5
+        col[at] = g.choice([0, 777, k - 1], int(at.sum()))
+    return torch.from_numpy(ptr), torch.from_numpy(col)
+
+
+def _check(lens, k, d, idx, hub=False, seed=0):
+    from cases.spmv import op
+    announce(f"spmm buckets rows={len(lens)} K={k} D={d} {idx} hub={hub}")
+    ptr, col = _csr(np.asarray(lens), k, seed, hub)
+    m, nnz = len(lens), col.numel()
+    g = torch.Generator().manual_seed(seed)
+    vals, X, G = (torch.randn(*s, generator=g) for s in ((nnz,), (k, d), (m, d)))
+    v, x = vals.cuda().requires_grad_(True), X.cuda().requires_grad_(True)
+    Y = op.candidate({"row_ptr": ptr.to(idx).cuda(), "col_idx": col.to(idx).cuda(), "vals": v,
+                      "X": x}, {})
+    dv, dx = torch.autograd.grad(Y, [v, x], G.cuda())
+    torch.cuda.synchronize()
+    rows = torch.repeat_interleave(torch.arange(m), ptr[1:] - ptr[:-1])
+    vd, Xd, Gd = vals.double(), X.double(), G.double()
+    want = {"Y": (Y, torch.zeros(m, d, dtype=torch.float64).index_add_(
+                      0, rows, vd[:, None] * Xd[col]), int(max(lens))),
+            "dvals": (dv, (Gd[rows] * Xd[col]).sum(1), d),
+            "dX": (dx, torch.zeros(k, d, dtype=torch.float64).index_add_(
+                      0, col, vd[:, None] * Gd[rows]), int(torch.bincount(col).max()))}
+    for name, (got, ref, n) in want.items():
+        tol = 2.0 ** -24 * (3 + math.sqrt(n / 3))
+        err = float((got.detach().cpu().double() - ref).norm() / ref.norm())
+        print(f"  {name}: {err:.2e} of {tol:.2e}")
+        assert err <= tol, name
+
+
+@pytest.mark.parametrize("d", [2, 3, 4, 5, 7, 32, 33, 64, 127, 130, 256, 300])
+@pytest.mark.parametrize("k", [16385, 40001])
+def test_spmm_column_buckets(k, d):
+    lens = np.random.default_rng(d).integers(0, 30, 700)
+    _check(lens, k, d, torch.int64 if d % 2 else torch.int32, seed=d)
+
+
+@pytest.mark.parametrize("d", [4, 33])
+@pytest.mark.parametrize("m,mean", [(3000, 20), (9000, 70)])
+def test_spmm_hub_columns(m, mean, d):
+    """Buckets of several parts (over 8192 entries, added with atomics) and
+    columns that cross from one lane group to the next; 9000 x 70 entries
+    take the larger scatter tiles."""
+    lens = np.full(m, mean)
+    _check(lens, 20000, d, torch.int32, hub=True, seed=m)
+
+
+@pytest.mark.parametrize("d", [1 + 1, 6, 16, 20, 40, 100, 260])
+def test_spmm_long_rows(d):
+    """Rows one short of, at and past the length a workgroup shares, between
+    empty and single-entry ones."""
+    lens = [0, 1, 63, 64, 65, 127, 128, 129, 255, 257, 1, 0, 513, 1025, 2, 3000, 0, 1] * 3 + [4000]
+    _check(lens, 500, d, torch.int64, seed=d)
+
+
+def test_spmm_bucket_route_needs_its_workspace():
+    """A caller with the smaller workspace (none, past 16384 columns) still
+    gets dX, through atomics."""
+    from cases.spmv import op
+    from framework import capi
+    m, k, d = 900, 20000, 8
+    announce("spmm without the bucket workspace")
+    lib = op._lib()
+    ptr, col = _csr(np.full(m, 11), k, 1, False)
+    nnz = col.numel()
+    assert lib.spmv_backward_workspace_bytes(m, k, d, nnz) == 0
+    assert lib.spmv_backward_best_workspace_bytes(m, k, d, nnz) >= 16 * nnz
+    ptr, col = ptr.int().cuda(), col.int().cuda()
+    vals, X, G = torch.randn(nnz).cuda(), torch.randn(k, d).cuda(), torch.randn(m, d).cuda()
+    dv0, dx0 = op.spmv_backward(ptr, col, vals, X, G)
+    dv, dx = torch.empty_like(vals), torch.empty_like(X)
+    P = capi.ptr
+    st = lib.spmv_backward_f32_i32(P(ptr), P(col), P(vals), P(X), P(G), P(dv), P(dx), m, k, d, nnz,
+                                   None, 0, capi.stream_of(X))
+    capi.check(st, lib.spmv_last_error, "spmv_backward")
+    torch.cuda.synchronize()
+    assert float((dx - dx0).norm() / dx0.norm()) < 1e-6
+    assert float((dv - dv0).norm() / dv0.norm()) < 1e-6
