@@ -27,15 +27,17 @@
 //    workgroup scheme with a shared counter measured slower: 1024 atomics on
 //    one address serialise.)
 //  * Backward: lse saved by the forward turns the gradient into a pure
-//    streaming pass (read logits, write dlogits, no reductions).  Rows of
-//    more than 1024 classes are laid out like the forward, so each row's lse
-//    and label are read once; shorter rows use a flat grid-stride kernel.
+//    streaming pass (read logits, write dlogits, no reductions).  Aligned
+//    float4 rows of 1025 to 8192 classes are laid out like the forward, so
+//    each row's lse and label are read once; the others stream flat, four
+//    floats a lane whatever the rows.
 //  * A label outside [0, C) makes its row's loss term and gradient NaN (the
 //    reference would index out of the row; torch raises).
 //  * Unaligned rows (or C % 4 != 0) of at most 32 classes take a lane each
-//    in the forward.  C not a multiple of 4, misaligned rows or C > 8192 take a
-//    workgroup per row in the forward (one pass with a running maximum,
-//    float4 loads when aligned) and the flat backward.
+//    in the forward; rows of more than 8192 classes take a workgroup each (one
+//    pass with a running maximum).  Rows start at any 4-byte boundary: the
+//    loads are 16 bytes all the same, a row's last one reaching back over what
+//    the one before holds.
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
@@ -47,6 +49,19 @@
 using nl2k::f32x4;
 
 namespace {
+
+// 16 bytes at any 4-byte boundary.
+typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
+
+// Window i of a row of C >= 4 floats: columns 4i .. 4i + 3, or the row's last
+// four for its last window.  `skip`: how many of those the window before
+// holds already (C no multiple of 4).
+__device__ __forceinline__ f32x4 load_window(const float* __restrict__ row, int64_t i, int64_t C,
+                                             int& skip) {
+  const int64_t c = min(4 * i, C - 4);
+  skip = (int)(4 * i - c);
+  return *reinterpret_cast<const f32x4_u*>(row + c);
+}
 
 constexpr int kBlock = 256;
 constexpr float kLog2e = 1.4426950408889634f;
@@ -151,6 +166,10 @@ __device__ void sum_partials(const unsigned long long* __restrict__ slots, nl2k:
 // Thread 0 of each row group keeps its rows' loss terms in row order; the
 // workgroup's sum (groups added in a fixed order) is published in slot pair
 // blockIdx.x, and workgroup 0 then adds all partials (sum_partials).
+// !FULL: any width, at any alignment, the last window of a row that is no
+// multiple of four reaching back (its repeated columns count as -inf).  Against
+// a workgroup per row there, us: [65536, 99] 118.6 -> 7.8, [65536, 257] 153.6 ->
+// 25.5, [16384, 1001] 41.2 -> 12.6, [8192, 4097] 32.6 -> 28.2.
 template <int TPR, int V, bool FULL>
 __global__ __launch_bounds__(kBlock) void sce_fwd_kernel(
     const float* __restrict__ logits, const int64_t* __restrict__ labels,
@@ -163,7 +182,7 @@ __global__ __launch_bounds__(kBlock) void sce_fwd_kernel(
   __shared__ float sacc[RPB];
   const int t = threadIdx.x % TPR;
   const int grp = threadIdx.x / TPR;
-  const int C4 = C >> 2;
+  const int W = (C + 3) >> 2;
   float acc = 0.f;
   for (int64_t base = (int64_t)blockIdx.x * RPI; base < B; base += (int64_t)gridDim.x * RPI) {
     f32x4 v[R][V];
@@ -176,10 +195,11 @@ __global__ __launch_bounds__(kBlock) void sce_fwd_kernel(
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      const f32x4* xr =
-          reinterpret_cast<const f32x4*>(logits + min(base + r * RPB + grp, B - 1) * C);
+      const float* xr = logits + min(base + r * RPB + grp, B - 1) * C;
 #pragma unroll
-      for (int k = 0; k < V; ++k) v[r][k] = xr[FULL ? t + k * TPR : min(t + k * TPR, C4 - 1)];
+      for (int k = 0; k < V; ++k)
+        v[r][k] = *reinterpret_cast<const f32x4_u*>(
+            xr + (FULL ? 4 * (t + k * TPR) : min(4 * (t + k * TPR), C - 4)));
     }
     __builtin_amdgcn_sched_barrier(0);
     // the label's logit, addressed by the labels loaded first (column 0 for
@@ -189,19 +209,32 @@ __global__ __launch_bounds__(kBlock) void sce_fwd_kernel(
       xl[r] = logits[min(base + r * RPB + grp, B - 1) * C + max(label_col(lab[r], C), 0)];
     // keep every load above any use of the row data
     __builtin_amdgcn_sched_barrier(0);
+    // windows past the row, and what its last window repeats, count as -inf
+    if constexpr (!FULL) {
+#pragma unroll
+      for (int k = 0; k < V; ++k) {
+        const int c = t + k * TPR;
+        const int skip = c < W ? max(4 * c - (C - 4), 0) : 4;
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+          for (int u = 0; u < 4; ++u) v[r][k][u] = u < skip ? -INFINITY : v[r][k][u];
+      }
+    }
     float m[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       m[r] = -INFINITY;
 #pragma unroll
       for (int k = 0; k < V; ++k) {
-        const bool ok = FULL || t + k * TPR < C4;
         const f32x4 x = v[r][k];
-        const float mk = fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]));
-        m[r] = fmaxf(m[r], ok ? mk : -INFINITY);
+        m[r] = fmaxf(m[r], fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])));
       }
     }
     row_reduce<TPR, R, true>(m, red);
+    // a row of -inf alone: lse = -inf (exp(-inf - 0) adds 0), not -inf - -inf
+#pragma unroll
+    for (int r = 0; r < R; ++r) m[r] = m[r] == -INFINITY ? 0.f : m[r];
     float se[R];  // per row: sum of exp(x - max)
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -211,7 +244,7 @@ __global__ __launch_bounds__(kBlock) void sce_fwd_kernel(
         float e4 = 0.f;
 #pragma unroll
         for (int u = 0; u < 4; ++u) e4 += __builtin_amdgcn_exp2f((v[r][k][u] - m[r]) * kLog2e);
-        se[r] += (FULL || t + k * TPR < C4) ? e4 : 0.f;
+        se[r] += e4;
       }
     }
     row_reduce<TPR, R, false>(se, red);
@@ -238,59 +271,48 @@ __global__ __launch_bounds__(kBlock) void sce_fwd_kernel(
   if (blockIdx.x == 0) sum_partials(slots, key, (int)gridDim.x, B, loss, red);
 }
 
-// Forward for the rows the row-cached kernel does not take (C % 4 != 0,
-// misaligned rows, C > 8192): a workgroup per row, one pass over it.  Each
-// thread keeps a running maximum m and the sum s of exp(x - m) over its
-// elements, taken in chunks of U loads issued together (float4 loads when
-// VEC); a chunk that raises the maximum rescales s once.  The row maximum M
+// Forward for the rows the row-cached kernel does not take (C > 8192): a
+// workgroup per row, one pass over it.  Each thread keeps a running maximum m
+// and the sum s of exp(x - m) over its windows of four columns, taken U at a
+// time; a chunk that raises the maximum rescales s once.  The row maximum M
 // is the workgroup's fmax of the m's and the row sum the workgroup's sum of
 // s exp(m - M), both in a fixed order.  Against two passes over the row
 // (the second from L2) with one float per load: 92.7 against 401 us at
-// [4096, 32000], 94.0 against 478 at [1024, 128256], 77.3 against 329 at
-// [2048, 50257].
-template <bool VEC>
+// [4096, 32000], 94.0 against 478 at [1024, 128256].  Eight windows in flight
+// against four: 13.6 -> 10.6 us at [100, 50257], the same on full grids.
 __global__ __launch_bounds__(kBlock) void sce_fwd_long_kernel(
     const float* __restrict__ logits, const int64_t* __restrict__ labels,
     float* __restrict__ lse_out, unsigned long long* __restrict__ slots, nl2k::slots::Key key,
     float* __restrict__ loss, int64_t B, int64_t C) {
-  constexpr int U = VEC ? 4 : 16;  // loads per thread per chunk
-  constexpr int W = VEC ? 4 : 1;   // floats per load
+  constexpr int U = 8;  // loads per thread per chunk
   __shared__ float red[4];
   float acc = 0.f;
-  const int64_t n = VEC ? C / 4 : C;  // loads per row
+  const int64_t n = (C + 3) / 4;  // windows per row
   for (int64_t row = blockIdx.x; row < B; row += gridDim.x) {
     const float* xr = logits + row * C;
     float m = -INFINITY, s = 0.f;
     for (int64_t base = threadIdx.x; base < n; base += (int64_t)kBlock * U) {
-      float v[U][W];
+      f32x4 v[U];
+      int skip[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int64_t i = min(base + (int64_t)u * kBlock, n - 1);  // clamped: no branch
-        if constexpr (VEC) {
-          const f32x4 q = reinterpret_cast<const f32x4*>(xr)[i];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) v[u][e] = q[e];
-        } else {
-          v[u][0] = xr[i];
-        }
+      for (int u = 0; u < U; ++u) {  // clamped: no branch
+        const int64_t i = base + (int64_t)u * kBlock;
+        v[u] = load_window(xr, min(i, n - 1), C, skip[u]);
+        skip[u] = i < n ? skip[u] : 4;
       }
       float cm = -INFINITY;
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const bool ok = base + (int64_t)u * kBlock < n;
+      for (int u = 0; u < U; ++u)
 #pragma unroll
-        for (int e = 0; e < W; ++e) cm = fmaxf(cm, ok ? v[u][e] : -INFINITY);
-      }
+        for (int e = 0; e < 4; ++e) cm = fmaxf(cm, e >= skip[u] ? v[u][e] : -INFINITY);
       const float nm = fmaxf(m, cm);
       if (nm != -INFINITY) {  // nothing but -inf so far adds nothing
         float cs = 0.f;
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const bool ok = base + (int64_t)u * kBlock < n;
+        for (int u = 0; u < U; ++u)
 #pragma unroll
-          for (int e = 0; e < W; ++e)
-            cs += ok ? __builtin_amdgcn_exp2f((v[u][e] - nm) * kLog2e) : 0.f;
-        }
+          for (int e = 0; e < 4; ++e)
+            cs += e >= skip[u] ? __builtin_amdgcn_exp2f((v[u][e] - nm) * kLog2e) : 0.f;
         s = s * __builtin_amdgcn_exp2f((m - nm) * kLog2e) + cs;
         m = nm;
       }
@@ -413,6 +435,51 @@ __global__ __launch_bounds__(kBlock) void sce_bwd_rows_kernel(
   }
 }
 
+// Backward of long rows whose width or alignment the vector kernels don't
+// take: a workgroup per segment of `per` <= kBlock * U windows of four columns
+// of one row (a row in equal segments), so the row's lse and label are scalar
+// loads and nothing is shared.  The row's last window reaches back
+// over columns its neighbour stores too, with the same bits.
+// Bound by memory.  Against the flat kernel below, element by element:
+// [4096, 50257] 415 -> 305 us (5.4 TB/s), [1000, 128257] 259 -> 187, [8192,
+// 2049] 26.4 -> 22.0, [16384, 777] 20.4 -> 17.0; rows of a few hundred classes
+// leave lanes idle here ([65536, 257] 29.0 -> 34.3), and aligned float4 rows
+// stream better flat ([4096, 32000] 198 against 209).
+constexpr int64_t kLongClasses = 512;
+template <int U>
+__global__ __launch_bounds__(kBlock) void sce_bwd_long_kernel(
+    const float* __restrict__ logits, const int64_t* __restrict__ labels,
+    const float* __restrict__ lse, const float* __restrict__ gout,
+    float* __restrict__ dlogits, int64_t B, int64_t C, uint32_t segs, int64_t per) {
+  const int64_t row = blockIdx.x / segs;
+  const int64_t first = (int64_t)(blockIdx.x - (uint32_t)row * segs) * per;
+  const int64_t n = min((C + 3) / 4, first + per);
+  const int64_t w0 = first + threadIdx.x;
+  const float* xr = logits + row * C;
+  float* dr = dlogits + row * C;
+  f32x4 v[U];
+#pragma unroll
+  for (int k = 0; k < U; ++k) {
+    int skip;
+    v[k] = load_window(xr, min(w0 + k * kBlock, n - 1), C, skip);
+  }
+  const float l = lse[row];
+  const int lab = label_col(labels[row], C);
+  const float bad = lab >= 0 ? 0.f : NAN;
+  const float scale = gout[0] / (float)B;
+#pragma unroll
+  for (int k = 0; k < U; ++k) {
+    const int64_t i = w0 + k * kBlock;
+    const int64_t c = min(4 * i, C - 4);
+    f32x4 o;
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      o[u] = scale * (__builtin_amdgcn_exp2f((v[k][u] - l) * kLog2e) - (c + u == lab ? 1.f : 0.f)) +
+             bad;
+    if (i < n) *reinterpret_cast<f32x4_u*>(dr + c) = o;
+  }
+}
+
 // Flat backward for the shapes the row-cached kernel does not take:
 // dlogits = gout / B * (exp(x - lse) - onehot); VEC: C % 4 == 0 and aligned
 // rows, one float4 per thread step.
@@ -451,7 +518,6 @@ __global__ __launch_bounds__(kBlock) void sce_bwd_kernel(
 struct FwdPlan {
   bool cached = false;  // row-cached kernel
   int lane_cm = 0;      // > 0: lane-per-row kernel for rows of at most lane_cm classes
-  bool vec = false;     // long-row kernel: float4 loads
   int tpr = 64, v = 4;
   unsigned blocks = 1;  // forward workgroups, one partial loss each
 };
@@ -462,9 +528,9 @@ FwdPlan plan_forward(int64_t B, int64_t C, bool aligned) {
   if (C <= 32 && !(aligned && C % 4 == 0)) {
     p.lane_cm = C <= 8 ? 8 : C <= 16 ? 16 : 32;
     rows_per_step = kBlock;
-  } else if (aligned && C % 4 == 0 && C <= 8192) {
+  } else if (C <= 8192) {
     p.cached = true;
-    const int64_t c4 = C / 4;
+    const int64_t c4 = (C + 3) / 4;
     if (c4 <= 32) { p.tpr = 16; p.v = c4 <= 16 ? 1 : 2; }
     else if (c4 <= 64) { p.tpr = 64; p.v = 1; }
     else if (c4 <= 256) { p.tpr = 64; p.v = 4; }
@@ -472,8 +538,6 @@ FwdPlan plan_forward(int64_t B, int64_t C, bool aligned) {
     const int r = p.v == 1 ? rows_in_flight<1>() : p.v == 2 ? rows_in_flight<2>()
                                                             : rows_in_flight<4>();
     rows_per_step = (kBlock / p.tpr) * r;
-  } else {
-    p.vec = aligned && C % 4 == 0;
   }
   // B == 0 still runs one workgroup: its partial is 0 and its loss sum
   // writes loss = 0 / 0 = NaN (the mean of no terms, as torch's mean of an
@@ -530,7 +594,7 @@ int softmax_ce_forward_f32(const float* logits, const int64_t* labels, float* lo
   if (p.cached && B > 0) {
 #define SCE_FWD(TPR, V)                                                                        \
   do {                                                                                         \
-    if (C / 4 == (TPR) * (V))                                                                  \
+    if (C == 4 * (TPR) * (V))                                                                  \
       hipLaunchKernelGGL((sce_fwd_kernel<TPR, V, true>), grid, dim3(kBlock), 0, stream, logits, \
                          labels, lse, slots, key, loss, B, (int)C);                            \
     else                                                                                       \
@@ -554,12 +618,9 @@ int softmax_ce_forward_f32(const float* logits, const int64_t* labels, float* lo
   } else if (p.lane_cm == 32) {
     hipLaunchKernelGGL(sce_fwd_lane_kernel<32>, grid, dim3(kBlock), 0, stream, logits, labels,
                        lse, slots, key, loss, B, (int)C);
-  } else if (p.vec) {
-    hipLaunchKernelGGL(sce_fwd_long_kernel<true>, grid, dim3(kBlock), 0, stream, logits, labels,
-                       lse, slots, key, loss, B, C);
   } else {
-    hipLaunchKernelGGL(sce_fwd_long_kernel<false>, grid, dim3(kBlock), 0, stream, logits, labels,
-                       lse, slots, key, loss, B, C);
+    hipLaunchKernelGGL(sce_fwd_long_kernel, grid, dim3(kBlock), 0, stream, logits, labels, lse,
+                       slots, key, loss, B, C);
   }
   return nl2k::check_launch(who);
 }
@@ -575,10 +636,10 @@ int softmax_ce_backward_f32(const float* logits, const int64_t* labels, const fl
     return nl2k::fail(NL2K_ERR_NULL, "%s: null pointer argument", who);
   const bool aligned = nl2k::aligned16(logits) && nl2k::aligned16(dlogits);
   const FwdPlan p = plan_forward(B, C, aligned);
-  // Rows of more than 1024 classes use the row kernel; shorter ones, whose
-  // row kernel would keep a wave per row with few float4 per lane, stream
-  // faster through the flat kernel (65536 x 64: 10.7 against 13.9 us).
-  if (p.cached && p.tpr == 256) {
+  // Aligned float4 rows of more than 1024 classes use the row kernel; shorter
+  // ones, whose row kernel would keep a wave per row with few float4 per lane,
+  // stream faster through the flat kernel (65536 x 64: 10.7 against 13.9 us).
+  if (p.cached && p.tpr == 256 && aligned && C % 4 == 0) {
     const dim3 grid(p.blocks);
 #define SCE_BWD(TPR, V)                                                                      \
   do {                                                                                       \
@@ -593,6 +654,16 @@ int softmax_ce_backward_f32(const float* logits, const int64_t* labels, const fl
     else if (p.v == 4) SCE_BWD(256, 4);
     else SCE_BWD(256, 8);
 #undef SCE_BWD
+  } else if (C > kLongClasses && !(aligned && C % 4 == 0)) {
+    const int u = C > 2048 ? 4 : C > 1024 ? 2 : 1;
+    const int64_t windows = nl2k::ceil_div(C, (int64_t)4);
+    const int64_t segs = nl2k::ceil_div(windows, (int64_t)kBlock * u);
+    if (B * segs > INT32_MAX) return nl2k::fail(NL2K_ERR_OVERFLOW, "%s: sizes too large", who);
+    auto* kernel = u == 4   ? &sce_bwd_long_kernel<4>
+                   : u == 2 ? &sce_bwd_long_kernel<2>
+                            : &sce_bwd_long_kernel<1>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(B * segs)), dim3(kBlock), 0, stream, logits, labels,
+                       lse, gout, dlogits, B, C, (uint32_t)segs, nl2k::ceil_div(windows, segs));
   } else {
     const bool vec = C % 4 == 0 && aligned;
     const int64_t work = vec ? B * C / 4 : B * C;
