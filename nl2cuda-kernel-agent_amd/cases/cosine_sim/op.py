@@ -37,6 +37,11 @@ def _lib():
     return bind_library(load_kernel(LIB_NAME, SOURCES, base_dir=KERNEL_DIR))
 
 
+@functools.lru_cache(maxsize=256)
+def _workspace_bytes(N, M, D):
+    return _lib().cosine_sim_backward_workspace_bytes(N, M, D)
+
+
 def _check_pair(A, B):
     capi.require(A.is_cuda and B.is_cuda, "A, B must be GPU tensors")
     capi.require(A.dtype == torch.float32 and B.dtype == torch.float32, "A, B must be float32")
@@ -53,14 +58,13 @@ def cos_forward(A, B, eps):
     A, B = A.contiguous(), B.contiguous()
     N, D = A.shape
     M = B.size(0)
-    S = torch.empty((N, M), dtype=torch.float32, device=A.device)
-    inv_a = torch.empty(N, dtype=torch.float32, device=A.device)
-    inv_b = torch.empty(M, dtype=torch.float32, device=A.device)
-    with torch.cuda.device(A.device):
-        st = lib.cosine_sim_forward_f32(capi.ptr(A), capi.ptr(B), capi.ptr(S), capi.ptr(inv_a),
-                                        capi.ptr(inv_b), N, M, D, float(eps),
-                                        capi.stream_of(A))
-    capi.check(st, lib.cosine_sim_last_error, "cos_forward")
+    S = A.new_empty((N, M))
+    inv_a = A.new_empty(N)
+    inv_b = A.new_empty(M)
+    st = capi.launch(lib.cosine_sim_forward_f32, A.get_device(), A.data_ptr(), B.data_ptr(),
+                     S.data_ptr(), inv_a.data_ptr(), inv_b.data_ptr(), N, M, D, float(eps))
+    if st:
+        capi.check(st, lib.cosine_sim_last_error, "cos_forward")
     return S, inv_a, inv_b
 
 
@@ -68,21 +72,20 @@ def cos_backward(A, B, inv_a, inv_b, dS):
     """(dA, dB) from upstream dS = dL/dS and the forward's inverse norms."""
     _check_pair(A, B)
     N, M = A.size(0), B.size(0)
-    capi.require(dS.is_cuda and dS.dtype == torch.float32 and tuple(dS.shape) == (N, M),
+    capi.require(dS.is_cuda and dS.dtype == torch.float32 and dS.shape == (N, M),
                  "dS must be a float32 GPU tensor of shape [N, M]")
     lib = _lib()
     A, B, dS = A.contiguous(), B.contiguous(), dS.contiguous()
     D = A.size(1)
     dA = torch.empty_like(A)
     dB = torch.empty_like(B)
-    ws_bytes = lib.cosine_sim_backward_workspace_bytes(N, M, D)
-    ws = torch.empty((max(ws_bytes, 4) + 3) // 4, dtype=torch.float32, device=A.device)
-    with torch.cuda.device(A.device):
-        st = lib.cosine_sim_backward_f32(capi.ptr(A), capi.ptr(B), capi.ptr(inv_a),
-                                         capi.ptr(inv_b), capi.ptr(dS), capi.ptr(dA),
-                                         capi.ptr(dB), N, M, D, capi.ptr(ws), ws_bytes,
-                                         capi.stream_of(A))
-    capi.check(st, lib.cosine_sim_last_error, "cos_backward")
+    ws_bytes = _workspace_bytes(N, M, D)
+    ws = A.new_empty((max(ws_bytes, 4) + 3) // 4)
+    st = capi.launch(lib.cosine_sim_backward_f32, A.get_device(), A.data_ptr(), B.data_ptr(),
+                     inv_a.data_ptr(), inv_b.data_ptr(), dS.data_ptr(), dA.data_ptr(),
+                     dB.data_ptr(), N, M, D, ws.data_ptr(), ws_bytes)
+    if st:
+        capi.check(st, lib.cosine_sim_last_error, "cos_backward")
     return dA, dB
 
 

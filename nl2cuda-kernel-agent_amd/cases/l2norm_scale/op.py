@@ -34,6 +34,11 @@ def _lib():
     return bind_library(load_kernel(LIB_NAME, SOURCES, base_dir=KERNEL_DIR))
 
 
+@functools.lru_cache(maxsize=256)
+def _workspace_bytes(N, D):
+    return _lib().l2norm_scale_backward_workspace_bytes(N, D)
+
+
 def _check(X, g):
     capi.require(X.is_cuda and g.is_cuda, "X, g must be GPU tensors")
     capi.require(X.dtype == torch.float32 and g.dtype == torch.float32, "X, g must be float32")
@@ -48,11 +53,11 @@ def l2n_forward(X, g, eps):
     X, g = X.contiguous(), g.contiguous()
     N, D = X.shape
     Y = torch.empty_like(X)
-    norm = torch.empty(N, dtype=torch.float32, device=X.device)
-    with torch.cuda.device(X.device):
-        st = lib.l2norm_scale_forward_f32(capi.ptr(X), capi.ptr(g), capi.ptr(Y), capi.ptr(norm),
-                                          N, D, float(eps), capi.stream_of(X))
-    capi.check(st, lib.l2norm_scale_last_error, "l2n_forward")
+    norm = X.new_empty(N)
+    st = capi.launch(lib.l2norm_scale_forward_f32, X.get_device(), X.data_ptr(), g.data_ptr(),
+                     Y.data_ptr(), norm.data_ptr(), N, D, float(eps))
+    if st:
+        capi.check(st, lib.l2norm_scale_last_error, "l2n_forward")
     return Y, norm
 
 
@@ -66,13 +71,13 @@ def l2n_backward(X, g, G, norm):
     N, D = X.shape
     dX = torch.empty_like(X)
     dg = torch.empty_like(g)
-    ws_bytes = lib.l2norm_scale_backward_workspace_bytes(N, D)
-    ws = torch.empty((max(ws_bytes, 4) + 3) // 4, dtype=torch.float32, device=X.device)
-    with torch.cuda.device(X.device):
-        st = lib.l2norm_scale_backward_f32(capi.ptr(G), capi.ptr(X), capi.ptr(g), capi.ptr(norm),
-                                           capi.ptr(dX), capi.ptr(dg), N, D, capi.ptr(ws),
-                                           ws_bytes, capi.stream_of(X))
-    capi.check(st, lib.l2norm_scale_last_error, "l2n_backward")
+    ws_bytes = _workspace_bytes(N, D)
+    ws = X.new_empty((max(ws_bytes, 4) + 3) // 4)
+    st = capi.launch(lib.l2norm_scale_backward_f32, X.get_device(), G.data_ptr(), X.data_ptr(),
+                     g.data_ptr(), norm.data_ptr(), dX.data_ptr(), dg.data_ptr(), N, D,
+                     ws.data_ptr(), ws_bytes)
+    if st:
+        capi.check(st, lib.l2norm_scale_last_error, "l2n_backward")
     return dX, dg
 
 

@@ -35,9 +35,15 @@ def _lib():
     return bind_library(load_kernel(LIB_NAME, SOURCES, base_dir=KERNEL_DIR))
 
 
+@functools.lru_cache(maxsize=256)
+def _workspace_bytes(B, D):
+    return _lib().layernorm_backward_workspace_bytes(B, D)
+
+
 def _check_inputs(x, gamma, beta):
     capi.require(x.is_cuda and gamma.is_cuda and beta.is_cuda, "X, gamma, beta must be GPU tensors")
-    capi.require(all(t.dtype == torch.float32 for t in (x, gamma, beta)),
+    f32 = torch.float32
+    capi.require(x.dtype == f32 and gamma.dtype == f32 and beta.dtype == f32,
                  "X, gamma, beta must be float32")
     capi.require(x.dim() == 2, "X must have shape [B, D]")
     capi.require(gamma.dim() == 1 and beta.dim() == 1, "gamma, beta must have shape [D]")
@@ -52,21 +58,23 @@ def layernorm_forward(x, gamma, beta, eps):
     x, gamma, beta = x.contiguous(), gamma.contiguous(), beta.contiguous()
     B, D = x.shape
     y = torch.empty_like(x)
-    mean = torch.empty(B, dtype=torch.float32, device=x.device)
-    rstd = torch.empty(B, dtype=torch.float32, device=x.device)
-    with torch.cuda.device(x.device):
-        st = lib.layernorm_forward_f32(capi.ptr(x), capi.ptr(gamma), capi.ptr(beta), capi.ptr(y),
-                                       capi.ptr(mean), capi.ptr(rstd), B, D, float(eps),
-                                       capi.stream_of(x))
-    capi.check(st, lib.layernorm_last_error, "layernorm_forward")
+    mean = x.new_empty(B)
+    rstd = x.new_empty(B)
+    st = capi.launch(lib.layernorm_forward_f32, x.get_device(), x.data_ptr(), gamma.data_ptr(),
+                     beta.data_ptr(), y.data_ptr(), mean.data_ptr(), rstd.data_ptr(), B, D,
+                     float(eps))
+    if st:
+        capi.check(st, lib.layernorm_last_error, "layernorm_forward")
     return y, mean, rstd
 
 
 def layernorm_backward(grad_y, x, gamma, mean, inv_std):
     """Returns (grad_x, grad_gamma, grad_beta) like the reference extension."""
-    capi.require(all(t.is_cuda for t in (grad_y, x, gamma, mean, inv_std)), "inputs must be GPU tensors")
-    capi.require(all(t.dtype == torch.float32 for t in (grad_y, x, gamma, mean, inv_std)),
-                 "inputs must be float32")
+    capi.require(grad_y.is_cuda and x.is_cuda and gamma.is_cuda and mean.is_cuda and
+                 inv_std.is_cuda, "inputs must be GPU tensors")
+    f32 = torch.float32
+    capi.require(grad_y.dtype == f32 and x.dtype == f32 and gamma.dtype == f32 and
+                 mean.dtype == f32 and inv_std.dtype == f32, "inputs must be float32")
     capi.require(grad_y.shape == x.shape and x.dim() == 2, "grad_y and X must have shape [B, D]")
     capi.require(gamma.dim() == 1 and gamma.size(0) == x.size(1), "gamma length must equal D")
     capi.require(mean.shape == (x.size(0),) and inv_std.shape == (x.size(0),),
@@ -76,16 +84,15 @@ def layernorm_backward(grad_y, x, gamma, mean, inv_std):
     mean, inv_std = mean.contiguous(), inv_std.contiguous()
     B, D = x.shape
     dx = torch.empty_like(x)
-    dgamma = torch.empty(D, dtype=torch.float32, device=x.device)
-    dbeta = torch.empty(D, dtype=torch.float32, device=x.device)
-    ws_bytes = lib.layernorm_backward_workspace_bytes(B, D)
-    ws = torch.empty((max(ws_bytes, 16) + 3) // 4, dtype=torch.float32, device=x.device)
-    with torch.cuda.device(x.device):
-        st = lib.layernorm_backward_f32(capi.ptr(grad_y), capi.ptr(x), capi.ptr(gamma),
-                                        capi.ptr(mean), capi.ptr(inv_std), capi.ptr(dx),
-                                        capi.ptr(dgamma), capi.ptr(dbeta), B, D, capi.ptr(ws),
-                                        ws_bytes, capi.stream_of(x))
-    capi.check(st, lib.layernorm_last_error, "layernorm_backward")
+    dgamma = x.new_empty(D)
+    dbeta = x.new_empty(D)
+    ws_bytes = _workspace_bytes(B, D)
+    ws = x.new_empty((max(ws_bytes, 16) + 3) // 4)
+    st = capi.launch(lib.layernorm_backward_f32, x.get_device(), grad_y.data_ptr(), x.data_ptr(),
+                     gamma.data_ptr(), mean.data_ptr(), inv_std.data_ptr(), dx.data_ptr(),
+                     dgamma.data_ptr(), dbeta.data_ptr(), B, D, ws.data_ptr(), ws_bytes)
+    if st:
+        capi.check(st, lib.layernorm_last_error, "layernorm_backward")
     return dx, dgamma, dbeta
 
 

@@ -39,46 +39,62 @@ def _lib():
     return bind_library(load_kernel(LIB_NAME, SOURCES, base_dir=KERNEL_DIR))
 
 
-def rbf_forward(X, Y, gamma):
-    """K = exp(-gamma * ||X_i - Y_j||^2) on the GPU (fp32)."""
+@functools.lru_cache(maxsize=256)
+def _workspace_bytes(N, M, D):
+    return _lib().rbf_backward_workspace_bytes(N, M, D)
+
+
+def _check_forward(X, Y):
     capi.require(X.is_cuda and Y.is_cuda, "X, Y must be GPU tensors")
     capi.require(X.dtype == torch.float32 and Y.dtype == torch.float32, "X, Y must be float32")
     capi.require(X.dim() == 2 and Y.dim() == 2, "X, Y must be 2D")
     capi.require(X.size(1) == Y.size(1), "X, Y must share feature dim D")
+
+
+def rbf_forward(X, Y, gamma):
+    """K = exp(-gamma * ||X_i - Y_j||^2) on the GPU (fp32)."""
+    _check_forward(X, Y)
     lib = _lib()
     X = X.contiguous()
     Y = Y.contiguous()
     N, D = X.shape
     M = Y.size(0)
-    K = torch.empty((N, M), dtype=torch.float32, device=X.device)
-    with torch.cuda.device(X.device):
-        st = lib.rbf_forward_f32(capi.ptr(X), capi.ptr(Y), capi.ptr(K), N, M, D,
-                                 float(gamma), capi.stream_of(X))
-    capi.check(st, lib.rbf_last_error, "rbf_forward")
+    K = X.new_empty((N, M))
+    st = capi.launch(lib.rbf_forward_f32, X.get_device(), X.data_ptr(), Y.data_ptr(),
+                     K.data_ptr(), N, M, D, float(gamma))
+    if st:
+        capi.check(st, lib.rbf_last_error, "rbf_forward")
     return K
+
+
+def _check_backward(X, Y, G, K):
+    f32 = torch.float32
+    capi.require(X.is_cuda and Y.is_cuda and G.is_cuda and K.is_cuda, "inputs must be GPU tensors")
+    capi.require(X.dtype == f32 and Y.dtype == f32 and G.dtype == f32 and K.dtype == f32,
+                 "inputs must be float32")
+    capi.require(X.dim() == 2 and Y.dim() == 2 and X.size(1) == Y.size(1),
+                 "X, Y must be 2D with a shared feature dim D")
+    shape = G.shape
+    capi.require(shape == (X.size(0), Y.size(0)) and K.shape == shape,
+                 "G and K must have shape [N, M]")
 
 
 def rbf_backward(X, Y, G, K, gamma):
     """(dX, dY) from upstream G = dL/dK and the saved forward output K."""
-    capi.require(X.is_cuda and Y.is_cuda and G.is_cuda and K.is_cuda, "inputs must be GPU tensors")
-    capi.require(all(t.dtype == torch.float32 for t in (X, Y, G, K)), "inputs must be float32")
-    capi.require(X.dim() == 2 and Y.dim() == 2 and X.size(1) == Y.size(1),
-                 "X, Y must be 2D with a shared feature dim D")
-    capi.require(tuple(G.shape) == (X.size(0), Y.size(0)) and tuple(K.shape) == tuple(G.shape),
-                 "G and K must have shape [N, M]")
+    _check_backward(X, Y, G, K)
     lib = _lib()
     X, Y, G, K = X.contiguous(), Y.contiguous(), G.contiguous(), K.contiguous()
     N, D = X.shape
     M = Y.size(0)
     dX = torch.empty_like(X)
     dY = torch.empty_like(Y)
-    ws_bytes = lib.rbf_backward_workspace_bytes(N, M, D)
-    ws = torch.empty((max(ws_bytes, 4) + 3) // 4, dtype=torch.float32, device=X.device)
-    with torch.cuda.device(X.device):
-        st = lib.rbf_backward_f32(capi.ptr(X), capi.ptr(Y), capi.ptr(G), capi.ptr(K),
-                                  capi.ptr(dX), capi.ptr(dY), N, M, D, float(gamma),
-                                  capi.ptr(ws), ws_bytes, capi.stream_of(X))
-    capi.check(st, lib.rbf_last_error, "rbf_backward")
+    ws_bytes = _workspace_bytes(N, M, D)
+    ws = X.new_empty((max(ws_bytes, 4) + 3) // 4)
+    st = capi.launch(lib.rbf_backward_f32, X.get_device(), X.data_ptr(), Y.data_ptr(),
+                     G.data_ptr(), K.data_ptr(), dX.data_ptr(), dY.data_ptr(), N, M, D,
+                     float(gamma), ws.data_ptr(), ws_bytes)
+    if st:
+        capi.check(st, lib.rbf_last_error, "rbf_backward")
     return dX, dY
 
 

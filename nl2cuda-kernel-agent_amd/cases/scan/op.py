@@ -44,7 +44,14 @@ def _lib():
     return bind_library(load_kernel(LIB_NAME, SOURCES, base_dir=KERNEL_DIR))
 
 
+@functools.lru_cache(maxsize=256)
+def _workspace_bytes(rows, d):
+    return _lib().scan_workspace_bytes(rows, d)
+
+
 def _check(x, what, dtypes):
+    if x.is_cuda and x.dtype in dtypes and x.dim() == 2 and x.size(0) > 0 and x.size(1) > 0:
+        return
     capi.require(x.is_cuda, f"{what} expects a GPU tensor")
     capi.require(x.dtype in dtypes, f"{what} only supports " + " / ".join(str(d) for d in dtypes))
     capi.require(x.dim() == 2, f"{what} expects a 2D tensor")
@@ -65,7 +72,7 @@ def _workspace(device, stream, nbytes):
     (shared capture) stream."""
     if torch.cuda.is_current_stream_capturing():
         return torch.empty(max((nbytes + 7) // 8, 1), dtype=torch.int64, device=device)
-    key = (device.index, stream.value)
+    key = (device.index, stream)
     ws = _WORKSPACES.get(key)
     if ws is None or ws.numel() * 8 < nbytes:
         ws = torch.empty(max((nbytes + 7) // 8, 1), dtype=torch.int64, device=device)
@@ -77,19 +84,21 @@ def _call(fn_name, x, out_dtype, what):
     lib = _lib()
     x = x.contiguous()
     rows, d = x.shape
-    y = torch.empty((rows, d), dtype=out_dtype, device=x.device)
-    ws_bytes = lib.scan_workspace_bytes(rows, d)
-    ws = _workspace(x.device, capi.stream_of(x), ws_bytes)
-    status = None
-    if capi.checking() and not torch.cuda.is_current_stream_capturing():
-        off = lib.scan_status_offset(rows, d)
-        if off != SIZE_MAX:
-            status = ws[off // 8:off // 8 + 1]
-            status.zero_()
-    with torch.cuda.device(x.device):
-        st = getattr(lib, fn_name)(capi.ptr(x), capi.ptr(y), rows, d, capi.ptr(ws),
-                                   ws.numel() * 8, capi.stream_of(x))
-    capi.check(st, lib.scan_last_error, what)
+    y = torch.empty_like(x) if out_dtype == x.dtype else x.new_empty((rows, d), dtype=out_dtype)
+    ws_bytes = _workspace_bytes(rows, d)
+    ws_ptr, status = 0, None
+    if ws_bytes:  # rows of one chunk need none
+        ws = _workspace(x.device, capi.stream_of(x).value, ws_bytes)
+        ws_ptr, ws_bytes = ws.data_ptr(), ws.numel() * 8
+        if capi.checking() and not torch.cuda.is_current_stream_capturing():
+            off = lib.scan_status_offset(rows, d)
+            if off != SIZE_MAX:
+                status = ws[off // 8:off // 8 + 1]
+                status.zero_()
+    st = capi.launch(getattr(lib, fn_name), x.get_device(), x.data_ptr(), y.data_ptr(), rows, d,
+                     ws_ptr, ws_bytes)
+    if st:
+        capi.check(st, lib.scan_last_error, what)
     if status is not None:
         trips = int(status.item()) & 0xFFFFFFFF
         capi.require(trips == 0, f"{what}: {trips} chunk(s) hit the carry-wait spin cap "

@@ -40,6 +40,11 @@ def _lib():
     return bind_library(load_kernel(LIB_NAME, SOURCES, base_dir=KERNEL_DIR))
 
 
+@functools.lru_cache(maxsize=256)
+def _workspace_bytes(B, C):
+    return _lib().softmax_ce_forward_workspace_bytes(B, C)
+
+
 def _check(logits, labels):
     capi.require(logits.is_cuda and labels.is_cuda, "logits, labels must be GPU tensors")
     capi.require(logits.dtype == torch.float32, "logits must be float32")
@@ -54,20 +59,20 @@ def sce_forward(logits, labels):
     lib = _lib()
     logits, labels = logits.contiguous(), labels.contiguous()
     B, C = logits.shape
-    loss = torch.empty((), dtype=torch.float32, device=logits.device)
-    lse = torch.empty(B, dtype=torch.float32, device=logits.device)
-    ws_bytes = lib.softmax_ce_forward_workspace_bytes(B, C)
-    ws = torch.empty((ws_bytes + 7) // 8, dtype=torch.int64, device=logits.device)
+    loss = logits.new_empty(())
+    lse = logits.new_empty(B)
+    ws_bytes = _workspace_bytes(B, C)
+    ws = labels.new_empty((ws_bytes + 7) // 8)
     status = None
     if capi.checking() and not torch.cuda.is_current_stream_capturing():
         off = lib.softmax_ce_status_offset() // 8
         status = ws[off:off + 1]
         status.zero_()
-    with torch.cuda.device(logits.device):
-        st = lib.softmax_ce_forward_f32(capi.ptr(logits), capi.ptr(labels), capi.ptr(loss),
-                                        capi.ptr(lse), B, C, capi.ptr(ws), ws_bytes,
-                                        capi.stream_of(logits))
-    capi.check(st, lib.softmax_ce_last_error, "sce_forward")
+    st = capi.launch(lib.softmax_ce_forward_f32, logits.get_device(), logits.data_ptr(),
+                     labels.data_ptr(), loss.data_ptr(), lse.data_ptr(), B, C, ws.data_ptr(),
+                     ws_bytes)
+    if st:
+        capi.check(st, lib.softmax_ce_last_error, "sce_forward")
     if status is not None:
         trips = int(status.item()) & 0xFFFFFFFF
         capi.require(trips == 0, "sce_forward: the partial-loss wait hit its spin cap")
@@ -84,11 +89,10 @@ def sce_backward(logits, labels, lse, gout):
     g = gout.reshape(1).contiguous()
     B, C = logits.shape
     dlogits = torch.empty_like(logits)
-    with torch.cuda.device(logits.device):
-        st = lib.softmax_ce_backward_f32(capi.ptr(logits), capi.ptr(labels), capi.ptr(lse),
-                                         capi.ptr(g), capi.ptr(dlogits), B, C,
-                                         capi.stream_of(logits))
-    capi.check(st, lib.softmax_ce_last_error, "sce_backward")
+    st = capi.launch(lib.softmax_ce_backward_f32, logits.get_device(), logits.data_ptr(),
+                     labels.data_ptr(), lse.data_ptr(), g.data_ptr(), dlogits.data_ptr(), B, C)
+    if st:
+        capi.check(st, lib.softmax_ce_last_error, "sce_backward")
     return dlogits
 
 

@@ -66,7 +66,22 @@ def _suffix(row_ptr, col_idx):
     return "i32" if row_ptr.dtype == torch.int32 else "i64"
 
 
+@functools.lru_cache(maxsize=256)
+def _workspace_bytes(M, K, D, nnz):
+    return _lib().spmv_backward_best_workspace_bytes(M, K, D, nnz)
+
+
+@functools.lru_cache(maxsize=None)
+def _entry(name):
+    return getattr(_lib(), name)
+
+
 def _validate(row_ptr, col_idx, vals, X):
+    if (row_ptr.is_cuda and col_idx.is_cuda and vals.is_cuda and X.is_cuda and
+            vals.dtype == torch.float32 and X.dtype == torch.float32 and X.dim() == 2 and
+            X.size(0) > 0 and X.size(1) > 0 and row_ptr.dim() == 1 and row_ptr.numel() >= 1 and
+            col_idx.dim() == 1 and vals.dim() == 1 and col_idx.numel() == vals.numel()):
+        return _suffix(row_ptr, col_idx)
     for name, t in (("row_ptr", row_ptr), ("col_idx", col_idx), ("vals", vals), ("X", X)):
         capi.require(t.is_cuda, f"{name} must be a GPU tensor")
     capi.require(vals.dtype == torch.float32, "vals must be float32")
@@ -116,25 +131,24 @@ def spmv_forward(row_ptr, col_idx, vals, X, keep_gather=False):
     X[col_idx] as the kernel read it, for spmv_backward(..., X_gathered=Xg)."""
     t = _validate(row_ptr, col_idx, vals, X)
     lib = _lib()
-    row_ptr, col_idx, vals, X = (a.contiguous() for a in (row_ptr, col_idx, vals, X))
+    row_ptr, col_idx = row_ptr.contiguous(), col_idx.contiguous()
+    vals, X = vals.contiguous(), X.contiguous()
     M = row_ptr.numel() - 1
     K, D = X.shape
     if capi.checking() and not torch.cuda.is_current_stream_capturing():
         check_structure(row_ptr, col_idx, K)
-    Y = torch.empty((M, D), dtype=torch.float32, device=X.device)
+    Y = X.new_empty((M, D))
+    head = (row_ptr.data_ptr(), col_idx.data_ptr(), vals.data_ptr(), X.data_ptr(), Y.data_ptr())
     if keep_gather:
         capi.require(D == 1, "keep_gather needs D == 1")
         Xg = torch.empty_like(vals)
-    with torch.cuda.device(X.device):
-        if keep_gather:
-            st = getattr(lib, f"spmv_forward_gather_f32_{t}")(
-                capi.ptr(row_ptr), capi.ptr(col_idx), capi.ptr(vals), capi.ptr(X), capi.ptr(Y),
-                capi.ptr(Xg), M, K, D, vals.numel(), capi.stream_of(X))
-        else:
-            st = getattr(lib, f"spmv_forward_f32_{t}")(
-                capi.ptr(row_ptr), capi.ptr(col_idx), capi.ptr(vals), capi.ptr(X), capi.ptr(Y),
-                M, K, D, vals.numel(), capi.stream_of(X))
-    capi.check(st, lib.spmv_last_error, "spmv_forward")
+        st = capi.launch(_entry(f"spmv_forward_gather_f32_{t}"), X.get_device(), *head,
+                         Xg.data_ptr(), M, K, D, vals.numel())
+    else:
+        st = capi.launch(_entry(f"spmv_forward_f32_{t}"), X.get_device(), *head, M, K, D,
+                         vals.numel())
+    if st:
+        capi.check(st, lib.spmv_last_error, "spmv_forward")
     return (Y, Xg) if keep_gather else Y
 
 
@@ -154,33 +168,32 @@ def spmv_backward(row_ptr, col_idx, vals, X, grad_Y, need_vals=True, need_X=True
     capi.require(grad_Y.dim() == 2 and grad_Y.size(0) == M and grad_Y.size(1) == X.size(1),
                  "grad_Y must have shape [M, D]")
     lib = _lib()
-    row_ptr, col_idx, vals, X, grad_Y = (a.contiguous() for a in (row_ptr, col_idx, vals, X, grad_Y))
+    row_ptr, col_idx = row_ptr.contiguous(), col_idx.contiguous()
+    vals, X, grad_Y = vals.contiguous(), X.contiguous(), grad_Y.contiguous()
     K, D = X.shape
     if capi.checking() and not torch.cuda.is_current_stream_capturing():
         check_structure(row_ptr, col_idx, K)
     grad_vals = torch.empty_like(vals) if need_vals else None
     grad_X = torch.empty_like(X) if need_X else None
-    ws_bytes = lib.spmv_backward_best_workspace_bytes(M, K, D, vals.numel()) if need_X else 0
+    nnz = vals.numel()
+    ws_bytes = _workspace_bytes(M, K, D, nnz) if need_X else 0
     ws = torch.empty(max(ws_bytes, 8), dtype=torch.uint8, device=X.device)  # scratch
     status = None
     if need_X and capi.checking() and not torch.cuda.is_current_stream_capturing():
-        off = lib.spmv_status_offset(M, K, D, vals.numel())
+        off = lib.spmv_status_offset(M, K, D, nnz)
         if off != SIZE_MAX:
             status = ws[off:off + 8].view(torch.int64)
             status.zero_()
-    outs = (capi.ptr(grad_vals) if need_vals else None, capi.ptr(grad_X) if need_X else None)
-    with torch.cuda.device(X.device):
-        if X_gathered is not None:
-            st = getattr(lib, f"spmv_backward_gathered_f32_{t}")(
-                capi.ptr(row_ptr), capi.ptr(col_idx), capi.ptr(vals), capi.ptr(X),
-                capi.ptr(X_gathered), capi.ptr(grad_Y), *outs, M, K, D, vals.numel(),
-                capi.ptr(ws), ws_bytes, capi.stream_of(X))
-        else:
-            st = getattr(lib, f"spmv_backward_f32_{t}")(
-                capi.ptr(row_ptr), capi.ptr(col_idx), capi.ptr(vals), capi.ptr(X),
-                capi.ptr(grad_Y), *outs, M, K, D, vals.numel(), capi.ptr(ws), ws_bytes,
-                capi.stream_of(X))
-    capi.check(st, lib.spmv_last_error, "spmv_backward")
+    tail = (grad_Y.data_ptr(), grad_vals.data_ptr() if need_vals else None,
+            grad_X.data_ptr() if need_X else None, M, K, D, nnz, ws.data_ptr(), ws_bytes)
+    head = (row_ptr.data_ptr(), col_idx.data_ptr(), vals.data_ptr(), X.data_ptr())
+    if X_gathered is not None:
+        st = capi.launch(_entry(f"spmv_backward_gathered_f32_{t}"), X.get_device(), *head,
+                         X_gathered.data_ptr(), *tail)
+    else:
+        st = capi.launch(_entry(f"spmv_backward_f32_{t}"), X.get_device(), *head, *tail)
+    if st:
+        capi.check(st, lib.spmv_last_error, "spmv_backward")
     if status is not None:
         trips = int(status.item()) & 0xFFFFFFFF
         capi.require(trips == 0, "spmv_backward: a column-total wait hit its spin cap")
