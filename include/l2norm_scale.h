@@ -33,13 +33,15 @@ extern "C" {
 #endif
 
 /* Y [N, D] and norm [N] (l2norm_scale.cu:140-150, `l2n_forward`).  The
- * row-cached path runs for D % 4 == 0, D <= 16384 and 16-byte aligned X, g,
- * Y; other shapes use generic kernels.  eps >= 0 (NL2K_ERR_VALUE). */
+ * row-cached path runs for D <= 16384, longer rows use generic kernels.
+ * eps >= 0 (NL2K_ERR_VALUE). */
 int l2norm_scale_forward_f32(const float* X, const float* g, float* Y, float* norm, int64_t N,
                              int64_t D, float eps, hipStream_t stream);
 
-/* Workspace bytes l2norm_scale_backward_f32 needs (scratch, 16-byte
- * aligned). */
+/* Workspace bytes for l2norm_scale_backward_f32 (scratch, 16-byte aligned).
+ * Rows that are no whole float4, or start off a 16-byte boundary, run in less
+ * too, on slower kernels (down to 2048 / (D / 64) partial rows of D floats,
+ * at most 512). */
 size_t l2norm_scale_backward_workspace_bytes(int64_t N, int64_t D);
 
 /* dX [N, D] and dg [D] from dY, given X, g and the forward's norm

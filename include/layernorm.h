@@ -40,8 +40,10 @@ int layernorm_forward_f32(const float* x, const float* w, const float* bias,
                           float* y, float* mean, float* rstd, int64_t B,
                           int64_t D, float eps, hipStream_t stream);
 
-/* Workspace bytes layernorm_backward_f32 needs for these sizes (per-block
- * partial sums of dw and dbias). */
+/* Workspace bytes for layernorm_backward_f32 at these sizes (per-block
+ * partial sums of dw and dbias; 16-byte aligned).  Rows that are no whole
+ * float4, or start off a 16-byte boundary, run in less too, on slower kernels
+ * (down to 2048 / (D / 64) partial rows of 2 D floats, at most 512). */
 size_t layernorm_backward_workspace_bytes(int64_t B, int64_t D);
 
 /*

@@ -76,15 +76,18 @@ int l2norm_scale_backward_f32(const float* dY, const float* X, const float* g, c
     return nl2k::rownorm::fill_zero(dg, nullptr, D, stream, who);
   const bool aligned = nl2k::aligned16(dY) && nl2k::aligned16(X) && nl2k::aligned16(g) &&
                        nl2k::aligned16(dX);
-  const size_t need = nl2k::rownorm::workspace_floats<L2NormRows>(
-                          D, nl2k::rownorm::plan(N, D, aligned)) * sizeof(float);
+  size_t need = 0;
+  const nl2k::rownorm::Plan plan = nl2k::rownorm::plan_backward<L2NormRows>(
+      N, D, aligned, workspace ? workspace_bytes / sizeof(float) : 0, &need);
+  need *= sizeof(float);
   if (!workspace || workspace_bytes < need)
     return nl2k::fail(NL2K_ERR_WORKSPACE, "%s: workspace of %zu bytes required, got %zu", who,
                       need, workspace ? workspace_bytes : (size_t)0);
   if (!nl2k::aligned16(workspace))
     return nl2k::fail(NL2K_ERR_ALIGN, "%s: workspace must be 16-byte aligned", who);
   return nl2k::rownorm::run_backward<L2NormRows>(dY, X, g, nullptr, norm, dX, dg, nullptr, N, D,
-                                                 static_cast<float*>(workspace), stream, who);
+                                                 plan, static_cast<float*>(workspace),
+                                                 stream, who);
 }
 
 }  // extern "C"

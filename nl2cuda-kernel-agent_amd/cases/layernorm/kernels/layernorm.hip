@@ -9,8 +9,8 @@
 //
 // Design: the row-normalisation kernels of csrc/rownorm.h (row-cached
 // two-pass statistics in registers, prefetching backward with per-block
-// dw / dbias partials summed deterministically, generic kernels for other
-// shapes) with the centered, biased policy below.
+// dw / dbias partials summed deterministically, generic kernels for rows past
+// 16384 floats) with the centered, biased policy below.
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
@@ -77,8 +77,10 @@ int layernorm_backward_f32(const float* dy, const float* x, const float* w,
     return nl2k::rownorm::fill_zero(dw, dbias, D, stream, "layernorm_backward_f32 (zero)");
   const bool aligned = nl2k::aligned16(dy) && nl2k::aligned16(x) && nl2k::aligned16(w) &&
                        nl2k::aligned16(dx);
-  const size_t need = nl2k::rownorm::workspace_floats<LayerNormRows>(
-                          D, nl2k::rownorm::plan(B, D, aligned)) * sizeof(float);
+  size_t need = 0;
+  const nl2k::rownorm::Plan plan = nl2k::rownorm::plan_backward<LayerNormRows>(
+      B, D, aligned, workspace ? workspace_bytes / sizeof(float) : 0, &need);
+  need *= sizeof(float);
   if (!workspace || workspace_bytes < need)
     return nl2k::fail(NL2K_ERR_WORKSPACE,
                       "layernorm_backward_f32: workspace of %zu bytes required, got %zu", need,
@@ -86,7 +88,8 @@ int layernorm_backward_f32(const float* dy, const float* x, const float* w,
   if (!nl2k::aligned16(workspace))
     return nl2k::fail(NL2K_ERR_ALIGN, "layernorm_backward_f32: workspace must be 16-byte aligned");
   return nl2k::rownorm::run_backward<LayerNormRows>(dy, x, w, mean, rstd, dx, dw, dbias, B, D,
-                                                    static_cast<float*>(workspace), stream, who);
+                                                    plan, static_cast<float*>(workspace),
+                                                    stream, who);
 }
 
 }  // extern "C"

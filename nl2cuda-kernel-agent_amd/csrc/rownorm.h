@@ -16,7 +16,7 @@
 //   dw = sum over rows of dy xh,  dbias = sum of dy.
 //
 // Design (HBM bound: read x, write y; read dy and x, write dx):
-//  * Row-cached path (D % 4 == 0, 16-byte aligned, D <= 16384): TPR threads
+//  * Row-cached path (D <= 16384, any alignment): TPR threads
 //    own a row at a time (16 lanes for rows of at most 128 floats, a wave,
 //    or a workgroup of 256 or 512 threads for long rows; the backward uses
 //    1024 above 8192 floats) and walk every
@@ -35,9 +35,19 @@
 //    fixed order) and writes one partial row.  The per-block partials
 //    ([G][D]) are summed by rn_colsum_kernel in one stream-ordered pass,
 //    every sum in a fixed order, so dw and dbias are deterministic.
-//  * Any other shape uses generic kernels that re-read x: one workgroup per
-//    row for y / dx, and rn_bwd_generic_partial_kernel (64 columns x a group
-//    of rows per block) for the partial rows, then the same column sums.
+//  * Rows that are no whole number of float4, or start off a 16-byte
+//    boundary, take the same kernels: 16-byte accesses need only 4-byte
+//    alignment here, and a buffer resource over the row cuts the last one
+//    off at the row's end.  Against the generic kernels (forward and
+//    backward with column sums, us): LayerNorm [8192, 4097] 129 against 276
+//    ([8192, 4096]: 128), [1000, 16383] 85 against 187, [20000, 101] 19
+//    against 52; L2 norm [5001, 1001] 24 against 41, [30000, 33] 13
+//    against 46.
+//  * Rows longer than 16384 floats, and a backward with a workspace too
+//    small for the partial rows of the row-cached plan, use generic kernels
+//    that re-read x: one workgroup per row for y / dx, and
+//    rn_bwd_generic_partial_kernel (64 columns x a group of rows per block)
+//    for the partial rows, then the same column sums.
 #pragma once
 
 #include <algorithm>
@@ -64,6 +74,12 @@ __device__ __forceinline__ float dot4(f32x4 a, f32x4 b) {
   return (a[0] * b[0] + a[1] * b[1]) + (a[2] * b[2] + a[3] * b[3]);
 }
 __device__ __forceinline__ float hsum4(f32x4 a) { return (a[0] + a[1]) + (a[2] + a[3]); }
+// Columns c .. c + 3 of a row of D, zero past its end.
+__device__ __forceinline__ f32x4 within(f32x4 a, int c, int D) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) a[e] = c + e < D ? a[e] : 0.f;
+  return a;
+}
 
 // Sum over the TPR threads that share a row (TPR = 64, 256, 512 or 1024),
 // result in all of them.  `red` is LDS scratch of at least 2 * TPR / 64
@@ -101,8 +117,9 @@ __device__ __forceinline__ float row_sum1(float a, float* red) {
 }
 
 // ------------------------------------------------------------------ forward
-// FULL: D/4 == V * TPR, so every thread's V float4 are in range and the
-// loads need no guard (guards become branches that defeat load batching).
+// FULL: D/4 == V * TPR and every operand on 16 bytes, so every thread's V
+// float4 are in range and the loads need no guard (guards become branches
+// that defeat load batching).
 // stat0 (the mean) is written only when P::kCentered, bias read only when
 // P::kBias.  Row group g (TPR threads; RPB = kBlock / TPR per block) walks
 // rows g, g + S, g + 2S, ... (S = the grid's row groups), with the next
@@ -125,7 +142,6 @@ __global__ __launch_bounds__(TPR > kBlock ? TPR : kBlock) void rn_fwd_kernel(
   const int64_t r0 =
       (int64_t)blockIdx.x * RPB + __builtin_amdgcn_readfirstlane((int)threadIdx.x) / TPR;
   const int t = threadIdx.x % TPR;
-  const int D4 = D >> 2;
   // TPR >= 256: the grid has at most B blocks, so a whole block walks the
   // same rows and takes the reductions' barriers together.  TPR = 64: a row
   // group past the end leaves (its reductions stay inside its wave).
@@ -133,11 +149,15 @@ __global__ __launch_bounds__(TPR > kBlock ? TPR : kBlock) void rn_fwd_kernel(
   const int64_t rlast = r0 + (B - 1 - r0) / S * S;
   const f32x4* w4 = reinterpret_cast<const f32x4*>(w);
   const f32x4* b4 = reinterpret_cast<const f32x4*>(bias);
+  const buffer_rsrc rw = make_rsrc(w, (uint32_t)D * 4u);
+  const buffer_rsrc rb = make_rsrc(bias, P::kBias ? (uint32_t)D * 4u : 0u);
   f32x4 wv[V], bv[V], cur[V], nxt[V];
-  // Ragged rows (not FULL) load and store through a buffer resource over
-  // the row: lanes past its end read zeros and write nothing, with no
-  // branch, so the count of memory operations in flight stays the same on
-  // every path and the loop waits only for the loads it uses.
+  // Ragged rows (not FULL: any D, any 4-byte alignment) load and store
+  // through a buffer resource over the row.  The range check is per float,
+  // also inside a 16-byte access: floats past the row's end read zeros and
+  // write nothing, with no branch, so the count of memory operations in
+  // flight stays the same on every path and the loop waits only for the
+  // loads it uses.
   auto load_row = [&](int64_t r, f32x4 (&v)[V]) {
     const f32x4* xr = reinterpret_cast<const f32x4*>(x + r * D);
     const buffer_rsrc rx = make_rsrc(x + r * D, (uint32_t)D * 4u);
@@ -150,9 +170,9 @@ __global__ __launch_bounds__(TPR > kBlock ? TPR : kBlock) void rn_fwd_kernel(
   load_row(r0, cur);
 #pragma unroll
   for (int k = 0; k < V; ++k) {
-    const int c = FULL ? t + k * TPR : min(t + k * TPR, D4 - 1);
-    wv[k] = w4[c];
-    if constexpr (P::kBias) bv[k] = b4[c];
+    const int c = t + k * TPR;
+    wv[k] = FULL ? w4[c] : buffer_load4(rw, (uint32_t)c * 16u, 0);
+    if constexpr (P::kBias) bv[k] = FULL ? b4[c] : buffer_load4(rb, (uint32_t)c * 16u, 0);
   }
   const float inv_d = 1.f / (float)D;
   for (int64_t r = r0; r < B; r += S) {
@@ -170,10 +190,9 @@ __global__ __launch_bounds__(TPR > kBlock ? TPR : kBlock) void rn_fwd_kernel(
 #pragma unroll
     for (int k = 0; k < V; ++k) {
       const int c = t + k * TPR;
-      if (FULL || c < D4) {
-        const f32x4 dv = cur[k] - mu;
-        q += dot4(dv, dv);
-      }
+      f32x4 dv = cur[k] - mu;
+      if constexpr (!FULL && P::kCentered) dv = within(dv, 4 * c, D);
+      q += dot4(dv, dv);
     }
     const float ss = row_sum1<TPR>(q, red) * (P::kCentered ? inv_d : 1.f) + eps;
     const float rs = 1.f / sqrtf(ss);
@@ -198,7 +217,7 @@ __global__ __launch_bounds__(TPR > kBlock ? TPR : kBlock) void rn_fwd_kernel(
   }
 }
 
-// Generic forward: one workgroup per row, any D and alignment.
+// Generic forward: one workgroup per row, any D.
 template <class P>
 __global__ __launch_bounds__(kBlock) void rn_fwd_generic_kernel(
     const float* __restrict__ x, const float* __restrict__ w,
@@ -274,7 +293,6 @@ __global__ __launch_bounds__(TPR * H) void rn_bwd_kernel(
   // pointers and the row predicate stay scalar.
   const int hf = H > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x) / TPR : 0;
   const int t = threadIdx.x % TPR;
-  const int D4 = D >> 2;
   const int64_t G = gridDim.x;  // G <= B: every block's half 0 has a row
   const int64_t S = (int64_t)H * G;
   const int64_t r0 = (int64_t)blockIdx.x + hf * G;
@@ -283,6 +301,7 @@ __global__ __launch_bounds__(TPR * H) void rn_bwd_kernel(
   // prefetch is clamped to, so the last step re-reads a row it already has.
   const int64_t rlast = r0 < B ? r0 + (B - 1 - r0) / S * S : B - 1;
   const f32x4* w4 = reinterpret_cast<const f32x4*>(w);
+  const buffer_rsrc rw = make_rsrc(w, (uint32_t)D * 4u);
 
   // TPR = 1024 (a block of 16 waves, at most 128 registers a lane) keeps w
   // in LDS, each thread its own entries, so that the prefetch fits.
@@ -292,11 +311,11 @@ __global__ __launch_bounds__(TPR * H) void rn_bwd_kernel(
 #pragma unroll
   for (int k = 0; k < V; ++k) {
     const int c = t + k * TPR;
-    const f32x4 wk = w4[FULL ? c : min(c, D4 - 1)];
+    const f32x4 wk = FULL ? w4[c] : buffer_load4(rw, (uint32_t)c * 16u, 0);
     if constexpr (kWLds)
-      s_w[c] = (FULL || c < D4) ? wk : zero4();
+      s_w[c] = wk;
     else
-      wv[k] = (FULL || c < D4) ? wk : zero4();
+      wv[k] = wk;
     aw[k] = zero4();
     ab[k] = zero4();
   }
@@ -333,8 +352,15 @@ __global__ __launch_bounds__(TPR * H) void rn_bwd_kernel(
     for (int k2 = 0; k2 < V; ++k2) {
       xh[k2] = (xcur[k2] - mu) * rs;
       const f32x4 g = gcur[k2] * w_at(k2);
-      if constexpr (P::kCentered) sg += hsum4(g);
-      sgx += dot4(g, xh[k2]);
+      if constexpr (P::kCentered) {
+        sg += hsum4(g);
+        sgx += dot4(g, xh[k2]);
+      } else {
+        // past the row's end g is 0 and xh is 0 rs: not a number where the
+        // norm of a row that is not zero underflowed
+        const int c = t + k2 * TPR;
+        sgx += dot4(g, FULL ? xh[k2] : within(xh[k2], 4 * c, D));
+      }
     }
     if (has) {
 #pragma unroll
@@ -391,15 +417,14 @@ __global__ __launch_bounds__(TPR * H) void rn_bwd_kernel(
       }
     }
   }
-  f32x4* pw4 = reinterpret_cast<f32x4*>(pw + (int64_t)blockIdx.x * D);
-  f32x4* pb4 = reinterpret_cast<f32x4*>(pb + (int64_t)blockIdx.x * D);
+  const buffer_rsrc rpw = make_rsrc(pw + (int64_t)blockIdx.x * D, (uint32_t)D * 4u);
+  const buffer_rsrc rpb =
+      make_rsrc(P::kBias ? pb + (int64_t)blockIdx.x * D : nullptr, P::kBias ? (uint32_t)D * 4u : 0u);
 #pragma unroll
   for (int k = 0; k < V; ++k) {
-    const int c = t + k * TPR;
-    if (FULL || c < D4) {
-      pw4[c] = aw[k];
-      if constexpr (P::kBias) pb4[c] = ab[k];
-    }
+    const uint32_t off = (uint32_t)(t + k * TPR) * 16u;
+    buffer_store4(rpw, aw[k], off, 0);
+    if constexpr (P::kBias) buffer_store4(rpb, ab[k], off, 0);
   }
 }
 
@@ -415,9 +440,31 @@ __device__ __forceinline__ float row16_sum(float v) { return row16_sum_dpp(v); }
 // stores write nothing, and no memory operation sits under a branch or
 // depends on a per-step select (the compiler turns such a select into a
 // branch).  With a wave per row, 48 of 64 lanes idled at D = 64.
+//
+// RAGGED (D % 4 != 0, D >= 4): the row's last float4 reaches back to end at
+// the row's end, since the bytes past it are the next row's.  Its first
+// floats then repeat those of the float4 before: they count once in the
+// sums and are stored twice with one value.
 constexpr uint32_t kOutside = 0x7FFFFFF0u;  // past any resource used here; no 32-bit wrap
 
-template <class P, int V>
+// Float4 c of a row: the column it starts at, and its floats that the sums
+// count (`own`, a bit each).
+template <bool RAGGED>
+__device__ __forceinline__ int row16_start(int c, int D, uint32_t& own) {
+  const int D4 = (D + 3) >> 2;
+  const int cc = min(c, D4 - 1);
+  const int start = RAGGED ? min(4 * cc, D - 4) : 4 * cc;
+  own = c < D4 ? (0xFu << (4 * cc - start)) & 0xFu : 0u;
+  return start;
+}
+template <bool RAGGED>
+__device__ __forceinline__ f32x4 row16_own(f32x4 a, uint32_t own) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) a[e] = (own >> (RAGGED ? e : 0)) & 1u ? a[e] : 0.f;
+  return a;
+}
+
+template <class P, int V, bool RAGGED>
 __global__ __launch_bounds__(kBlock) void rn_fwd_row16_kernel(
     const float* __restrict__ x, const float* __restrict__ w,
     const float* __restrict__ bias, float* __restrict__ y,
@@ -428,23 +475,24 @@ __global__ __launch_bounds__(kBlock) void rn_fwd_row16_kernel(
   const int j = lane >> 4;  // the lane's row among the wave's four
   const int t = lane & 15;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x) >> 6;
-  const int D4 = D >> 2;
+  const int D4 = (D + 3) >> 2;
   const int64_t S = (int64_t)gridDim.x * RPB;
   const int64_t rw0 = (int64_t)blockIdx.x * RPB + 4 * wave;  // the wave's first row
   if (rw0 >= B) return;  // wave uniform; no barriers below
   const int64_t rwl = rw0 + (B - 1 - rw0) / S * S;       // its last row set
   const uint32_t rbytes = (uint32_t)D * 4u;
   auto rows = [&](int64_t rw) { return (uint32_t)min(B - rw, (int64_t)4); };
-  const f32x4* w4 = reinterpret_cast<const f32x4*>(w);
-  const f32x4* b4 = reinterpret_cast<const f32x4*>(bias);
-  uint32_t off[V];
+  const buffer_rsrc rwt = make_rsrc(w, rbytes);
+  const buffer_rsrc rbs = make_rsrc(bias, P::kBias ? rbytes : 0u);
+  uint32_t off[V], own[V];
   f32x4 wv[V], bv[V];
 #pragma unroll
   for (int k = 0; k < V; ++k) {
     const int c = t + 16 * k;
-    off[k] = c < D4 ? (uint32_t)j * rbytes + (uint32_t)c * 16u : kOutside;
-    wv[k] = w4[min(c, D4 - 1)];
-    if constexpr (P::kBias) bv[k] = b4[min(c, D4 - 1)];
+    const uint32_t start = 4u * (uint32_t)row16_start<RAGGED>(c, D, own[k]);
+    off[k] = c < D4 ? (uint32_t)j * rbytes + start : kOutside;
+    wv[k] = buffer_load4(rwt, start, 0);
+    if constexpr (P::kBias) bv[k] = buffer_load4(rbs, start, 0);
   }
   const uint32_t soff = t == 0 ? (uint32_t)j * 4u : kOutside;
   auto load = [&](int64_t rw, f32x4 (&v)[V]) {
@@ -463,14 +511,15 @@ __global__ __launch_bounds__(kBlock) void rn_fwd_row16_kernel(
     if constexpr (P::kCentered) {
       float sx = 0.f;
 #pragma unroll
-      for (int k = 0; k < V; ++k) sx += hsum4(cur[k]);  // zeros past the row
+      for (int k = 0; k < V; ++k)  // zeros past the row
+        sx += hsum4(RAGGED ? row16_own<RAGGED>(cur[k], own[k]) : cur[k]);
       mu = row16_sum(sx) * inv_d;
     }
     float q = 0.f;
 #pragma unroll
     for (int k = 0; k < V; ++k) {
-      const f32x4 dv = cur[k] - mu;
-      q += t + 16 * k < D4 ? dot4(dv, dv) : 0.f;
+      const f32x4 dv = row16_own<RAGGED>(cur[k] - mu, own[k]);
+      q += dot4(dv, dv);
     }
     const float ss = row16_sum(q) * (P::kCentered ? inv_d : 1.f) + eps;
     const float rs = 1.f / sqrtf(ss);
@@ -494,7 +543,7 @@ __global__ __launch_bounds__(kBlock) void rn_fwd_row16_kernel(
 // (/ dbias) in registers per lane.  At the end the four row groups of a
 // wave are added by two lane exchanges (16 apart, then 32 apart) and the
 // four waves in LDS (0 + 1 + 2 + 3), and the block writes one partial row.
-template <class P, int V>
+template <class P, int V, bool RAGGED>
 __global__ __launch_bounds__(kBlock) void rn_bwd_row16_kernel(
     const float* __restrict__ dy, const float* __restrict__ x,
     const float* __restrict__ w, const float* __restrict__ stat0,
@@ -508,20 +557,20 @@ __global__ __launch_bounds__(kBlock) void rn_bwd_row16_kernel(
   const int j = lane >> 4;
   const int t = lane & 15;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x) >> 6;
-  const int D4 = D >> 2;
+  const int D4 = (D + 3) >> 2;
   const int64_t S = (int64_t)gridDim.x * RPB;
   const int64_t rw0 = (int64_t)blockIdx.x * RPB + 4 * wave;
   const uint32_t rbytes = (uint32_t)D * 4u;
   auto rows = [&](int64_t rw) { return (uint32_t)min(B - rw, (int64_t)4); };
-  const f32x4* w4 = reinterpret_cast<const f32x4*>(w);
-  uint32_t off[V];
+  const buffer_rsrc rwt = make_rsrc(w, rbytes);
+  uint32_t off[V], own[V];
   f32x4 wv[V], aw[V], ab[V];
 #pragma unroll
   for (int k = 0; k < V; ++k) {
     const int c = t + 16 * k;
-    off[k] = c < D4 ? (uint32_t)j * rbytes + (uint32_t)c * 16u : kOutside;
-    const f32x4 wk = w4[min(c, D4 - 1)];
-    wv[k] = c < D4 ? wk : zero4();
+    const uint32_t start = 4u * (uint32_t)row16_start<RAGGED>(c, D, own[k]);
+    off[k] = c < D4 ? (uint32_t)j * rbytes + start : kOutside;
+    wv[k] = buffer_load4(rwt, c < D4 ? start : kOutside, 0);
     aw[k] = zero4();
     ab[k] = zero4();
   }
@@ -559,8 +608,14 @@ __global__ __launch_bounds__(kBlock) void rn_bwd_row16_kernel(
       for (int k = 0; k < V; ++k) {
         xh[k] = (cur.xv[k] - mu) * rs;
         const f32x4 g = cur.g[k] * wv[k];
-        if constexpr (P::kCentered) sg += hsum4(g);
-        sgx += dot4(g, xh[k]);
+        if constexpr (RAGGED) {
+          const f32x4 gx = row16_own<RAGGED>(g * xh[k], own[k]);
+          if constexpr (P::kCentered) sg += hsum4(row16_own<RAGGED>(g, own[k]));
+          sgx += hsum4(gx);
+        } else {
+          if constexpr (P::kCentered) sg += hsum4(g);
+          sgx += dot4(g, xh[k]);
+        }
       }
       const float mg = P::kCentered ? row16_sum(sg) * inv_d : 0.f;
       const float mgx = row16_sum(sgx) * (P::kCentered ? inv_d : 1.f);
@@ -608,19 +663,18 @@ __global__ __launch_bounds__(kBlock) void rn_bwd_row16_kernel(
       if constexpr (P::kBias) ab[k] += sp[16 * V + t + 16 * k];
     }
   }
-  f32x4* pw4 = reinterpret_cast<f32x4*>(pw + (int64_t)blockIdx.x * D);
-  f32x4* pb4 = reinterpret_cast<f32x4*>(pb + (int64_t)blockIdx.x * D);
+  // here j = 0, so off is the column's offset in a row
+  const buffer_rsrc rpw = make_rsrc(pw + (int64_t)blockIdx.x * D, rbytes);
+  const buffer_rsrc rpb =
+      make_rsrc(P::kBias ? pb + (int64_t)blockIdx.x * D : nullptr, P::kBias ? rbytes : 0u);
 #pragma unroll
   for (int k = 0; k < V; ++k) {
-    const int c = t + 16 * k;
-    if (c < D4) {
-      pw4[c] = aw[k];
-      if constexpr (P::kBias) pb4[c] = ab[k];
-    }
+    buffer_store4(rpw, aw[k], off[k], 0);
+    if constexpr (P::kBias) buffer_store4(rpb, ab[k], off[k], 0);
   }
 }
 
-// Generic backward (any D / alignment): one workgroup per row writes dx;
+// Generic backward (any D): one workgroup per row writes dx;
 // rn_bwd_generic_partial_kernel then forms the partial parameter rows.
 template <class P>
 __global__ __launch_bounds__(kBlock) void rn_bwd_generic_kernel(
@@ -708,11 +762,9 @@ __global__ __launch_bounds__(64 * kColsumWaves) void rn_colsum_kernel(
       if constexpr (TWO) vb[k] = in_b[(r + k * kColsumWaves) * D + cc];
     }
     __builtin_amdgcn_sched_barrier(0);  // the batch's loads issue before the adds
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      aw += vw[k];
-      if constexpr (TWO) ab += vb[k];
-    }
+    aw += ((vw[0] + vw[1]) + (vw[2] + vw[3])) + ((vw[4] + vw[5]) + (vw[6] + vw[7]));
+    if constexpr (TWO)
+      ab += ((vb[0] + vb[1]) + (vb[2] + vb[3])) + ((vb[4] + vb[5]) + (vb[6] + vb[7]));
   }
   for (; r < R; r += kColsumWaves) {
     aw += in_w[r * D + cc];
@@ -724,9 +776,10 @@ __global__ __launch_bounds__(64 * kColsumWaves) void rn_colsum_kernel(
   if (wave == 0 && c < D) {
     float tw = 0.f, tb = 0.f;
 #pragma unroll
-    for (int w = 0; w < kColsumWaves; ++w) {
-      tw += sw[w][lane];
-      if constexpr (TWO) tb += sb[w][lane];
+    for (int w = 0; w < kColsumWaves; w += 4) {
+      tw += (sw[w][lane] + sw[w + 1][lane]) + (sw[w + 2][lane] + sw[w + 3][lane]);
+      if constexpr (TWO)
+        tb += (sb[w][lane] + sb[w + 1][lane]) + (sb[w + 2][lane] + sb[w + 3][lane]);
     }
     out_w[c] = tw;
     if constexpr (TWO) out_b[c] = tb;
@@ -746,6 +799,7 @@ __global__ __launch_bounds__(kBlock) void rn_fill_zero_kernel(float* __restrict_
 // ----------------------------------------------------------------- planning
 struct Plan {
   bool cached = false;  // row-cached vector path
+  bool whole = false;   // rows of whole float4, every operand 16-byte aligned
   int tpr = 256;        // forward threads per row
   int v = 4;            // float4 per thread
   int btpr = 256;       // backward (cached): threads per row
@@ -760,21 +814,26 @@ inline int64_t row_groups(int64_t B, int64_t target) {
   return ceil_div(B, std::max<int64_t>(1, ceil_div(B, target)));
 }
 
-inline Plan plan(int64_t B, int64_t D, bool aligned) {
+inline Plan plan_generic(int64_t B, int64_t D) {
   Plan p;
-  p.cached = aligned && D % 4 == 0 && D <= 16384;
-  if (!p.cached) {
-    // ~2048 blocks of 64 columns x (B / S1) rows
-    const int64_t slices = ceil_div(D, 64);
-    const int64_t s1 = std::min<int64_t>(
-        std::min<int64_t>(std::max<int64_t>(1, ceil_div(2048, slices)), kGenericMaxSplit),
-        std::max<int64_t>(B, 1));
-    p.rpb = std::max<int64_t>(1, ceil_div(B, s1));
-    p.G = B > 0 ? ceil_div(B, p.rpb) : 0;
-    return p;
-  }
-  const int64_t d4 = D / 4;
-  if (d4 <= 32) {  // 16 lanes per row, both directions
+  // ~2048 blocks of 64 columns x (B / S1) rows
+  const int64_t slices = ceil_div(D, 64);
+  const int64_t s1 = std::min<int64_t>(
+      std::min<int64_t>(std::max<int64_t>(1, ceil_div(2048, slices)), kGenericMaxSplit),
+      std::max<int64_t>(B, 1));
+  p.rpb = std::max<int64_t>(1, ceil_div(B, s1));
+  p.G = B > 0 ? ceil_div(B, p.rpb) : 0;
+  return p;
+}
+
+// `aligned`: every operand on 16 bytes.
+inline Plan plan(int64_t B, int64_t D, bool aligned) {
+  if (D > 16384) return plan_generic(B, D);
+  Plan p;
+  p.cached = true;
+  p.whole = aligned && D % 4 == 0;
+  const int64_t d4 = ceil_div(D, 4);
+  if (d4 <= 32 && D >= 4) {  // 16 lanes per row, both directions (D < 4: a wave)
     p.tpr = p.btpr = 16;
     p.v = p.bv = d4 <= 16 ? 1 : 2;
     p.bh = 16;
@@ -826,10 +885,23 @@ size_t workspace_floats(int64_t D, const Plan& p) {
 
 template <class P>
 size_t backward_workspace_bytes(int64_t B, int64_t D) {
-  // Pointer alignment picks the path at call time: cover both.
   const size_t cached = workspace_floats<P>(D, plan(B, D, true));
-  const size_t generic = workspace_floats<P>(D, plan(B, D, false));
+  const size_t generic = workspace_floats<P>(D, plan_generic(B, D));
   return std::max(cached, generic) * sizeof(float);
+}
+
+// The backward's plan in a workspace of `floats`; G = 0 where it is too
+// small, and *need is what the call asks for.  Whole aligned rows need the
+// row-cached plan's partial rows; the others need only the generic plan's
+// (at D = 16383 8 against 256) and take the row-cached plan where the
+// workspace holds it, as backward_workspace_bytes does.
+template <class P>
+Plan plan_backward(int64_t B, int64_t D, bool aligned, size_t floats, size_t* need) {
+  const Plan p = plan(B, D, aligned), g = plan_generic(B, D);
+  const size_t np = workspace_floats<P>(D, p), ng = workspace_floats<P>(D, g);
+  *need = p.whole ? np : ng;
+  if (floats < *need) return Plan{};
+  return floats >= np ? p : g;
 }
 
 // ----------------------------------------------------------------- launches
@@ -844,17 +916,19 @@ int run_forward(const float* x, const float* w, const float* bias, float* y, flo
   if (p.cached && p.tpr == 16) {
     const dim3 grid((unsigned)std::min<int64_t>(
         ceil_div(B, 16), p.v == 1 ? kRow16FwdBlocks1 : kRow16FwdBlocks2));
-    if (p.v == 1)
-      hipLaunchKernelGGL((rn_fwd_row16_kernel<P, 1>), grid, dim3(kBlock), 0, stream, x, w, bias,
-                         y, stat0, stat1, B, (int)D, eps);
-    else
-      hipLaunchKernelGGL((rn_fwd_row16_kernel<P, 2>), grid, dim3(kBlock), 0, stream, x, w, bias,
-                         y, stat0, stat1, B, (int)D, eps);
+#define RN_FWD16(V, RAGGED)                                                                  \
+  hipLaunchKernelGGL((rn_fwd_row16_kernel<P, V, RAGGED>), grid, dim3(kBlock), 0, stream, x, w, \
+                     bias, y, stat0, stat1, B, (int)D, eps)
+    if (p.v == 1 && D % 4 == 0) RN_FWD16(1, false);
+    else if (p.v == 1) RN_FWD16(1, true);
+    else if (D % 4 == 0) RN_FWD16(2, false);
+    else RN_FWD16(2, true);
+#undef RN_FWD16
     return check_launch(who);
   }
   if (p.cached && p.tpr == 512) {  // one 512-thread row group per block
     const dim3 grid((unsigned)std::min<int64_t>(B, kFwdBlocks));
-    if (D == 512 * 4 * 8)
+    if (p.whole && D == 512 * 4 * 8)
       hipLaunchKernelGGL((rn_fwd_kernel<P, 512, 8, true>), grid, dim3(512), 0, stream, x, w, bias,
                          y, stat0, stat1, B, (int)D, eps);
     else
@@ -867,7 +941,7 @@ int run_forward(const float* x, const float* w, const float* bias, float* y, flo
     const dim3 grid((unsigned)std::min<int64_t>(ceil_div(B, rpb), kFwdBlocks));
 #define RN_FWD(TPR, V)                                                                      \
   do {                                                                                       \
-    if (D / 4 == (TPR) * (V))                                                                \
+    if (p.whole && D / 4 == (TPR) * (V))                                                     \
       hipLaunchKernelGGL((rn_fwd_kernel<P, TPR, V, true>), grid, dim3(kBlock), 0, stream, x,  \
                          w, bias, y, stat0, stat1, B, (int)D, eps);                          \
     else                                                                                     \
@@ -897,21 +971,19 @@ inline int fill_zero(float* a, float* b, int64_t D, hipStream_t stream, const ch
   return check_launch(who);
 }
 
-// Backward launches for B >= 1 (the caller validated sizes, pointers and the
-// workspace size / alignment against backward_workspace_bytes).
+// Backward launches for B >= 1 with a plan of plan_backward (the caller
+// validated sizes, pointers and the workspace).
 template <class P>
 int run_backward(const float* dy, const float* x, const float* w, const float* stat0,
                  const float* stat1, float* dx, float* dw, float* dbias, int64_t B,
-                 int64_t D, float* ws, hipStream_t stream, const char* who) {
-  const bool aligned = aligned16(dy) && aligned16(x) && aligned16(w) && aligned16(dx);
-  const Plan p = plan(B, D, aligned);
+                 int64_t D, const Plan& p, float* ws, hipStream_t stream, const char* who) {
   float* pw = ws;
   float* pb = pw + p.G * D;
   int st;
   if (p.cached) {
 #define RN_BWD(TPR, V, H)                                                                     \
   do {                                                                                        \
-    if (D / 4 == (TPR) * (V))                                                                 \
+    if (p.whole && D / 4 == (TPR) * (V))                                                      \
       hipLaunchKernelGGL((rn_bwd_kernel<P, TPR, V, true, H>), dim3((unsigned)p.G),            \
                          dim3((TPR) * (H)), 0, stream, dy, x, w, stat0, stat1, dx, pw, pb, B, \
                          (int)D);                                                             \
@@ -920,12 +992,13 @@ int run_backward(const float* dy, const float* x, const float* w, const float* s
                          dim3((TPR) * (H)), 0, stream, dy, x, w, stat0, stat1, dx, pw, pb, B, \
                          (int)D);                                                             \
   } while (0)
-    if (p.btpr == 16 && p.bv == 1)
-      hipLaunchKernelGGL((rn_bwd_row16_kernel<P, 1>), dim3((unsigned)p.G), dim3(kBlock), 0,
-                         stream, dy, x, w, stat0, stat1, dx, pw, pb, B, (int)D);
-    else if (p.btpr == 16)
-      hipLaunchKernelGGL((rn_bwd_row16_kernel<P, 2>), dim3((unsigned)p.G), dim3(kBlock), 0,
-                         stream, dy, x, w, stat0, stat1, dx, pw, pb, B, (int)D);
+#define RN_BWD16(V, RAGGED)                                                                   \
+  hipLaunchKernelGGL((rn_bwd_row16_kernel<P, V, RAGGED>), dim3((unsigned)p.G), dim3(kBlock), 0, \
+                     stream, dy, x, w, stat0, stat1, dx, pw, pb, B, (int)D)
+    if (p.btpr == 16 && p.bv == 1 && D % 4 == 0) RN_BWD16(1, false);
+    else if (p.btpr == 16 && p.bv == 1) RN_BWD16(1, true);
+    else if (p.btpr == 16 && D % 4 == 0) RN_BWD16(2, false);
+    else if (p.btpr == 16) RN_BWD16(2, true);
     else if (p.btpr == 64 && p.bv == 1) RN_BWD(64, 1, 4);
     else if (p.btpr == 64 && p.bv == 2) RN_BWD(64, 2, 4);
     else if (p.btpr == 64 && p.bv == 3) RN_BWD(64, 3, 4);
@@ -935,6 +1008,7 @@ int run_backward(const float* dy, const float* x, const float* w, const float* s
     else if (p.btpr == 512) RN_BWD(512, 4, 1);
     else RN_BWD(1024, 4, 1);
 #undef RN_BWD
+#undef RN_BWD16
     st = check_launch(who);
   } else {
     hipLaunchKernelGGL(rn_bwd_generic_kernel<P>, dim3((unsigned)B), dim3(kBlock), 0, stream, dy,
