@@ -17,8 +17,10 @@
 //    range, then a short one per wave inside it.  A wave then walks
 //    its nonzeros in steps of 256: lane l loads positions 4l..4l+3 with one
 //    16-byte load of col_idx and one of vals, gathers x, and finds each
-//    position's row by binary search over the next 512 row starts staged in
-//    a wave-private LDS slice.  Per step: a serial sum over each lane's four
+//    position's row from the next 512 row starts staged in a wave-private
+//    LDS slice (the forward: those of the step mark their positions, and a
+//    running maximum does the rest; the backward: a binary search).  Per
+//    step: a serial sum over each lane's four
 //    products by row, a wave64 segmented inclusive scan (key = row) of the
 //    lanes' trailing partial sums, and every row that ends inside the step
 //    is written once; the row still open at the end of the step is carried
@@ -135,9 +137,11 @@ __device__ int64_t rows_lower_bound(const I* __restrict__ ptr, int64_t M, int64_
 // nnz_full = nnz rounded down to a multiple of 4; a wave takes it only when
 // all its positions lie below nnz_full, so no entry it uses is clamped.  The
 // scalar form reads each entry at its position clamped to [0, nnz - 1].
-// The vector loads are nontemporal: the structure is read once, and lines
-// that do not stay in the L2 leave more of it to the gathered x (forward
-// 131.0 -> 127.7 us at the acceptance shape).
+// The vector loads of 32-bit indices are nontemporal: the structure is read
+// once, and lines that do not stay in the L2 leave more of it to the gathered
+// x (2^20 rows, 16 M nonzeros: forward 125.9 -> 122.7 us).  With 64-bit
+// indices they gain nothing there (135.5 against 136.1 us) and cost the
+// backward that reads the structure next (128.4 us without, 136.5 with).
 template <typename I, bool VEC>
 struct Quad {
   I c[4];
@@ -174,9 +178,9 @@ struct Quad<int64_t, true> {
   __device__ void issue(const int64_t* __restrict__ col, const float* __restrict__ vals,
                         int64_t q0, int64_t nnz) {
     const int64_t q = max((int64_t)0, min(q0, (nnz & ~(int64_t)3) - 4));
-    c0 = __builtin_nontemporal_load(reinterpret_cast<const i64x2_t*>(col + q));
-    c1 = __builtin_nontemporal_load(reinterpret_cast<const i64x2_t*>(col + q + 2));
-    v = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(vals + q));
+    c0 = *reinterpret_cast<const i64x2_t*>(col + q);
+    c1 = *reinterpret_cast<const i64x2_t*>(col + q + 2);
+    v = *reinterpret_cast<const f32x4*>(vals + q);
   }
   __device__ int64_t col_at(int j) const { return j < 2 ? c0[j] : c1[j - 2]; }
   __device__ float val_at(int j) const { return v[j]; }
@@ -334,21 +338,108 @@ __device__ __forceinline__ void window_rows(const int64_t* bnd, const Walk& s, i
 // every row is summed in the same order however the rows are split between
 // waves: results do not depend on the wave count, which follows the
 // device's CU count and each instantiation's occupancy.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_or(int old, int v) {  // old where there is no source lane
+  return __builtin_amdgcn_update_dpp(old, v, CTRL, ROWS, 0xF, false);
+}
+constexpr int kRowShr = 0x110, kWaveShl1 = 0x130, kWaveShr1 = 0x138, kBcast15 = 0x142, kBcast31 = 0x143;
+
+// Maximum over lanes 0 .. lane of values >= 0.
+__device__ __forceinline__ int wave_scan_max(int v) {
+  v = max(v, dpp_or<kRowShr + 1, 0xF>(0, v));
+  v = max(v, dpp_or<kRowShr + 2, 0xF>(0, v));
+  v = max(v, dpp_or<kRowShr + 4, 0xF>(0, v));
+  v = max(v, dpp_or<kRowShr + 8, 0xF>(0, v));
+  v = max(v, dpp_or<kBcast15, 0xA>(0, v));
+  return max(v, dpp_or<kBcast31, 0xC>(0, v));
+}
+
+// One level of the segmented sum below: adds the other lane's sum where its
+// key is the lane's own.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float seg_level(float t, int key) {
+  const float u = __builtin_bit_cast(float, dpp_or<CTRL, ROWS>(0, __builtin_bit_cast(int, t)));
+  return dpp_or<CTRL, ROWS>(-1, key) == key ? t + u : t;
+}
+// Sum over the lanes 0 .. lane of equal key (keys >= 0, ascending).
+__device__ __forceinline__ float wave_seg_scan(float t, int key) {
+  t = seg_level<kRowShr + 1, 0xF>(t, key);
+  t = seg_level<kRowShr + 2, 0xF>(t, key);
+  t = seg_level<kRowShr + 4, 0xF>(t, key);
+  t = seg_level<kRowShr + 8, 0xF>(t, key);
+  t = seg_level<kBcast15, 0xA>(t, key);
+  return seg_level<kBcast31, 0xC>(t, key);
+}
+
+// Column clamped into [0, K), in 32 bits where the index is.
+__device__ __forceinline__ uint32_t clamp_col(int32_t c, int64_t K) {
+  return (uint32_t)min(max(c, 0), (int32_t)min(K - 1, (int64_t)INT32_MAX));
+}
+__device__ __forceinline__ int64_t clamp_col(int64_t c, int64_t K) {
+  return min(max(c, (int64_t)0), K - 1);
+}
+
+// The LDS of one wave of the forward: starts of rows wr + 1 + k relative to
+// the step they were staged at (clamped to kFar), and a mark per position of
+// the step.
+constexpr int kFar = 1 << 30;
+struct alignas(16) FwdLds {
+  int mark[kStep];
+  int win[kWin];
+};
+
+// stage_window in 32 bits, relative to position `from`.
+template <typename I>
+__device__ __forceinline__ void stage_window32(const I* __restrict__ ptr, int64_t nnz, Walk& s,
+                                               int lane, int64_t from, FwdLds& l) {
+  int64_t v[kWin / 64];
+#pragma unroll
+  for (int i = 0; i < kWin / 64; ++i)  // all loads first, then the LDS writes
+    v[i] = (int64_t)ptr[min(s.carry_row + 1 + lane + 64 * i, s.r1)];
+  __builtin_amdgcn_wave_barrier();
+  int64_t last = 0;
+#pragma unroll
+  for (int i = 0; i < kWin / 64; ++i) {
+    const int64_t r = s.carry_row + 1 + lane + 64 * i;
+    last = r < s.r1 ? min(max(v[i], (int64_t)0), nnz) : s.b;
+    l.win[lane + 64 * i] = (int)min(max(last - from, (int64_t)-1), (int64_t)kFar);
+  }
+  __builtin_amdgcn_wave_barrier();
+  s.wr = s.carry_row;
+  s.wlimit = readlane64(last, 63);
+}
+
+// Rows inside a step are counted from wr and positions from the step's base,
+// in 32 bits.  A position's row is the last one that starts at or before it:
+// every row start of the step marks its position with its row (the last of
+// several there by the maximum), and a maximum over the positions before
+// gives the rest.  Marks, maximum and the sums by row are a few LDS accesses
+// and lane moves: against 64-bit rows, a binary search of the window for each
+// lane and exchanges through LDS 126.6 -> 122.7 us at 2^20 rows and 16 M
+// nonzeros, where the gathers bind (a loop that does nothing else takes 90 to
+// 102), and 18.7 -> 14.5 us at 100000 rows and 0.8 M nonzeros.  Gathering a
+// step ahead on top of it changed nothing (122.3 us): the waves of a CU
+// already keep its requests going.
 template <typename I, bool VEC, bool SAVE>
 __device__ __forceinline__ void fwd_walk(const I* __restrict__ ptr, const I* __restrict__ col,
                                          const float* __restrict__ vals,
                                          const float* __restrict__ x, float* __restrict__ y,
                                          float* __restrict__ xg, int64_t K, int64_t nnz, Walk& s,
-                                         int lane, int64_t* bnd) {
+                                         int lane, FwdLds& l) {
   float carry_val = 0.f;
-  stage_window(ptr, nnz, s, lane, bnd);
+  int64_t wfrom = s.pos & ~(int64_t)(kStep - 1);
+  stage_window32(ptr, nnz, s, lane, wfrom, l);
   Quad<I, VEC> cur;
-  if (s.pos < s.b) cur.issue(col, vals, (s.pos & ~(int64_t)(kStep - 1)) + kPer * lane, nnz);
+  if (s.pos < s.b) cur.issue(col, vals, wfrom + kPer * lane, nnz);
+  const int q0 = kPer * lane;
 
   while (s.pos < s.b) {
     const int64_t base = s.pos & ~(int64_t)(kStep - 1);
     const int64_t want = min(base + kStep, s.b);
-    if (s.wlimit < want && s.wr != s.carry_row) stage_window(ptr, nnz, s, lane, bnd);
+    if ((s.wlimit < want && s.wr != s.carry_row) || base - wfrom >= kFar / 2) {
+      wfrom = base;
+      stage_window32(ptr, nnz, s, lane, wfrom, l);
+    }
     if (s.wlimit <= s.pos) {
       // Rows carry_row .. carry_row + kWin - 1 all end at or before pos.
       if (lane == 0) y[s.carry_row] = carry_val;
@@ -358,48 +449,62 @@ __device__ __forceinline__ void fwd_walk(const I* __restrict__ ptr, const I* __r
       continue;  // restaged next iteration (wr != carry_row)
     }
     const int64_t step_end = min(want, s.wlimit);
-    const int64_t q0 = base + kPer * lane;
-    int64_t c[4];
-    float v[4];
+    const int lo = (int)(s.pos - base), hi = (int)(step_end - base);
     bool in[4];
-    quad_get(cur, K, q0, s.pos, step_end, c, v, in);
     float xv[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) xv[j] = x[c[j]];
+    for (int j = 0; j < 4; ++j) {
+      in[j] = q0 + j >= lo && q0 + j < hi;
+      xv[j] = x[in[j] ? clamp_col((I)cur.col_at(j), K) : 0];
+    }
     Quad<I, VEC> nxt;  // the next step starts at step_end
-    nxt.issue(col, vals, (step_end & ~(int64_t)(kStep - 1)) + kPer * lane, nnz);
+    nxt.issue(col, vals, (step_end & ~(int64_t)(kStep - 1)) + q0, nnz);
     if constexpr (SAVE) {
       // Streaming stores: the copy is read once, by the backward, and must
       // not displace x from L2.
       if (VEC && in[0] && in[3]) {
         __builtin_nontemporal_store(f32x4{xv[0], xv[1], xv[2], xv[3]},
-                                    reinterpret_cast<f32x4*>(xg + q0));
+                                    reinterpret_cast<f32x4*>(xg + base + q0));
       } else {
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          if (in[j]) __builtin_nontemporal_store(xv[j], xg + q0 + j);
+          if (in[j]) __builtin_nontemporal_store(xv[j], xg + base + q0 + j);
       }
     }
-    int64_t rid[4];
-    window_rows(bnd, s, q0, step_end - 1, rid);
+    const int crel = (int)(s.carry_row - s.wr);
+    const int sh = (int)(base - wfrom);
+    *reinterpret_cast<i32x4_t*>(l.mark + q0) = i32x4_t{0, 0, 0, 0};
+    __builtin_amdgcn_wave_barrier();
+    for (int k = crel + lane;; k += 64) {
+      const int at = k < kWin ? l.win[k] - sh : kFar;
+      if (at < hi) atomicMax(&l.mark[max(at, lo)], k + 1);
+      if (__ballot(at < hi) >> 63 == 0) break;  // row starts ascend with the lanes
+    }
+    __builtin_amdgcn_wave_barrier();
+    const i32x4_t m = *reinterpret_cast<const i32x4_t*>(l.mark + q0);
+    int rid[4] = {m[0], max(m[0], m[1]), 0, 0};
+    rid[2] = max(rid[1], m[2]);
+    rid[3] = max(rid[2], m[3]);
+    const int before = max(crel, dpp_or<kWaveShr1, 0xF>(0, wave_scan_max(rid[3])));
     // Positions at or past step_end (a step cut short by the window or by
     // the wave's end) take a row id past the last real row: the rows in
     // between are empty, and the last real row ends where it ends, as when
     // another row follows it.  (Giving them the last real row instead would
     // read that row's sum from lane 63, in another order of additions.)
-    const int64_t after = min(s.r1, s.wr + kWin);
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (q0 + j >= step_end) rid[j] = after;
+    const int after = (int)min(s.r1 - s.wr, (int64_t)kWin);
     float pr[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) pr[j] = in[j] ? v[j] * xv[j] : 0.f;
+    for (int j = 0; j < 4; ++j) {
+      rid[j] = q0 + j >= hi ? after : max(before, rid[j]);
+      pr[j] = in[j] ? cur.val_at(j) * xv[j] : 0.f;
+    }
 
     // Lane-local segments: first (kf, sf), last (kl, sl); middle rows are
     // complete and written here, as are empty rows in the gaps.
-    int64_t cur_row = rid[0];
+    float* yw = y + s.wr;
+    int cur_row = rid[0];
     float acc = pr[0];
-    int64_t kf = cur_row;
+    const int kf = cur_row;
     float sf = 0.f;
     bool single = true;
 #pragma unroll
@@ -411,45 +516,38 @@ __device__ __forceinline__ void fwd_walk(const I* __restrict__ ptr, const I* __r
           sf = acc;
           single = false;
         } else {
-          y[cur_row] = acc;
+          yw[cur_row] = acc;
         }
-        for (int64_t r = cur_row + 1; r < rid[j]; ++r) y[r] = 0.f;
+        for (int r = cur_row + 1; r < rid[j]; ++r) yw[r] = 0.f;
         cur_row = rid[j];
         acc = pr[j];
       }
     }
-    const int64_t kl = cur_row;
+    const int kl = cur_row;
     const float sl = acc;
     if (single) sf = acc;
 
-    // Segmented inclusive scan of sl over lanes, key kl (keys are sorted).
-    float T = sl;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const float tu = __shfl_up(T, d, 64);
-      const int64_t ku = __shfl_up(kl, d, 64);
-      if (lane >= d && ku == kl) T += tu;
-    }
-    const int64_t prev_k = __shfl_up(kl, 1, 64);
-    const float prev_T = __shfl_up(T, 1, 64);
-    const int64_t next_kf = __shfl_down(kf, 1, 64);
-    const int64_t carry_row = s.carry_row;
+    const float T = wave_seg_scan(sl, kl);
+    const int prev_k = dpp_or<kWaveShr1, 0xF>(crel, kl);
+    const float prev_T = __builtin_bit_cast(
+        float, dpp_or<kWaveShr1, 0xF>(0, __builtin_bit_cast(int, T)));
+    const int next_kf = dpp_or<kWaveShl1, 0xF>(kl, kf);
 
     if (kf != kl) {  // the lane's first row ends inside the lane
       float tot = sf;
       if (lane > 0 && prev_k == kf) tot += prev_T;
-      if (kf == carry_row) tot += carry_val;
-      y[kf] = tot;
+      if (kf == crel) tot += carry_val;
+      yw[kf] = tot;
     }
-    const int64_t gap_lo = lane > 0 ? prev_k : carry_row;
-    for (int64_t r = gap_lo + 1; r < kf; ++r) y[r] = 0.f;
-    if (lane < 63 && next_kf != kl) y[kl] = kl == carry_row ? T + carry_val : T;
-    if (lane == 0 && kf != carry_row) y[carry_row] = carry_val;
+    for (int r = prev_k + 1; r < kf; ++r) yw[r] = 0.f;
+    if (next_kf != kl) yw[kl] = kl == crel ? T + carry_val : T;  // never lane 63
+    if (lane == 0 && kf != crel) yw[crel] = carry_val;
 
-    const int64_t new_row = __shfl(kl, 63, 64);
-    const float new_T = __shfl(T, 63, 64);
-    carry_val = new_row == carry_row ? new_T + carry_val : new_T;
-    s.carry_row = new_row;
+    const int new_rel = __builtin_amdgcn_readlane(kl, 63);
+    const float new_T =
+        __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, T), 63));
+    carry_val = new_rel == crel ? new_T + carry_val : new_T;
+    s.carry_row = s.wr + new_rel;
     s.pos = step_end;
     cur = nxt;
   }
@@ -463,7 +561,7 @@ __global__ __launch_bounds__(kThreads) void spmv_d1_fwd_kernel(
     const I* __restrict__ ptr, const I* __restrict__ col, const float* __restrict__ vals,
     const float* __restrict__ x, float* __restrict__ y, float* __restrict__ xg, int64_t M,
     int64_t K, int64_t nnz, int64_t n_waves) {
-  __shared__ int64_t bnd_s[kThreads / 64][kWin];
+  __shared__ FwdLds lds[kThreads / 64];
   __shared__ int64_t starts[kThreads / 64 + 1];
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -471,11 +569,11 @@ __global__ __launch_bounds__(kThreads) void spmv_d1_fwd_kernel(
   if (!walk_begin(ptr, M, nnz, n_waves, lane, wave, starts, s)) return;  // wave-uniform
   if constexpr (VEC) {
     if (s.b <= (nnz & ~(int64_t)3)) {
-      fwd_walk<I, true, SAVE>(ptr, col, vals, x, y, xg, K, nnz, s, lane, bnd_s[wave]);
+      fwd_walk<I, true, SAVE>(ptr, col, vals, x, y, xg, K, nnz, s, lane, lds[wave]);
       return;
     }
   }
-  fwd_walk<I, false, SAVE>(ptr, col, vals, x, y, xg, K, nnz, s, lane, bnd_s[wave]);
+  fwd_walk<I, false, SAVE>(ptr, col, vals, x, y, xg, K, nnz, s, lane, lds[wave]);
 }
 
 // ----------------------------------------------------------- D == 1 backward
