@@ -3,7 +3,8 @@ of its steps of 256 positions and of its window of 512 row starts, more row
 starts in a step than lanes, runs of empty rows around the window's length,
 rows longer than many steps.  Values and x are small integers, so every sum is
 exact in fp32 whatever its order, and y is compared bit for bit; with the copy
-of the gathered x too."""
+of the gathered x too.  The backward's column sums likewise, over tile counts
+that split differently between waves."""
 
 import numpy as np
 import pytest
@@ -57,3 +58,25 @@ def test_forward_walk(name, cut, idx):
     assert np.array_equal(y.cpu().numpy()[:, 0], want)
     assert np.array_equal(y2.cpu().numpy()[:, 0], want)
     assert np.array_equal(kept.cpu().numpy().ravel(), x[col, 0])
+
+
+@pytest.mark.parametrize("k", [1, 300, 70_000])
+@pytest.mark.parametrize("tiles", [1, 3, 15, 16, 17, 33, 65, 1030])
+def test_column_sums_over_tiles(tiles, k):
+    """dX where the waves of a bucket's workgroup share a tile of 8192 entries
+    (up to 15), take one to 64 tiles each, and take more than one group."""
+    from cases.spmv import op
+    announce(f"spmv column sums of {tiles} tiles, K={k}")
+    nnz, m = 8192 * tiles - 5, 999
+    g = np.random.default_rng(tiles)
+    ptr = np.sort(np.concatenate([[0, nnz], g.integers(0, nnz + 1, m - 1)]))
+    col = g.integers(0, k, nnz)
+    vals = g.integers(-1, 2, nnz).astype(np.float32)
+    dy = g.integers(-1, 2, (m, 1)).astype(np.float32)
+    x = g.integers(-4, 5, (k, 1)).astype(np.float32)
+    rows = np.repeat(np.arange(m), np.diff(ptr))
+    want = np.bincount(col, weights=vals.astype(np.float64) * dy[rows, 0], minlength=k)
+    dv, dx = op.spmv_backward(*(torch.from_numpy(t).cuda() for t in (ptr, col, vals, x, dy)))
+    torch.cuda.synchronize()
+    assert np.array_equal(dx.cpu().numpy()[:, 0], want)
+    assert np.array_equal(dv.cpu().numpy().ravel(), dy[rows, 0] * x[col, 0])
