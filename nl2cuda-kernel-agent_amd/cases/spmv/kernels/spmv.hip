@@ -889,11 +889,17 @@ __device__ __forceinline__ void spmm_chunk(const I* __restrict__ col,
 // a D that is no multiple of 4 owns the row's last four, some of them with
 // its neighbour (both sum and store the same bits).
 // Bound by the gather of X rows (D floats per nonzero, from L2 and MALL).
-// 100000 rows of 1 to 516 entries, 1.6 M in all, D = 32: 120 -> 59 us (eight
+// 100000 rows of 1 to 516 entries, 1.6 M in all, D = 32: 118 -> 60 us (eight
 // lanes a row instead of sixteen half idle, long rows shared).
+// Registers are held to what the rows alone need, short of spills (72503 rows
+// of 27, D = 8: 13.7 us without the bound, 12.2 with; 11.8 without the shared
+// rows, of which one row of 516 entries costs more than that).
 constexpr int kLongRow = 64;
+constexpr int fwd_waves(int G, bool vec, size_t index) {
+  return index == 8 ? 4 : vec ? (G == 1 ? 6 : G <= 4 ? 5 : 4) : 5;
+}
 template <typename I, int L, int G, bool VEC>
-__global__ __launch_bounds__(kThreads) void spmm_fwd_kernel(
+__global__ __launch_bounds__(kThreads, fwd_waves(G, VEC, sizeof(I))) void spmm_fwd_kernel(
     const I* __restrict__ ptr, const I* __restrict__ col, const float* __restrict__ vals,
     const float* __restrict__ X, float* __restrict__ Y, int64_t M, int64_t K, int64_t D,
     int64_t nnz) {
@@ -902,7 +908,7 @@ __global__ __launch_bounds__(kThreads) void spmm_fwd_kernel(
   static_assert(kRowLanes <= 64 && (kRowLanes & (kRowLanes - 1)) == 0, "rows inside a wave");
   constexpr int kRows = kThreads / kRowLanes;  // rows per workgroup
   constexpr int kWaves = kThreads / 64;
-  __shared__ int s_n, s_long[kRows];
+  __shared__ unsigned long long s_long[kWaves];  // a bit at the first lane of each long row
   __shared__ typename V::T s_sum[kWaves][L];
   const int64_t row0 = (int64_t)blockIdx.x * kRows;
   const int64_t row = row0 + threadIdx.x / kRowLanes;
@@ -912,9 +918,8 @@ __global__ __launch_bounds__(kThreads) void spmm_fwd_kernel(
   const int64_t s = live ? ld_ptr(ptr, row, nnz) : 0;
   const int64_t e = live ? max(s, ld_ptr(ptr, row + 1, nnz)) : 0;
   const bool is_long = e - s > kLongRow * G;
-  if (threadIdx.x == 0) s_n = 0;
-  __syncthreads();
-  if (is_long && gl == 0 && grp == 0) s_long[atomicAdd(&s_n, 1)] = threadIdx.x / kRowLanes;
+  const unsigned long long long_rows = __ballot(is_long && gl == 0 && grp == 0);
+  if ((threadIdx.x & 63) == 0) s_long[threadIdx.x >> 6] = long_rows;
   const int64_t own_e = is_long ? s : e;
   for (int64_t d0 = 0; d0 < D; d0 += (int64_t)L * V::W) {
     const int64_t d = d0 + (int64_t)gl * V::W;
@@ -931,11 +936,15 @@ __global__ __launch_bounds__(kThreads) void spmm_fwd_kernel(
     if (live && !is_long && active && grp == 0) V::store(Y + row * D + dc, acc);
   }
   __syncthreads();
-  const int n_long = s_n;
   constexpr int kGroups = kThreads / L;  // of the workgroup
   const int wave = threadIdx.x >> 6, wg = threadIdx.x / L;
-  for (int k = 0; k < n_long; ++k) {
-    const int64_t r = row0 + s_long[k];
+  int lw = 0;
+  unsigned long long left = s_long[0];
+  while (true) {  // the workgroup's long rows, wave after wave
+    while (left == 0 && lw < kWaves - 1) left = s_long[++lw];
+    if (left == 0) break;
+    const int64_t r = row0 + (64 * lw + __builtin_ctzll(left)) / kRowLanes;
+    left &= left - 1;
     const int64_t ls = ld_ptr(ptr, r, nnz), le = max(ls, ld_ptr(ptr, r + 1, nnz));
     for (int64_t d0 = 0; d0 < D; d0 += (int64_t)L * V::W) {
       const int64_t d = d0 + (int64_t)gl * V::W;
@@ -2551,12 +2560,17 @@ int row_lanes(int64_t units) {
 
 // Groups of L lanes that share a column in the SpMM backward's gather: 2
 // when L * 2 <= 64 and an average column has two 16-entry steps or more,
-// else 1.  At the reference default (64 entries per column, L = 16, 159
+// else 1; more, up to a whole wave a column, while the launch has fewer than
+// 2048 waves and a group keeps four steps (K = 1267 with 1545 entries a
+// column at D = 8: 131 -> 38 us with 16 groups).  At the reference default (64 entries per column, L = 16, 159
 // VGPRs: 3 waves per SIMD) the backward measured 41.9 us with G = 1, 39.5
 // with G = 2 and 41.2 with G = 4, whose 4096 waves overflow one round.
 int spmm_col_groups(int L, int64_t K, int64_t nnz) {
   const int64_t avg = K > 0 ? nnz / K : 0;
-  return (2 * L <= 64 && avg >= 32) ? 2 : 1;
+  int G = (2 * L <= 64 && avg >= 32) ? 2 : 1;
+  if (G == 2)
+    while (2 * G * L <= 64 && avg >= 64 * 2 * G && K * G * L / 64 < 2048) G *= 2;
+  return G;
 }
 
 // Groups of L lanes that split each row's nonzeros in the SpMM forward: the
@@ -2888,12 +2902,15 @@ int transpose_backward(const TransposePlan& tp, const I* ptr, const I* col, cons
 #define SPMM_T(LL, GG, VV, DVV)                                                                   \
   hipLaunchKernelGGL((spmm_t_gather_kernel<I, LL, GG, VV, DVV>), grid, block, 0, stream, colptr, \
                      crec, X, dY, dX, dvals, M, K, D, nnz)
-#define SPMM_T_G(LL, VV, DVV)         \
-  if (G == 1) SPMM_T(LL, 1, VV, DVV); \
-  else SPMM_T(LL, 2, VV, DVV)
-#define SPMM_T_L(VV, DVV)                     \
-  if (L == 4) { SPMM_T_G(4, VV, DVV); }       \
-  else if (L == 16) { SPMM_T_G(16, VV, DVV); } \
+#define SPMM_T_L(VV, DVV)                                 \
+  if (L == 4 && G == 1) SPMM_T(4, 1, VV, DVV);            \
+  else if (L == 4 && G == 2) SPMM_T(4, 2, VV, DVV);       \
+  else if (L == 4 && G == 4) SPMM_T(4, 4, VV, DVV);       \
+  else if (L == 4 && G == 8) SPMM_T(4, 8, VV, DVV);       \
+  else if (L == 4) SPMM_T(4, 16, VV, DVV);                \
+  else if (L == 16 && G == 1) SPMM_T(16, 1, VV, DVV);     \
+  else if (L == 16 && G == 2) SPMM_T(16, 2, VV, DVV);     \
+  else if (L == 16) SPMM_T(16, 4, VV, DVV);               \
   else SPMM_T(64, 1, VV, DVV)
   if (vec) {
     if (dv) { SPMM_T_L(true, true); } else { SPMM_T_L(true, false); }
@@ -2901,7 +2918,6 @@ int transpose_backward(const TransposePlan& tp, const I* ptr, const I* col, cons
     if (dv) { SPMM_T_L(false, true); } else { SPMM_T_L(false, false); }
   }
 #undef SPMM_T_L
-#undef SPMM_T_G
 #undef SPMM_T
   st = nl2k::check_launch(who);
   if (st || dvals == nullptr || dv) return st;

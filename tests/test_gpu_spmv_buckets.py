@@ -101,3 +101,11 @@ def test_spmm_bucket_route_needs_its_workspace():
     torch.cuda.synchronize()
     assert float((dx - dx0).norm() / dx0.norm()) < 1e-6
     assert float((dv - dv0).norm() / dv0.norm()) < 1e-6
+
+
+@pytest.mark.parametrize("d", [3, 7, 8, 13, 16, 33, 60, 64, 128])
+@pytest.mark.parametrize("k", [1, 5, 20, 40, 80])
+def test_spmm_few_long_columns(k, d):
+    """Few columns of many entries: 1 to 16 lane groups share a column."""
+    lens = np.random.default_rng(k).integers(0, 30, 700)
+    _check(lens, k, d, torch.int64 if d % 2 else torch.int32, seed=d)
