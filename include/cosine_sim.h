@@ -36,8 +36,8 @@ extern "C" {
 #endif
 
 /* S [N, M] and the inverse norms inv_a [N], inv_b [M] (cosine_sim.cu:104-115,
- * `cos_forward`).  The fp32 MFMA path runs for D == 64 with 16-byte aligned
- * A, B; other shapes use generic kernels.  eps >= 0 (NL2K_ERR_VALUE
+ * `cos_forward`).  MFMA on three-term bf16 splits of fp32 at any D and
+ * alignment.  eps >= 0 (NL2K_ERR_VALUE
  * otherwise).  With N == 0 or M == 0 only the inverse norms are written. */
 int cosine_sim_forward_f32(const float* A, const float* B, float* S, float* inv_a,
                            float* inv_b, int64_t N, int64_t M, int64_t D, float eps,

@@ -29,8 +29,9 @@
 //  * Backward: lse saved by the forward turns the gradient into a pure
 //    streaming pass (read logits, write dlogits, no reductions).  Aligned
 //    float4 rows of 1025 to 8192 classes are laid out like the forward, so
-//    each row's lse and label are read once; the others stream flat, four
-//    floats a lane whatever the rows.
+//    each row's lse and label are read once; ragged rows of 512 classes
+//    or more go by segments of a row; the others stream flat, four floats a
+//    lane whatever the rows.
 //  * A label outside [0, C) makes its row's loss term and gradient NaN (the
 //    reference would index out of the row; torch raises).
 //  * Unaligned rows (or C % 4 != 0) of at most 32 classes take a lane each
