@@ -35,10 +35,10 @@ extern "C" {
  * Replaces the pybind entry `rbf_forward(Tensor X, Tensor Y, double gamma)
  * -> Tensor` of the reference (cases/rbf/kernels/rbf_forward.cu:94-120),
  * which cases/rbf/op.py:30 calls.  N, M >= 0, D >= 1, any alignment.
- * Distances come from norms and products, each product from three-term bf16
- * splits of the fp32 rows; with D != 64, tiles holding a row with
- * gamma |x|^2 > 4 (or a norm that is not finite, at any D) sum the squared
- * differences directly.
+ * Distances are formed in 64 bits (gamma |x|^2 up to 2^24); at D == 64 with
+ * 16-byte aligned X and Y from norms and products in fp32, each product from
+ * three-term bf16 splits (gamma |x|^2 up to 4).  Tiles holding a larger row, or
+ * one that is not finite, sum the squared differences directly in fp32.
  */
 int rbf_forward_f32(const float* X, const float* Y, float* K, int64_t N,
                     int64_t M, int64_t D, float gamma, hipStream_t stream);

@@ -9,10 +9,11 @@
 //
 // Design:
 //  * Forward: K[i,j] = exp2(min(2 kappa x_i.y_j - kappa (|x_i|^2 + |y_j|^2), 0))
-//    with kappa = gamma log2(e), on bf16 splits of the fp32 rows
-//    (csrc/pairwise_split.h), at any D and alignment.  Tiles whose distances
-//    that form would round too coarsely (norm_max below) sum the squared
-//    differences directly, on SIMT tiles.
+//    with kappa = gamma log2(e): at D = 64 on bf16 splits of the fp32 rows
+//    (csrc/pairwise_split.h), else in 64 bits (rbf_fwd_kernel), at any D and
+//    alignment.  Tiles whose distances that form would round too coarsely
+//    (split_norm_max, f64_norm_max) sum the squared differences directly, on
+//    SIMT tiles.
 //  * Backward: one pass over dK and K per 64 features.  Workgroups own
 //    regions of W = dK o K and write raw partial contractions W . Y and
 //    W^T . X and partial row and column sums of W to workspace slots, on the
@@ -34,11 +35,13 @@
 #include "../../../csrc/pairwise_split.h"
 #include "rbf.h"
 
+using nl2k::f32x2;
+using nl2k::f32x4;
 using nl2k::pairwise::kD;
 
 namespace {
 
-constexpr float kLog2e = 1.4426950408889634f;
+constexpr double kLog2e = 1.4426950408889634;
 
 // Forward policy of the SIMT tiles: the squared differences summed directly,
 // as the reference kernel does.
@@ -53,9 +56,9 @@ struct RbfGenFwd {
   __device__ __forceinline__ float out(float s) const { return expf(-gamma * s); }
 };
 
-// Forward policy: the row term is -kappa |x|^2, the column term |y|^2, and
-// K = exp2(min(2 kappa x.y - kappa (|x|^2 + |y|^2), 0)); the clamp keeps
-// K <= 1 when the distance cancels to a tiny negative value.
+// Forward policy on the splits: the row term is -kappa |x|^2, the column term
+// |y|^2, and K = exp2(min(2 kappa x.y - kappa (|x|^2 + |y|^2), 0)); the clamp
+// keeps K <= 1 when the distance cancels to a tiny negative value.
 struct RbfFwdOp {
   float neg_kappa;  // -gamma log2(e)
   float gamma;
@@ -75,6 +78,120 @@ struct RbfFwdOp {
 struct RbfBwdOp {
   static constexpr bool kProduct = true, kScale = false, kSums = true;
 };
+
+// ------------------------------------------------------------------- forward
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2_u __attribute__((ext_vector_type(2), aligned(4)));
+
+// K = exp2(-kappa max(|x|^2 + |y|^2 - 2 x.y, 0)), the distance in 64 bits on
+// v_mfma_f64_16x16x4_f64: fp32 products are exact there, and what the
+// difference of norms and products loses is 2^-52 of the norms, so near rows
+// keep their distance, K(x, x) = 1 and K(X, X) is symmetric.
+// A workgroup of four waves takes 64 x 64 outputs, a wave 32 x 32: two blocks
+// of 16 rows (operand A, X), and two of every second column (operand B, Y), so
+// that a lane's outputs of a row lie side by side.  Lane (n, h) holds four
+// features of a row, k + 4 h .. + 3, straight from global memory (the next 16
+// features are in flight while these are multiplied), and the norms are summed
+// from the same registers.
+// Bound by the matrix instruction, which takes 120 cycles on a full chip (42
+// TFLOP/s).  Against the squared differences summed in fp32 on SIMT tiles:
+// 53 -> 39 us at 3000 x 2500 x 100, 20 -> 9.2 at 1000 x 1000 x 100, 39 -> 33
+// at 4096^2 x 32, 104 -> 82 at 4096^2 x 128.  Error of K against 64 bits
+// (2-norm) 1.4e-7 -> 3.4e-8 at D = 100.  (bf16 splits take 21 us at 3000 x 2500
+// x 100, but a pair of rows 1 % apart is off by 7e-8 at gamma |x|^2 = 0.5 and
+// 6e-7 at 4 there, against 2e-8 directly.)
+constexpr int kFwdTile = 64;
+__global__ __launch_bounds__(256, 2) void rbf_fwd_kernel(
+    const float* __restrict__ X, const float* __restrict__ Y, float* __restrict__ K, int N, int M,
+    int D, double neg_kappa, double norm_max, float gamma, int n_jt) {
+  __shared__ __attribute__((aligned(16))) nl2k::pairwise::SimtTile simt;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int n = lane & 15, h = lane >> 4;
+  const int i0 = (int)(blockIdx.x / n_jt) * kFwdTile, j0 = (int)(blockIdx.x % n_jt) * kFwdTile;
+  const int ib = i0 + (wave >> 1) * 32, j = j0 + (wave & 1) * 32 + 2 * n;
+  const float* src[4];  // rows ib + n, + 16 of X, rows j, j + 1 of Y
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    src[b] = X + (size_t)min(ib + 16 * b + n, N - 1) * D;
+    src[2 + b] = Y + (size_t)min(j + b, M - 1) * D;
+  }
+  f64x4 acc[2][2];
+  double nsq[4];
+#pragma unroll
+  for (int a = 0; a < 2; ++a) {
+    nsq[a] = nsq[2 + a] = 0.;
+#pragma unroll
+    for (int b = 0; b < 2; ++b) acc[a][b] = f64x4{0., 0., 0., 0.};
+  }
+  auto step = [&](const float (&x)[4]) {  // one feature of each row a lane
+    double v[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      v[s] = (double)x[s];
+      nsq[s] = fma(v[s], v[s], nsq[s]);
+    }
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+        acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(v[a], v[2 + b], acc[a][b], 0, 0, 0);
+  };
+  f32x4 nxt[4];
+  auto load = [&](int k) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) nxt[s] = nl2k::pairwise::load4_u(src[s] + k + 4 * h);
+  };
+  const int whole = D & ~15;
+  if (whole > 0) load(0);
+  for (int k = 0; k < whole; k += 16) {
+    f32x4 cur[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) cur[s] = nxt[s];
+    if (k + 16 < whole) load(k + 16);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) step({cur[0][u], cur[1][u], cur[2][u], cur[3][u]});
+  }
+  for (int k = whole; k < D; k += 4) {  // the last features, four at a time: zeros past D
+    float x[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) x[s] = src[s][min(k + h, D - 1)];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) x[s] = k + h < D ? x[s] : 0.f;
+    step(x);
+  }
+  bool direct = false;
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {  // over the row's four lanes
+    nsq[s] += __shfl_xor(nsq[s], 16, 64);
+    nsq[s] += __shfl_xor(nsq[s], 32, 64);
+    direct |= !(nsq[s] <= norm_max);
+  }
+  if (__syncthreads_or(direct)) {
+    nl2k::pairwise::simt_fwd_tile(simt, X, Y, K, (int64_t)N, (int64_t)M, (int64_t)D, (int64_t)i0,
+                                  (int64_t)j0, RbfGenFwd{gamma});
+    return;
+  }
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {  // accumulator r of lane (n, h): row 4 r + h, column n
+      const double nx = __shfl(nsq[a], 4 * r + h, 64);
+      const int i = ib + 16 * a + 4 * r + h;
+      float o[2];
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        const double d2 = fma(-2., acc[a][b][r], nx + nsq[2 + b]);
+        o[b] = exp2f((float)(neg_kappa * fmax(d2, 0.)));
+      }
+      if (i >= N) continue;
+      float* p = K + (size_t)i * M + j;
+      if (j + 1 < M)
+        *reinterpret_cast<f32x2_u*>(p) = f32x2{o[0], o[1]};
+      else if (j < M)
+        p[0] = o[0];
+    }
+}
 
 // ------------------------------------------------------------------ backward
 // out[r][:] = neg2g (sum_s S[s][r] A[r][:] - sum_s P[s][r][:]), one thread
@@ -220,18 +337,28 @@ inline size_t workspace_floats(int64_t N, int64_t M, int64_t D) {
   return std::max(generic_ws_floats(N, M, D), nl2k::pairwise::split_floats(N, M, D, true));
 }
 
-// Largest squared row norm whose distances the forward forms from norms and
-// products (|x|^2 + |y|^2 - 2 x.y); a tile with a larger one (or with a norm
-// that is not finite) sums the squared differences directly.  The former
-// leaves an error of about 2^-24 (|x|^2 + |y|^2) in the distance whatever the
-// distance is, which gamma carries into K: at gamma (|x|^2 + |y|^2) <= 8 the
-// error of K stays within a few 1e-7, as small as the direct sum's.  D = 64
-// takes the products for every finite norm, as it always has.  A negative or
-// NaN gamma always sums directly.
-inline float norm_max(float gamma, int64_t D) {
+// Forward route: D = 64 with 16-byte aligned X, Y on the bf16 splits, whose
+// rounding there is that of the fp32 instructions (24.5 us at 4096^2; 64-bit
+// distances take 51, fp32 instructions 30), everything else in 64 bits: as the
+// reference sums squared differences, near rows keep their distance.
+bool takes_split_forward(int64_t D, const float* X, const float* Y) {
+  return D == kD && nl2k::aligned16(X) && nl2k::aligned16(Y);
+}
+
+// Largest squared row norm whose distances come from norms and products, |x|^2
+// + |y|^2 - 2 x.y; a tile with a larger one (or with a norm that is not
+// finite) sums the squared differences directly.  The former leaves an error
+// in the distance of about 2^-24 of |x|^2 + |y|^2 on the splits and 2^-52 in
+// 64 bits, whatever the distance is, and gamma carries it into K: a few 1e-7
+// at gamma |x|^2 = 4, and a quarter of K's last bit at gamma |x|^2 = 2^24.  A
+// negative or NaN gamma always sums directly.
+inline float split_norm_max(float gamma) {
   if (!(gamma >= 0.f)) return -1.f;
-  const float cap = gamma > 1e7f ? 1e37f / gamma : 1e30f;  // gamma times it stays finite
-  return D == kD || gamma == 0.f ? cap : std::min(cap, 4.f / gamma);
+  return gamma <= 4e-30f ? 1e30f : 4.f / gamma;
+}
+inline double f64_norm_max(float gamma) {
+  if (!(gamma >= 0.f)) return -1.;
+  return gamma == 0.f ? 1e300 : 16777216. / gamma;
 }
 
 int launch_fill_zero(float* p, size_t count, hipStream_t stream) {
@@ -405,11 +532,21 @@ int rbf_forward_f32(const float* X, const float* Y, float* K, int64_t N,
   if (!X || !Y || !K)
     return nl2k::fail(NL2K_ERR_NULL, "rbf_forward_f32: X, Y and K must be non-null");
 
-  const nl2k::pairwise::SplitFwdPlan fp = nl2k::pairwise::plan_split_forward(N, M, D);
-  if (fp.n_jt > 0)
-    return nl2k::pairwise::launch_fwd_split(fp, X, Y, K, N, M, D,
-                                            RbfFwdOp{-gamma * kLog2e, gamma, norm_max(gamma, D)},
-                                            nullptr, nullptr, stream, "rbf_forward_f32");
+  if (takes_split_forward(D, X, Y)) {
+    const nl2k::pairwise::SplitFwdPlan fp = nl2k::pairwise::plan_split_forward(N, M, D);
+    if (fp.n_jt > 0)
+      return nl2k::pairwise::launch_fwd_split(
+          fp, X, Y, K, N, M, D, RbfFwdOp{(float)(-gamma * kLog2e), gamma, split_norm_max(gamma)},
+          nullptr, nullptr, stream, "rbf_forward_f32");
+  }
+  const int64_t n_jt = nl2k::ceil_div(M, (int64_t)kFwdTile);
+  const int64_t n_tiles = nl2k::ceil_div(N, (int64_t)kFwdTile) * n_jt;
+  if (std::max(std::max(N, M), D) <= INT32_MAX - 1024 && n_tiles <= INT32_MAX) {
+    hipLaunchKernelGGL(rbf_fwd_kernel, dim3((unsigned)n_tiles), dim3(256), 0, stream, X, Y, K,
+                       (int)N, (int)M, (int)D, -gamma * kLog2e, f64_norm_max(gamma), gamma,
+                       (int)n_jt);
+    return nl2k::check_launch("rbf_forward_f32");
+  }
   const int64_t ntiles = nl2k::ceil_div(N, (int64_t)nl2k::pairwise::kGT) *
                          nl2k::ceil_div(M, (int64_t)nl2k::pairwise::kGT);
   hipLaunchKernelGGL(nl2k::pairwise::pair_fwd_generic_kernel<RbfGenFwd>,

@@ -113,11 +113,10 @@ __device__ constexpr int kTermB[kProducts] = {0, 2, 1, 0, 1, 0};
 // of a row and leave in one 16-byte store.
 // Bound by vector and matrix issue together (splits and exponentials beside
 // the products) and, at 64 features, by the waits of two tiles per CU; the
-// stores are 5 of 27 us at 4096^2 x 64.  Measured against the fp32 kernels
-// before (MFMA at D = 64, SIMT elsewhere): 31.3 -> 26.9 us at 4096^2 x 64,
-// 103 -> 82 at 8192^2 x 64, 58 -> 27 at 4095 x 4097 x 64, 55 -> 20 at 3000 x
-// 2500 x 100, 118 -> 39 at 4096^2 x 128.  Error against 64 bits (2-norm)
-// 5.4e-8, as before at D = 64, 1.4e-7 -> 5.5e-8 at D = 100 and 128.
+// stores are 5 of 27 us at 4096^2 x 64.  RBF against the fp32 MFMA kernel
+// before: 31.3 -> 26.9 us at 4096^2 x 64, 103 -> 82 at 8192^2 x 64, error against
+// 64 bits (2-norm) 5.7e-8 -> 5.5e-8.  (At other widths the RBF forward sums
+// squared differences, or forms them in 64 bits: cases/rbf.)
 constexpr int kQuarter = 288;
 constexpr int kBlock = 4 * kQuarter;
 
