@@ -424,10 +424,17 @@ constexpr int kBwdThreads = 512;
 constexpr int kStripCols = 256;
 constexpr int kStepRows = 32;
 constexpr int kFeat = 64;  // features per pass
-// Byte offsets of 32 rows of W have to fit 32 bits; rows and columns are
-// indexed with int up to a region past the last one.
-constexpr int64_t kMaxSplitCols = int64_t(1) << 24;
-constexpr int64_t kMaxSplitDim = INT32_MAX - (int64_t(1) << 20);
+// Byte offsets of 32 rows of W (M floats) and of X and the partials (D floats)
+// stay below 2^31; rows are indexed with int up to a step past the last one, and
+// columns up to a strip; a launch holds fewer than 2^32 threads.
+constexpr int64_t kMaxSplitWidth = int64_t(1) << 24;  // M and D
+constexpr int64_t kMaxSplitRows = INT32_MAX - (int64_t(1) << 20);
+constexpr int64_t kMaxSplitBlocks = UINT32_MAX / kBwdThreads;
+
+inline bool split_in_range(int64_t N, int64_t M, int64_t D) {
+  return N > 0 && M > 0 && D > 0 && N <= kMaxSplitRows && M <= kMaxSplitWidth &&
+         D <= kMaxSplitWidth;
+}
 
 struct BwdLds {
   unsigned char w[2][3][2][8][1024];  // [buffer][term][16 rows][32 columns]
@@ -468,7 +475,7 @@ __global__ __launch_bounds__(kBwdThreads) void pair_bwd_split_kernel(
   const int fb = wave & 3, kh = wave >> 2;  // W . Y: features, half of the columns
   const int c = lane & 15, h = lane >> 4;   // also (n, h) of the operands
   const int d0 = dc * kFeat;
-  const int i_begin = ri * RI, i_end = min(N, i_begin + RI);
+  const int i_begin = ri * RI, i_end = i_begin + min(RI, N - i_begin);
   const uint32_t m4 = (uint32_t)M * 4u;
 
   // W stores: columns 32 wave + 2c, + 1 are a quarter of a 16-byte slot of
@@ -774,8 +781,10 @@ __global__ __launch_bounds__(kBwdThreads) void pair_bwd_split_kernel(
 
 // Workspace floats with which a split backward fills the chip: at most 16
 // partial rows for each row of X, one per 256 columns of W, and one for each
-// row of Y per region of at least 256 rows, as many as make 256 workgroups.
+// row of Y per region of at least 256 rows, as many as make 256 workgroups (0:
+// the shape is out of range).
 inline size_t split_floats(int64_t N, int64_t M, int64_t D, bool sums) {
+  if (!split_in_range(N, M, D)) return 0;
   const int64_t nrj = std::min(ceil_div(M, (int64_t)kStripCols), (int64_t)16);
   const int64_t want = ceil_div((int64_t)256, nrj * ceil_div(D, (int64_t)kFeat));
   const int64_t nri = std::min(ceil_div(N, (int64_t)256), want);
@@ -799,8 +808,7 @@ struct SplitBwdPlan {
 inline SplitBwdPlan plan_split_backward(int64_t N, int64_t M, int64_t D, bool sums,
                                         size_t budget) {
   SplitBwdPlan best;
-  if (N <= 0 || M <= 0 || D <= 0 || N > kMaxSplitDim || M > kMaxSplitCols || D > kMaxSplitDim)
-    return best;
+  if (!split_in_range(N, M, D)) return best;
   constexpr double kFill = 1.5, kStepBytes = 15e6;
   const int64_t n_dc = ceil_div(D, (int64_t)kFeat), strips = ceil_div(M, (int64_t)kStripCols);
   const int64_t steps = ceil_div(N, (int64_t)kStepRows), row = D + (sums ? 1 : 0);
@@ -814,7 +822,7 @@ inline SplitBwdPlan plan_split_backward(int64_t N, int64_t M, int64_t D, bool su
       const int64_t nri = ceil_div(steps, k);
       const size_t floats = (size_t)(nrj * N + nri * M) * (size_t)row;
       const int64_t wgs = ceil_div(nri * nrj, (int64_t)8) * 8 * n_dc;
-      if (floats <= budget && wgs <= INT32_MAX && nri * nrj <= INT32_MAX / 2) {
+      if (floats <= budget && wgs <= kMaxSplitBlocks) {
         const double moved = 2.0 * (double)floats + (double)((strips - nrj) * N * row);
         const double c = (double)(ceil_div(nri * nrj * n_dc, (int64_t)256) * sj) * (k + kFill) +
                          moved * sizeof(float) / kStepBytes;

@@ -1,0 +1,71 @@
+"""The pairwise cases past the split kernels' 32-bit offsets, on the general
+kernels.  Against float64; the bound on the 2-norm error is 2^-24 (4 +
+sqrt(k)), k the contraction of a sequential sum."""
+
+import math
+
+import pytest
+import torch
+
+from conftest import announce
+
+pytestmark = pytest.mark.gpu
+
+
+def _close(name, got, ref_of, width, k, step=1 << 20):
+    """got [rows, width] against ref_of(slice of features), in float64."""
+    num = den = 0.0
+    for c in range(0, width, step):
+        s = slice(c, min(c + step, width))
+        ref = ref_of(s)
+        num += float((got[:, s].double() - ref).square().sum())
+        den += float(ref.square().sum())
+    err, tol = math.sqrt(num / den), 2.0 ** -24 * (4 + math.sqrt(k))
+    print(f"  {name}: {err:.2e} of {tol:.2e}")
+    assert err <= tol, name
+
+
+def _rows(n, d, seed):
+    return torch.randn(n, d, device="cuda", generator=torch.Generator("cuda").manual_seed(seed))
+
+
+# 32 rows of this many features pass 3 GiB, the largest buffer resource used
+WIDE = 25_200_004
+
+
+def test_rbf_backward_wide_features():
+    announce(f"rbf backward n=32 m=32 d={WIDE}")
+    from cases.rbf import op
+    n, d, gamma = 32, WIDE, 0.25
+    X, Y, G, K = _rows(n, d, 1), _rows(n, d, 2), _rows(n, n, 3), _rows(n, n, 4).sigmoid()
+    dX, dY = op.rbf_backward(X, Y, G, K, gamma)
+    W = G.double() * K.double()
+    for name, got, A, B, w in (("dX", dX, X, Y, W), ("dY", dY, Y, X, W.t().contiguous())):
+        _close(name, got, lambda s: -2 * gamma * (w.sum(1, keepdim=True) * A[:, s].double()
+                                                  - w @ B[:, s].double()), d, n)
+
+
+def test_cosine_backward_wide_features():
+    announce(f"cosine backward n=32 m=32 d={WIDE}")
+    from cases.cosine_sim import op
+    n, d = 32, WIDE
+    A, B, G = _rows(n, d, 1), _rows(n, d, 2), _rows(n, n, 3)
+    na, nb = (torch.stack([r.double().norm() for r in t]) for t in (A, B))
+    ia, ib = (1 / na).float(), (1 / nb).float()
+    dA, dB = op.cos_backward(A, B, ia, ib, G)
+    for name, got, P, Q, ip, iq, w in (("dA", dA, A, B, ia, ib, G.double()),
+                                       ("dB", dB, B, A, ib, ia, G.double().t().contiguous())):
+        dot = torch.zeros(n, 1, dtype=torch.float64, device="cuda")
+        ip, iq = ip.double()[:, None], iq.double()[:, None]
+
+        def part(s):
+            return P[:, s].double() * ip, w @ (Q[:, s].double() * iq)
+
+        for c in range(0, d, 1 << 20):
+            ph, acc = part(slice(c, c + (1 << 20)))
+            dot += (ph * acc).sum(1, keepdim=True)
+
+        def ref(s):
+            ph, acc = part(s)
+            return ip * (acc - dot * ph)
+        _close(name, got, ref, d, n + d / 64 / 4)
