@@ -541,7 +541,7 @@ int rbf_forward_f32(const float* X, const float* Y, float* K, int64_t N,
   }
   const int64_t n_jt = nl2k::ceil_div(M, (int64_t)kFwdTile);
   const int64_t n_tiles = nl2k::ceil_div(N, (int64_t)kFwdTile) * n_jt;
-  if (std::max(std::max(N, M), D) <= INT32_MAX - 1024 && n_tiles <= INT32_MAX) {
+  if (std::max(std::max(N, M), D) <= INT32_MAX - 1024 && n_tiles <= nl2k::max_blocks(256)) {
     hipLaunchKernelGGL(rbf_fwd_kernel, dim3((unsigned)n_tiles), dim3(256), 0, stream, X, Y, K,
                        (int)N, (int)M, (int)D, -gamma * kLog2e, f64_norm_max(gamma), gamma,
                        (int)n_jt);

@@ -66,6 +66,10 @@ inline int check_hip(hipError_t e, const char* what) {
 
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+// Workgroups of `threads` a launch may have: HIP refuses 2^32 threads and more
+// along one dimension of the grid.
+constexpr int64_t max_blocks(int threads) { return UINT32_MAX / threads; }
+
 // Workgroups of `kernel` (launched with `threads` threads and no dynamic LDS)
 // that the current device holds at once: its CU count times the occupancy
 // the runtime computes from the kernel's registers, LDS and launch bounds.

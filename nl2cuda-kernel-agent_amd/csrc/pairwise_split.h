@@ -375,7 +375,7 @@ inline SplitFwdPlan plan_split_forward(int64_t N, int64_t M, int64_t D) {
   p.tb = cost128 <= 1.05 * cost64 ? 128 : 64;
   const int64_t n_jt = ceil_div(M, (int64_t)p.tb);
   p.n_tiles = ceil_div(N, (int64_t)p.tb) * n_jt;
-  if (p.n_tiles <= INT32_MAX) p.n_jt = (int)n_jt;
+  if (p.n_tiles <= max_blocks(256)) p.n_jt = (int)n_jt;
   return p;
 }
 
@@ -429,7 +429,6 @@ constexpr int kFeat = 64;  // features per pass
 // columns up to a strip; a launch holds fewer than 2^32 threads.
 constexpr int64_t kMaxSplitWidth = int64_t(1) << 24;  // M and D
 constexpr int64_t kMaxSplitRows = INT32_MAX - (int64_t(1) << 20);
-constexpr int64_t kMaxSplitBlocks = UINT32_MAX / kBwdThreads;
 
 inline bool split_in_range(int64_t N, int64_t M, int64_t D) {
   return N > 0 && M > 0 && D > 0 && N <= kMaxSplitRows && M <= kMaxSplitWidth &&
@@ -822,7 +821,7 @@ inline SplitBwdPlan plan_split_backward(int64_t N, int64_t M, int64_t D, bool su
       const int64_t nri = ceil_div(steps, k);
       const size_t floats = (size_t)(nrj * N + nri * M) * (size_t)row;
       const int64_t wgs = ceil_div(nri * nrj, (int64_t)8) * 8 * n_dc;
-      if (floats <= budget && wgs <= kMaxSplitBlocks) {
+      if (floats <= budget && wgs <= max_blocks(kBwdThreads)) {
         const double moved = 2.0 * (double)floats + (double)((strips - nrj) * N * row);
         const double c = (double)(ceil_div(nri * nrj * n_dc, (int64_t)256) * sj) * (k + kFill) +
                          moved * sizeof(float) / kStepBytes;

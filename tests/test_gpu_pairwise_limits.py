@@ -1,5 +1,5 @@
-"""The pairwise cases past the split kernels' 32-bit offsets, on the general
-kernels.  Against float64; the bound on the 2-norm error is 2^-24 (4 +
+"""The pairwise cases past the limits of their tile kernels (32-bit offsets,
+workgroups of a launch), on the general kernels.  Against float64; the bound on the 2-norm error is 2^-24 (4 +
 sqrt(k)), k the contraction of a sequential sum."""
 
 import math
@@ -69,3 +69,35 @@ def test_cosine_backward_wide_features():
             ph, acc = part(s)
             return ip * (acc - dot * ph)
         _close(name, got, ref, d, n + d / 64 / 4)
+
+
+# more outputs in a row than a launch has tiles of 64 columns
+TALL = ((1 << 24) << 6) + 5
+
+
+def _slices(width):
+    return [slice(0, 4096), slice(width // 2, width // 2 + 4096), slice(width - 4096, width)]
+
+
+@pytest.mark.parametrize("turned", [False, True])
+def test_rbf_forward_more_tiles_than_a_launch(turned):
+    announce(f"rbf forward {TALL} outputs, turned={turned}")
+    from cases.rbf import op
+    x, Y = _rows(1, 1, 1), _rows(TALL, 1, 2)
+    K = op.rbf_forward(Y, x, 0.5) if turned else op.rbf_forward(x, Y, 0.5)
+    K = K.flatten()
+    for s in _slices(TALL):
+        ref = torch.exp(-0.5 * (x[0].double() - Y[s, 0].double()).square())
+        assert float((K[s].double() - ref).norm() / ref.norm()) <= 2.0 ** -21
+
+
+def test_cosine_forward_more_tiles_than_a_launch():
+    announce(f"cosine forward {TALL} outputs")
+    from cases.cosine_sim import op
+    a, B = _rows(1, 2, 1), _rows(TALL, 2, 2)
+    S, inv_a, inv_b = op.cos_forward(a, B, 1e-8)
+    for s in _slices(TALL):
+        b, inv = B[s].double(), 1 / (B[s].double().norm(dim=1) + 1e-8)
+        ref = (b * inv[:, None]) @ (a[0].double() / (a.double().norm() + 1e-8))
+        assert float((S[0, s].double() - ref).norm() / ref.norm()) <= 2.0 ** -21
+        assert float((inv_b[s].double() - inv).norm() / inv.norm()) <= 2.0 ** -21

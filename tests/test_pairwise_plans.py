@@ -20,8 +20,9 @@ int main() {
   while (std::scanf("%lld %lld %lld", &n, &m, &d) == 3) {
     const size_t floats = nl2k::pairwise::split_floats(n, m, d, true);
     const auto p = nl2k::pairwise::plan_split_backward(n, m, d, true, floats);
-    std::printf("%d %zu %zu %lld %d\n", (int)p.ok, floats, p.ws_floats,
-                (long long)p.nRI * p.nRJ, p.n_dc);
+    const auto f = nl2k::pairwise::plan_split_forward(n, m, d);
+    std::printf("%d %zu %zu %lld %d %d %lld\n", (int)p.ok, floats, p.ws_floats,
+                (long long)p.nRI * p.nRJ, p.n_dc, f.n_jt, (long long)f.n_tiles);
   }
 }
 """
@@ -53,7 +54,7 @@ WIDTHS = [1, 64, 100, 1 << 20, 1 << 24, (1 << 24) + 1, 17_400_000, 25_165_825, 3
 def test_split_backward_offsets_fit_32_bits(plans):
     shapes = [(n, m, d) for n in SIZES for m in SIZES for d in WIDTHS
               if n * m <= 1 << 36 and n * d <= 1 << 36 and m * d <= 1 << 36]
-    for (n, m, d), (ok, floats, used, regions, passes) in zip(shapes, plans(shapes)):
+    for (n, m, d), (ok, floats, used, regions, passes, *_) in zip(shapes, plans(shapes)):
         if not ok:
             continue
         assert 32 * d * 4 <= 1 << 31, (n, m, d)
@@ -66,3 +67,11 @@ def test_split_backward_takes_ordinary_shapes(plans):
     shapes = [(64, 64, 64), (4096, 4096, 64), (1, 1, 1), (3000, 2500, 100), (100000, 7, 3),
               (7, 100000, 300), (8192, 8192, 256), (32, 32, 1 << 24)]
     assert all(p[0] for p in plans(shapes))
+
+
+def test_split_forward_launches_below_2_32_threads(plans):
+    shapes = [(n, m, 1) for n in SIZES + [(1 << 30) + 65] for m in SIZES if n * m <= 1 << 36]
+    got = plans(shapes)
+    for shape, (*_, n_jt, tiles) in zip(shapes, got):
+        assert n_jt == 0 or tiles * 256 < 1 << 32, shape
+    assert any(p[-2] == 0 for p in got) and any(p[-2] > 0 for p in got)
