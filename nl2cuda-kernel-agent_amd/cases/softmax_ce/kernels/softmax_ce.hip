@@ -655,11 +655,13 @@ int softmax_ce_backward_f32(const float* logits, const int64_t* labels, const fl
     else if (p.v == 4) SCE_BWD(256, 4);
     else SCE_BWD(256, 8);
 #undef SCE_BWD
-  } else if (C > kLongClasses && !(aligned && C % 4 == 0)) {
-    const int u = C > 2048 ? 4 : C > 1024 ? 2 : 1;
-    const int64_t windows = nl2k::ceil_div(C, (int64_t)4);
-    const int64_t segs = nl2k::ceil_div(windows, (int64_t)kBlock * u);
-    if (B * segs > INT32_MAX) return nl2k::fail(NL2K_ERR_OVERFLOW, "%s: sizes too large", who);
+    return nl2k::check_launch(who);
+  }
+  // Ragged rows go by segments of a row while a launch holds them all.
+  const int u = C > 2048 ? 4 : C > 1024 ? 2 : 1;
+  const int64_t windows = nl2k::ceil_div(C, (int64_t)4);
+  const int64_t segs = nl2k::ceil_div(windows, (int64_t)kBlock * u);
+  if (C > kLongClasses && !(aligned && C % 4 == 0) && B <= nl2k::max_blocks(kBlock) / segs) {
     auto* kernel = u == 4   ? &sce_bwd_long_kernel<4>
                    : u == 2 ? &sce_bwd_long_kernel<2>
                             : &sce_bwd_long_kernel<1>;
