@@ -111,6 +111,11 @@ __device__ __forceinline__ int label_col(int64_t lab, int64_t C) {
   return (lab >= 0 && lab < C) ? (int)lab : -1;
 }
 
+// What exponents are taken from: a maximum, or 0 where all is -inf (or NaN), so
+// that exp(-inf - 0) adds 0, a NaN adds NaN, and the lse of a row of -inf is
+// -inf, not -inf - -inf.
+__device__ __forceinline__ float finite_max(float m) { return m == -INFINITY ? 0.f : m; }
+
 // Rows per block step for a width class: enough rows that each thread has
 // about eight float4 loads in flight before the first is used.
 template <int V>
@@ -233,9 +238,8 @@ __global__ __launch_bounds__(kBlock) void sce_fwd_kernel(
       }
     }
     row_reduce<TPR, R, true>(m, red);
-    // a row of -inf alone: lse = -inf (exp(-inf - 0) adds 0), not -inf - -inf
 #pragma unroll
-    for (int r = 0; r < R; ++r) m[r] = m[r] == -INFINITY ? 0.f : m[r];
+    for (int r = 0; r < R; ++r) m[r] = finite_max(m[r]);
     float se[R];  // per row: sum of exp(x - max)
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -307,21 +311,21 @@ __global__ __launch_bounds__(kBlock) void sce_fwd_long_kernel(
 #pragma unroll
         for (int e = 0; e < 4; ++e) cm = fmaxf(cm, e >= skip[u] ? v[u][e] : -INFINITY);
       const float nm = fmaxf(m, cm);
-      if (nm != -INFINITY) {  // nothing but -inf so far adds nothing
-        float cs = 0.f;
+      const float base_m = finite_max(nm);
+      float cs = 0.f;
 #pragma unroll
-        for (int u = 0; u < U; ++u)
+      for (int u = 0; u < U; ++u)
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            cs += e >= skip[u] ? __builtin_amdgcn_exp2f((v[u][e] - nm) * kLog2e) : 0.f;
-        s = s * __builtin_amdgcn_exp2f((m - nm) * kLog2e) + cs;
-        m = nm;
-      }
+        for (int e = 0; e < 4; ++e)
+          cs += e >= skip[u] ? __builtin_amdgcn_exp2f((v[u][e] - base_m) * kLog2e) : 0.f;
+      s = s * __builtin_amdgcn_exp2f((m - base_m) * kLog2e) + cs;
+      m = nm;
     }
     float mm[1] = {m};
     row_reduce<kBlock, 1, true>(mm, red);
     const float M = mm[0];
-    float ss[1] = {M == -INFINITY ? 0.f : s * __builtin_amdgcn_exp2f((m - M) * kLog2e)};
+    // a thread whose windows hold -inf alone has m = -inf and s = 0, or NaN
+    float ss[1] = {m == M ? s : s * __builtin_amdgcn_exp2f((m - M) * kLog2e)};
     row_reduce<kBlock, 1, false>(ss, red);
     if (threadIdx.x == 0) {
       const float lse = M + __builtin_amdgcn_logf(ss[0]) * kLn2;
@@ -355,6 +359,7 @@ __global__ __launch_bounds__(kBlock) void sce_fwd_lane_kernel(
     float m = -INFINITY;
 #pragma unroll
     for (int c = 0; c < CM; ++c) m = fmaxf(m, c < C ? v[c] : -INFINITY);
+    m = finite_max(m);
     float se = 0.f;
 #pragma unroll
     for (int c = 0; c < CM; ++c) se += c < C ? __builtin_amdgcn_exp2f((v[c] - m) * kLog2e) : 0.f;

@@ -28,3 +28,25 @@ def test_backward_more_segments_than_a_launch():
         ref.scatter_add_(1, lab[s, None], torch.full((512, 1), -1.0, dtype=ref.dtype,
                                                      device="cuda"))
         assert float((dx[s].double() - ref).abs().max()) <= 2.0 ** -24 * 2 * (16 + 4)
+
+
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("c", [1, 7, 12, 13, 31, 32, 33, 100, 1024, 1025, 8193, 50257])
+def test_rows_of_infinities(c, offset):
+    """At every width, as torch.logsumexp: a row of -inf has lse = -inf, one NaN
+    among -inf gives NaN, one finite logit among -inf gives that logit."""
+    announce(f"softmax_ce rows of -inf, width {c}, offset {offset}")
+    from cases.softmax_ce import op
+    b = 70
+    x = torch.full((b, c), float("-inf"))
+    x[2, c // 2] = float("nan")
+    x[3] = float("nan")
+    x[4, c - 1] = 2.5
+    x[5:] = torch.randn(b - 5, c, generator=torch.Generator().manual_seed(c))
+    flat = torch.zeros(b * c + offset, device="cuda")
+    xd = flat[offset:].view(b, c)
+    xd.copy_(x)
+    loss, lse = op.sce_forward(xd, torch.zeros(b, dtype=torch.int64, device="cuda"))
+    want = torch.logsumexp(x.double(), 1)
+    assert bool(torch.isnan(loss))
+    assert torch.allclose(lse.cpu().double(), want, rtol=1e-6, atol=1e-6, equal_nan=True)
