@@ -62,17 +62,34 @@ struct CosBwdOp {
 // by L lanes of V features each (the sums over the row's lanes leave every
 // lane the same bits).  The first kKeep groups of a lane stay in registers
 // between the two passes; wider rows add their partials up again.
+// Split partials carry kSplitScale and are added up directly where they are
+// not finite.
 constexpr int kKeep = 4;
-template <int V, int L>
-__device__ __forceinline__ void project_row(const float* __restrict__ P, const float* __restrict__ A,
-                                            const float* __restrict__ inv, float* __restrict__ out,
-                                            int64_t rows, int64_t r, int D, int slots, int lane) {
+
+// One side of the backward: its own rows A, their inverse norms and gradient,
+// the other side's rows B, entry (r, o) of dS at r own + o other.
+struct ReduceSide {
+  const float *P, *A, *inv, *B, *inv_b;
+  float* out;
+  int64_t rows, others;
+  size_t own, other;
+  int slots;
+};
+
+template <int V, int L, bool SPLIT>
+__device__ __forceinline__ void project_row(const ReduceSide& side, const float* __restrict__ dS,
+                                            int64_t r, int D, int lane) {
   typedef float vec __attribute__((ext_vector_type(V), aligned(4)));
+  const float* __restrict__ P = side.P;
+  const float* __restrict__ A = side.A;
+  float* out = side.out;
+  const int64_t rows = side.rows;
+  const int slots = side.slots;
   const int per = D / V;
   const int64_t stride = rows * (int64_t)D;
   const float* p = P + r * D;
   const float* a = A + r * D;
-  const float sc = inv[r];
+  const float sc = side.inv[r];
   auto partial = [&](int e) {
     auto at = [&](int s) { return *reinterpret_cast<const vec*>(p + s * stride + (int64_t)e * V); };
     vec a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
@@ -84,7 +101,8 @@ __device__ __forceinline__ void project_row(const float* __restrict__ P, const f
       a3 += at(s + 3);
     }
     for (; s < slots; ++s) a0 += at(s);
-    return (a0 + a1) + (a2 + a3);
+    const vec acc = (a0 + a1) + (a2 + a3);
+    return SPLIT ? acc * nl2k::pairwise::kPartialUnscale : acc;
   };
   float dot = 0.f, nn = 0.f;
   vec keep[kKeep], row[kKeep];
@@ -107,41 +125,58 @@ __device__ __forceinline__ void project_row(const float* __restrict__ P, const f
   }
   for (int e = lane + L * kKeep; e < per; e += L)
     add(partial(e), *reinterpret_cast<const vec*>(a + (int64_t)e * V));
+  auto over_row = [&](float v) {
 #pragma unroll
-  for (int off = 1; off < L; off <<= 1) {
-    dot += __shfl_xor(dot, off, 64);
-    nn += __shfl_xor(nn, off, 64);
-  }
-  const float nrm = sqrtf(nn);
-  const float coef = nrm > 0.f ? dot / nrm : 0.f;
-  auto store = [&](int e, const vec& acc, const vec& av) {
+    for (int off = 1; off < L; off <<= 1) v += __shfl_xor(v, off, 64);
+    return v;
+  };
+  dot = over_row(dot);
+  const float nrm = sqrtf(over_row(nn));
+  auto store = [&](int e, const vec& acc, const vec& av, float coef) {
     *reinterpret_cast<vec*>(out + r * D + (int64_t)e * V) = sc * acc - coef * (av * sc);
   };
+  if (SPLIT && !(fabsf(dot) < INFINITY)) {  // a partial is not finite, or dot overflowed
+    dot = 0.f;
+    for (int e = lane; e < per; e += L) {
+      vec acc;
+      float sum;
+      nl2k::pairwise::direct_sums<CosBwdOp>(dS, nullptr, (size_t)r * side.own, side.other,
+                                            side.B + (int64_t)e * V, side.inv_b, side.others, D,
+                                            acc, sum);
+      *reinterpret_cast<vec*>(out + r * D + (int64_t)e * V) = acc;  // read back below
+      add(acc, *reinterpret_cast<const vec*>(a + (int64_t)e * V));
+    }
+    dot = over_row(dot);
+    const float coef = nrm > 0.f ? dot / nrm : 0.f;
+    for (int e = lane; e < per; e += L)
+      store(e, *reinterpret_cast<const vec*>(out + r * D + (int64_t)e * V),
+            *reinterpret_cast<const vec*>(a + (int64_t)e * V), coef);
+    return;
+  }
+  const float coef = nrm > 0.f ? dot / nrm : 0.f;
 #pragma unroll
   for (int k = 0; k < kKeep; ++k)
-    if (lane + L * k < per) store(lane + L * k, keep[k], row[k]);
+    if (lane + L * k < per) store(lane + L * k, keep[k], row[k], coef);
   for (int e = lane + L * kKeep; e < per; e += L)
-    store(e, partial(e), *reinterpret_cast<const vec*>(a + (int64_t)e * V));
+    store(e, partial(e), *reinterpret_cast<const vec*>(a + (int64_t)e * V), coef);
 }
 
 // Both outputs in one launch: block b < bx handles dA, the rest dB.  A row's
 // lanes stay together: every lane of a group has the same row.
-template <int V, int L>
-__global__ __launch_bounds__(256) void cos_bwd_reduce_kernel(
-    const float* __restrict__ Px, const float* __restrict__ A,
-    const float* __restrict__ inv_a, float* __restrict__ dA, int64_t N, int sx,
-    const float* __restrict__ Py, const float* __restrict__ B,
-    const float* __restrict__ inv_b, float* __restrict__ dB, int64_t M, int sy, int D, int bx) {
+template <int V, int L, bool SPLIT>
+__global__ __launch_bounds__(256) void cos_bwd_reduce_kernel(ReduceSide x, ReduceSide y,
+                                                             const float* __restrict__ dS, int D,
+                                                             int bx) {
   constexpr int kRows = 256 / L;
   const int b = (int)blockIdx.x;
   const int lane = threadIdx.x % L, g = threadIdx.x / L;
   if (b < bx) {
-    for (int64_t r = (int64_t)b * kRows + g; r < N; r += (int64_t)bx * kRows)
-      project_row<V, L>(Px, A, inv_a, dA, N, r, D, sx, lane);
+    for (int64_t r = (int64_t)b * kRows + g; r < x.rows; r += (int64_t)bx * kRows)
+      project_row<V, L, SPLIT>(x, dS, r, D, lane);
   } else {
     const int64_t nb = (int)gridDim.x - bx;
-    for (int64_t r = (int64_t)(b - bx) * kRows + g; r < M; r += nb * kRows)
-      project_row<V, L>(Py, B, inv_b, dB, M, r, D, sy, lane);
+    for (int64_t r = (int64_t)(b - bx) * kRows + g; r < y.rows; r += nb * kRows)
+      project_row<V, L, SPLIT>(y, dS, r, D, lane);
   }
 }
 
@@ -236,16 +271,19 @@ int fill_zero(float* p, size_t count, hipStream_t stream) {
 }
 
 // Sums the partial rows (sx of each row of A, sy of B) into dA and dB.
+template <bool SPLIT>
 int reduce(const float* px, const float* py, int64_t sx, int64_t sy, const float* A,
-           const float* B, const float* inv_a, const float* inv_b, float* dA, float* dB,
-           int64_t N, int64_t M, int64_t D, hipStream_t stream, const char* who) {
+           const float* B, const float* inv_a, const float* inv_b, const float* dS, float* dA,
+           float* dB, int64_t N, int64_t M, int64_t D, hipStream_t stream, const char* who) {
   const bool vec = D % 4 == 0;
   const bool wide = D > (vec ? 64 : 16);  // a wave per row, else 16 lanes
-  auto* kernel = vec ? (wide ? &cos_bwd_reduce_kernel<4, 64> : &cos_bwd_reduce_kernel<4, 16>)
-                     : (wide ? &cos_bwd_reduce_kernel<1, 64> : &cos_bwd_reduce_kernel<1, 16>);
+  auto* kernel =
+      vec ? (wide ? &cos_bwd_reduce_kernel<4, 64, SPLIT> : &cos_bwd_reduce_kernel<4, 16, SPLIT>)
+          : (wide ? &cos_bwd_reduce_kernel<1, 64, SPLIT> : &cos_bwd_reduce_kernel<1, 16, SPLIT>);
   const int bx = grid_for(N, wide ? 4 : 16, 2048), by = grid_for(M, wide ? 4 : 16, 2048);
-  hipLaunchKernelGGL(kernel, dim3(bx + by), dim3(256), 0, stream, px, A, inv_a, dA, N, (int)sx,
-                     py, B, inv_b, dB, M, (int)sy, (int)D, bx);
+  const ReduceSide x = {px, A, inv_a, B, inv_b, dA, N, M, (size_t)M, 1, (int)sx};
+  const ReduceSide y = {py, B, inv_b, A, inv_a, dB, M, N, 1, (size_t)M, (int)sy};
+  hipLaunchKernelGGL(kernel, dim3(bx + by), dim3(256), 0, stream, x, y, dS, (int)D, bx);
   return nl2k::check_launch(who);
 }
 
@@ -330,16 +368,16 @@ int cosine_sim_backward_f32(const float* A, const float* B, const float* inv_a,
   if (nl2k::pairwise::takes_regions(rp, M, A, B, dS, dS)) {
     st = nl2k::pairwise::launch_bwd_regions<CosBwdOp>(rp, A, B, dS, nullptr, ws, N, M, inv_a,
                                                       inv_b, stream, who);
-    return st ? st : reduce(ws + rp.px, ws + rp.py, rp.nRJ, rp.nRI, A, B, inv_a, inv_b, dA, dB, N,
-                            M, D, stream, who);
+    return st ? st : reduce<false>(ws + rp.px, ws + rp.py, rp.nRJ, rp.nRI, A, B, inv_a, inv_b, dS,
+                                   dA, dB, N, M, D, stream, who);
   }
   const nl2k::pairwise::SplitBwdPlan p =
       nl2k::pairwise::plan_split_backward(N, M, D, false, floats);
   if (p.ok) {
     st = nl2k::pairwise::launch_bwd_split<CosBwdOp>(p, A, B, dS, nullptr, ws, N, M, D, inv_a,
                                                     inv_b, stream, who);
-    return st ? st : reduce(ws + p.px, ws + p.py, p.nRJ, p.nRI, A, B, inv_a, inv_b, dA, dB, N, M,
-                            D, stream, who);
+    return st ? st : reduce<true>(ws + p.px, ws + p.py, p.nRJ, p.nRI, A, B, inv_a, inv_b, dS, dA,
+                                  dB, N, M, D, stream, who);
   }
 
   // generic kernels: the walks in slices when the workspace holds their
@@ -369,8 +407,8 @@ int cosine_sim_backward_f32(const float* A, const float* B, const float* inv_a,
                      gy.chunk, op);
   st = nl2k::check_launch("cosine_sim_backward_f32 (generic dB)");
   if (st) return st;
-  return reduce(dah, dbh, gx.s, gy.s, A, B, inv_a, inv_b, dA, dB, N, M, D, stream,
-                "cosine_sim_backward_f32 (generic reduce)");
+  return reduce<false>(dah, dbh, gx.s, gy.s, A, B, inv_a, inv_b, dS, dA, dB, N, M, D, stream,
+                       "cosine_sim_backward_f32 (generic reduce)");
 }
 
 }  // extern "C"

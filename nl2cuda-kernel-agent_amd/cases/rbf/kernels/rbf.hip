@@ -194,17 +194,30 @@ __global__ __launch_bounds__(256, 2) void rbf_fwd_kernel(
 }
 
 // ------------------------------------------------------------------ backward
+// One side of the backward: its own rows A and their gradient, the other
+// side's rows B, entry (r, o) of dK and K at r own + o other.
+struct ReduceSide {
+  const float *P, *S, *A, *B;
+  float* out;
+  int64_t rows, others;
+  size_t own, other;
+  int slots;
+};
+
 // out[r][:] = neg2g (sum_s S[s][r] A[r][:] - sum_s P[s][r][:]), one thread
 // per V features (V = 4 when D is a multiple of 4: rows then hold whole
 // groups); the slot loop is unrolled by 4 so that the loads of several slots
-// are in flight together.
-template <int V, typename I>
-__device__ __forceinline__ void reduce_side(const float* __restrict__ P,
-                                            const float* __restrict__ S,
-                                            const float* __restrict__ A, float* __restrict__ out,
-                                            int64_t rows, int D, int slots, float neg2g, I first,
-                                            I step) {
+// are in flight together.  Split partials carry kSplitScale and are added up
+// directly where they are not finite.
+template <int V, bool SPLIT, typename I>
+__device__ __forceinline__ void reduce_side(const ReduceSide& side, const float* __restrict__ dK,
+                                            const float* __restrict__ K, int D, float neg2g,
+                                            I first, I step) {
   typedef float vec __attribute__((ext_vector_type(V), aligned(4)));
+  const float* __restrict__ P = side.P;
+  const float* __restrict__ S = side.S;
+  const int64_t rows = side.rows;
+  const int slots = side.slots;
   const I per = (I)(D / V), groups = (I)(rows * per);
   const size_t stride = (size_t)rows * D;
   for (I e = first; e < groups; e += step) {
@@ -229,27 +242,36 @@ __device__ __forceinline__ void reduce_side(const float* __restrict__ P,
       a0 += at(s);
       s0 += q[(size_t)s * rows];
     }
-    const vec acc = (a0 + a1) + (a2 + a3);
-    const float sum = (s0 + s1) + (s2 + s3);
-    const vec a = *reinterpret_cast<const vec*>(A + (size_t)e * V);
-    *reinterpret_cast<vec*>(out + (size_t)e * V) = neg2g * (sum * a - acc);
+    vec acc = (a0 + a1) + (a2 + a3);
+    float sum = (s0 + s1) + (s2 + s3);
+    if constexpr (SPLIT) {
+      bool finite = fabsf(sum) < INFINITY;
+#pragma unroll
+      for (int v = 0; v < V; ++v) finite &= fabsf(acc[v]) < INFINITY;
+      sum *= nl2k::pairwise::kSumUnscale;
+      acc *= nl2k::pairwise::kPartialUnscale;
+      if (!finite)
+        nl2k::pairwise::direct_sums<RbfBwdOp>(dK, K, (size_t)r * side.own, side.other,
+                                              side.B + (size_t)(e - r * per) * V, nullptr,
+                                              side.others, D, acc, sum);
+    }
+    const vec a = *reinterpret_cast<const vec*>(side.A + (size_t)e * V);
+    *reinterpret_cast<vec*>(side.out + (size_t)e * V) = neg2g * (sum * a - acc);
   }
 }
 
 // Both outputs in one launch: block b < bx handles dX, the rest dY.
-template <int V, typename I>
-__global__ __launch_bounds__(256) void rbf_bwd_reduce_kernel(
-    const float* __restrict__ Px, const float* __restrict__ Rx,
-    const float* __restrict__ X, float* __restrict__ dX, int N, int sx,
-    const float* __restrict__ Py, const float* __restrict__ Ry,
-    const float* __restrict__ Y, float* __restrict__ dY, int M, int sy, int D,
-    int bx, float neg2g) {
+template <int V, bool SPLIT, typename I>
+__global__ __launch_bounds__(256) void rbf_bwd_reduce_kernel(ReduceSide x, ReduceSide y,
+                                                             const float* __restrict__ dK,
+                                                             const float* __restrict__ K, int D,
+                                                             int bx, float neg2g) {
   const int b = (int)blockIdx.x;
   if (b < bx)
-    reduce_side<V, I>(Px, Rx, X, dX, N, D, sx, neg2g, (I)b * 256 + threadIdx.x, (I)bx * 256);
+    reduce_side<V, SPLIT, I>(x, dK, K, D, neg2g, (I)b * 256 + threadIdx.x, (I)bx * 256);
   else
-    reduce_side<V, I>(Py, Ry, Y, dY, M, D, sy, neg2g, (I)(b - bx) * 256 + threadIdx.x,
-                      (I)((int)gridDim.x - bx) * 256);
+    reduce_side<V, SPLIT, I>(y, dK, K, D, neg2g, (I)(b - bx) * 256 + threadIdx.x,
+                             (I)((int)gridDim.x - bx) * 256);
 }
 
 // ------------------------------------------------------- generic (any D)
@@ -378,21 +400,22 @@ bool needs_workspace(int64_t N, int64_t M, int64_t D, const float* X, const floa
          nl2k::aligned16(dX) && nl2k::aligned16(dY);
 }
 
-template <class Plan>
-int reduce(const Plan& p, const float* ws, const float* X, const float* Y, float* dX,
-           float* dY, int64_t N, int64_t M, int64_t D, float neg2g, hipStream_t stream,
-           const char* who) {
+template <bool SPLIT, class Plan>
+int reduce(const Plan& p, const float* ws, const float* X, const float* Y, const float* dK,
+           const float* K, float* dX, float* dY, int64_t N, int64_t M, int64_t D, float neg2g,
+           hipStream_t stream, const char* who) {
   const int64_t v = D % 4 == 0 ? 4 : 1;
   const int64_t gx = N * (D / v), gy = M * (D / v);
   const int bx = (int)std::min<int64_t>(nl2k::ceil_div(gx, (int64_t)256), 2048);
   const int by = (int)std::min<int64_t>(nl2k::ceil_div(gy, (int64_t)256), 2048);
   const bool small = std::max(gx, gy) < (int64_t(1) << 31);  // the strides fit 32 bits beside it
-  auto* kernel = v == 4 ? (small ? &rbf_bwd_reduce_kernel<4, uint32_t>
-                                 : &rbf_bwd_reduce_kernel<4, uint64_t>)
-                        : (small ? &rbf_bwd_reduce_kernel<1, uint32_t>
-                                 : &rbf_bwd_reduce_kernel<1, uint64_t>);
-  hipLaunchKernelGGL(kernel, dim3(bx + by), dim3(256), 0, stream, ws + p.px, ws + p.rx, X, dX,
-                     (int)N, p.nRJ, ws + p.py, ws + p.ry, Y, dY, (int)M, p.nRI, (int)D, bx, neg2g);
+  auto* kernel = v == 4 ? (small ? &rbf_bwd_reduce_kernel<4, SPLIT, uint32_t>
+                                 : &rbf_bwd_reduce_kernel<4, SPLIT, uint64_t>)
+                        : (small ? &rbf_bwd_reduce_kernel<1, SPLIT, uint32_t>
+                                 : &rbf_bwd_reduce_kernel<1, SPLIT, uint64_t>);
+  const ReduceSide x = {ws + p.px, ws + p.rx, X, Y, dX, N, M, (size_t)M, 1, p.nRJ};
+  const ReduceSide y = {ws + p.py, ws + p.ry, Y, X, dY, M, N, 1, (size_t)M, p.nRI};
+  hipLaunchKernelGGL(kernel, dim3(bx + by), dim3(256), 0, stream, x, y, dK, K, (int)D, bx, neg2g);
   return nl2k::check_launch(who);
 }
 
@@ -428,14 +451,14 @@ int backward_impl(const float* X, const float* Y, const float* dK, const float* 
         nl2k::pairwise::takes_regions(rp, M, X, Y, dK, K)) {
       st = nl2k::pairwise::launch_bwd_regions<RbfBwdOp>(rp, X, Y, dK, K, ws, N, M, nullptr,
                                                         nullptr, stream, who);
-      return st ? st : reduce(rp, ws, X, Y, dX, dY, N, M, D, neg2g, stream, who);
+      return st ? st : reduce<false>(rp, ws, X, Y, dK, K, dX, dY, N, M, D, neg2g, stream, who);
     }
     const nl2k::pairwise::SplitBwdPlan p =
         nl2k::pairwise::plan_split_backward(N, M, D, true, floats);
     if (p.ok) {
       st = nl2k::pairwise::launch_bwd_split<RbfBwdOp>(p, X, Y, dK, K, ws, N, M, D, nullptr,
                                                       nullptr, stream, who);
-      return st ? st : reduce(p, ws, X, Y, dX, dY, N, M, D, neg2g, stream, who);
+      return st ? st : reduce<true>(p, ws, X, Y, dK, K, dX, dY, N, M, D, neg2g, stream, who);
     }
   }
 
