@@ -89,7 +89,11 @@ size_t spmv_backward_workspace_bytes(int64_t M, int64_t K, int64_t D, int64_t nn
  * size above, or, at D > 1 with more than 16384 columns (where that is 0),
  * room for the entries grouped by bucket of columns (16 bytes per nonzero),
  * whose columns are then summed in LDS instead of with atomics: 981 against
- * 90 us on 100000 rows and columns, 1.6 M nonzeros, D = 32.  A call with less runs as the size above says. */
+ * 90 us on 100000 rows and columns, 1.6 M nonzeros, D = 32.  A call with less
+ * runs as the size above says.  0, and atomics, where more than 8192 buckets
+ * would be needed, of 1024 columns or of the largest power of two up to
+ * 8192 / D (K > 2^23 up to D = 8, K > 2^19 at D = 128), and from 2^30 nonzeros
+ * on. */
 size_t spmv_backward_best_workspace_bytes(int64_t M, int64_t K, int64_t D, int64_t nnz);
 
 /* Byte offset in that workspace of a uint32 trip counter for shapes that

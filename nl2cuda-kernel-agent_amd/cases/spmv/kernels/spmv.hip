@@ -2925,10 +2925,11 @@ int transpose_backward(const TransposePlan& tp, const I* ptr, const I* col, cons
 }
 
 // dX by column buckets (spmm_c_* kernels): D > 1, K past the column-major
-// copy's limit.  Buckets of a power of two of columns, as many as keep an
-// average bucket's entries within one round of the gather and its rows within
-// kCbFloats.  Workspace: counts [nb], cursors [nb], the number of parts, parts
-// (16 B each), records [nnz] (16 B).
+// copy's limit.  Buckets of a power of two of columns: their rows within
+// kCbFloats, an average bucket's entries within one round of the gather, and
+// past one where there would be more than kCbMaxBuckets.  Workspace: counts
+// [nb], cursors [nb], the number of parts, parts (16 B each), records [nnz]
+// (16 B).
 struct ColBucketPlan {
   bool use = false;
   int shift = 0, nb = 0;
@@ -2943,10 +2944,11 @@ ColBucketPlan col_bucket_plan(int64_t M, int64_t K, int64_t D, int64_t nnz) {
     return p;
   const double avg = (double)nnz / (double)K;
   int shift = 1;
+  auto buckets = [&] { return nl2k::ceil_div(K, (int64_t)1 << shift); };
   while ((2 << shift) <= kCbMaxCols && ((int64_t)2 << shift) * D <= kCbFloats &&
-         (double)(2 << shift) * avg <= 0.9 * kCbCap)
+         ((double)(2 << shift) * avg <= 0.9 * kCbCap || buckets() > kCbMaxBuckets))
     ++shift;
-  const int64_t nb = nl2k::ceil_div(K, (int64_t)1 << shift);
+  const int64_t nb = buckets();
   if (nb > kCbMaxBuckets) return p;
   p.use = true;
   p.shift = shift;

@@ -370,3 +370,15 @@ def test_delivery_archive_exports_every_declared_symbol():
     for header in ("rbf_delivery.h", "rbf.h"):
         missing = [n for n in declared_functions(header) if n not in defined]
         assert not missing, f"{header}: not in librbf.a: {missing}"
+
+
+def test_spmv_best_workspace_covers_many_entries_without_gpu():
+    """The column-bucket route's workspace is reported up to 8192 buckets of
+    1024 columns or 8192 / D, however many entries a bucket then holds."""
+    lib = _load("cases.spmv.op")
+    best = lib.spmv_backward_best_workspace_bytes
+    for m, k, d, nnz in [(2**20, 100000, 4, 2**24), (2**18, 20000, 4, 2**24), (2**20, 2**20, 2, 2**24),
+                         (2**20, 2**20, 64, 2**26), (1000, 2**23, 8, 2**29), (1000, 2**19, 128, 2**24)]:
+        assert best(m, k, d, nnz) >= 16 * nnz, (m, k, d, nnz)
+    for m, k, d, nnz in [(1000, 2**23 + 1, 8, 2**20), (1000, 2**19 + 1, 128, 2**20), (1000, 20000, 4, 2**30)]:
+        assert best(m, k, d, nnz) == 0, (m, k, d, nnz)

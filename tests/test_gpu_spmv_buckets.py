@@ -70,6 +70,15 @@ def test_spmm_hub_columns(m, mean, d):
     _check(lens, 20000, d, torch.int32, hub=True, seed=m)
 
 
+@pytest.mark.parametrize("m,mean,k,d", [(1 << 18, 64, 20000, 2), (1 << 20, 15, 1 << 20, 3)])
+def test_spmm_many_entries(m, mean, k, d):
+    """More entries than 8192 buckets hold in one round of the gather each."""
+    from cases.spmv import op
+    lib = op._lib()
+    assert lib.spmv_backward_best_workspace_bytes(m, k, d, m * mean) >= 16 * m * mean
+    _check(np.full(m, mean), k, d, torch.int32, seed=d)
+
+
 @pytest.mark.parametrize("d", [1 + 1, 6, 16, 20, 40, 100, 260])
 def test_spmm_long_rows(d):
     """Rows one short of, at and past the length a workgroup shares, between
