@@ -43,8 +43,9 @@ int cosine_sim_forward_f32(const float* A, const float* B, float* S, float* inv_
                            float* inv_b, int64_t N, int64_t M, int64_t D, float eps,
                            hipStream_t stream);
 
-/* Workspace bytes cosine_sim_backward_f32 needs (scratch: no initial
- * contents, nothing kept; 16-byte aligned). */
+/* Workspace bytes for cosine_sim_backward_f32 (scratch: no initial contents,
+ * nothing kept; 16-byte aligned).  At D != 64 it also runs with less, if slower,
+ * down to 4 (N + M) D bytes. */
 size_t cosine_sim_backward_workspace_bytes(int64_t N, int64_t M, int64_t D);
 
 /* dA [N, D], dB [M, D] from dS [N, M], given A, B and the forward's inverse

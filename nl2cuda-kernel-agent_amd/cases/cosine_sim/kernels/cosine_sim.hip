@@ -300,6 +300,13 @@ size_t workspace_floats(int64_t N, int64_t M, int64_t D) {
                   nl2k::pairwise::split_floats(N, M, D, false));
 }
 
+// What a call needs at least: all of that at D = 64, else one partial row for
+// each row.
+size_t least_floats(int64_t N, int64_t M, int64_t D) {
+  return D == nl2k::pairwise::kD ? workspace_floats(N, M, D)
+                                 : generic_ws_floats(N, M, D, false);
+}
+
 }  // namespace
 
 extern "C" {
@@ -356,7 +363,7 @@ int cosine_sim_backward_f32(const float* A, const float* B, const float* inv_a,
   if (M == 0) return fill_zero(dA, (size_t)(N * D), stream);
   if (N == 0) return fill_zero(dB, (size_t)(M * D), stream);
   if (!dS) return nl2k::fail(NL2K_ERR_NULL, "%s: dS must be non-null", who);
-  const size_t floats = workspace_floats(N, M, D), need = floats * sizeof(float);
+  const size_t floats = workspace_floats(N, M, D), need = least_floats(N, M, D) * sizeof(float);
   if (workspace == nullptr || workspace_bytes < need)
     return nl2k::fail(NL2K_ERR_WORKSPACE, "%s: workspace of %zu bytes required, got %zu", who,
                       need, workspace ? workspace_bytes : (size_t)0);
@@ -372,7 +379,8 @@ int cosine_sim_backward_f32(const float* A, const float* B, const float* inv_a,
                                    dA, dB, N, M, D, stream, who);
   }
   const nl2k::pairwise::SplitBwdPlan p =
-      nl2k::pairwise::plan_split_backward(N, M, D, false, floats);
+      nl2k::pairwise::plan_split_backward(N, M, D, false,
+                                          std::min(floats, workspace_bytes / sizeof(float)));
   if (p.ok) {
     st = nl2k::pairwise::launch_bwd_split<CosBwdOp>(p, A, B, dS, nullptr, ws, N, M, D, inv_a,
                                                     inv_b, stream, who);

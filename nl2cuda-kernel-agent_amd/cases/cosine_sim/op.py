@@ -79,8 +79,8 @@ def cos_backward(A, B, inv_a, inv_b, dS):
     D = A.size(1)
     dA = torch.empty_like(A)
     dB = torch.empty_like(B)
-    ws_bytes = _workspace_bytes(N, M, D)
-    ws = A.new_empty((max(ws_bytes, 4) + 3) // 4)
+    best = _workspace_bytes(N, M, D)
+    ws, ws_bytes = capi.scratch(A, best, best if D == 64 else 4 * (N + M) * D)
     st = capi.launch(lib.cosine_sim_backward_f32, A.get_device(), A.data_ptr(), B.data_ptr(),
                      inv_a.data_ptr(), inv_b.data_ptr(), dS.data_ptr(), dA.data_ptr(),
                      dB.data_ptr(), N, M, D, ws.data_ptr(), ws_bytes)

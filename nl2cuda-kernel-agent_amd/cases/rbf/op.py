@@ -88,8 +88,8 @@ def rbf_backward(X, Y, G, K, gamma):
     M = Y.size(0)
     dX = torch.empty_like(X)
     dY = torch.empty_like(Y)
-    ws_bytes = _workspace_bytes(N, M, D)
-    ws = X.new_empty((max(ws_bytes, 4) + 3) // 4)
+    best = _workspace_bytes(N, M, D)
+    ws, ws_bytes = capi.scratch(X, best, best if D == 64 else 0)
     st = capi.launch(lib.rbf_backward_f32, X.get_device(), X.data_ptr(), Y.data_ptr(),
                      G.data_ptr(), K.data_ptr(), dX.data_ptr(), dY.data_ptr(), N, M, D,
                      float(gamma), ws.data_ptr(), ws_bytes)

@@ -68,7 +68,10 @@ def _suffix(row_ptr, col_idx):
 
 @functools.lru_cache(maxsize=256)
 def _workspace_bytes(M, K, D, nnz):
-    return _lib().spmv_backward_best_workspace_bytes(M, K, D, nnz)
+    """(bytes of the fastest route, bytes the call needs)."""
+    lib = _lib()
+    return (lib.spmv_backward_best_workspace_bytes(M, K, D, nnz),
+            lib.spmv_backward_workspace_bytes(M, K, D, nnz))
 
 
 @functools.lru_cache(maxsize=None)
@@ -176,13 +179,13 @@ def spmv_backward(row_ptr, col_idx, vals, X, grad_Y, need_vals=True, need_X=True
     grad_vals = torch.empty_like(vals) if need_vals else None
     grad_X = torch.empty_like(X) if need_X else None
     nnz = vals.numel()
-    ws_bytes = _workspace_bytes(M, K, D, nnz) if need_X else 0
-    ws = torch.empty(max(ws_bytes, 8), dtype=torch.uint8, device=X.device)  # scratch
+    best, least = _workspace_bytes(M, K, D, nnz) if need_X else (0, 0)
+    ws, ws_bytes = capi.scratch(X, best, least)
     status = None
     if need_X and capi.checking() and not torch.cuda.is_current_stream_capturing():
         off = lib.spmv_status_offset(M, K, D, nnz)
         if off != SIZE_MAX:
-            status = ws[off:off + 8].view(torch.int64)
+            status = ws[off // 4:off // 4 + 2].view(torch.int64)
             status.zero_()
     tail = (grad_Y.data_ptr(), grad_vals.data_ptr() if need_vals else None,
             grad_X.data_ptr() if need_X else None, M, K, D, nnz, ws.data_ptr(), ws_bytes)

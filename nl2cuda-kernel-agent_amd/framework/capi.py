@@ -72,6 +72,18 @@ def launch(fn, device, *args):
         return fn(*args, _current_raw_stream(device))
 
 
+def scratch(like, best, least):
+    """A workspace of ``best`` bytes beside the float32 tensor ``like``, or of
+    ``least`` where that does not fit: (tensor, bytes).  For calls that run with
+    less, if slower."""
+    try:
+        return like.new_empty((max(best, 8) + 3) // 4), best
+    except torch.OutOfMemoryError:
+        if least >= best:
+            raise
+    return like.new_empty((max(least, 8) + 3) // 4), least
+
+
 def require(cond, msg):
     """TORCH_CHECK equivalent for the Python boundary."""
     if not cond:
