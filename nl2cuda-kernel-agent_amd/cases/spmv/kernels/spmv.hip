@@ -2147,7 +2147,8 @@ __global__ __launch_bounds__(kCbThreads) void spmm_c_gather_kernel(
             }
           }
         };
-        // a lane's own columns of row r (of dY or of the LDS copy of X)
+        // a lane's own columns of a row (of dY and of the LDS copy of X, where a
+        // zero beside an infinity of another lane's would make a NaN)
         auto own = [&](typename V::T v) {
           if constexpr (MODE == kCbTail) {
 #pragma unroll
@@ -2181,7 +2182,7 @@ __global__ __launch_bounds__(kCbThreads) void spmm_c_gather_kernel(
             if (in) sum += __int_as_float(r[u][2]) * gy[u];
             if constexpr (DV) {
               const float dt =
-                  group_sum<L>(active ? V::dot(gy[u], lds_row(xs + r[u][3] * (int)D + dc)) : 0.f);
+                  group_sum<L>(active ? V::dot(gy[u], own(lds_row(xs + r[u][3] * (int)D + dc))) : 0.f);
               const int64_t p = min(max((int64_t)r[u][1], (int64_t)0), nnz - 1);
               if (in && gl == 0) dvals[p] = dt;
             }

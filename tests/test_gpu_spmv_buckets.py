@@ -118,3 +118,26 @@ def test_spmm_few_long_columns(k, d):
     """Few columns of many entries: 1 to 16 lane groups share a column."""
     lens = np.random.default_rng(k).integers(0, 30, 700)
     _check(lens, k, d, torch.int64 if d % 2 else torch.int32, seed=d)
+
+
+@pytest.mark.parametrize("d", [3, 4, 5, 6, 7, 33, 130])
+def test_spmm_bucket_infinities(d):
+    """An infinite entry of X, dY or vals reaches the outputs it belongs to and
+    no other: lanes that share a row's last four columns keep apart."""
+    from cases.spmv import op
+    announce(f"spmm buckets with infinities, D={d}")
+    m, k = 700, 20000
+    ptr, col = _csr(np.full(m, 9), k, d, False)
+    g = torch.Generator().manual_seed(d)
+    vals, X, G = (torch.randn(*s, generator=g) for s in ((9 * m,), (k, d), (m, d)))
+    # column d - 4 is loaded by the last lane, and another's where d % 4 != 0
+    X[col[5], max(d - 4, 0)], X[col[900], d - 1] = math.inf, -math.inf
+    G[300, d - 2] = math.inf
+    vals[4000] = math.inf
+    dv, dx = op.spmv_backward(ptr.int().cuda(), col.int().cuda(), vals.cuda(), X.cuda(), G.cuda())
+    rows = torch.repeat_interleave(torch.arange(m), 9)
+    want_v = (G[rows].double() * X[col].double()).sum(1)
+    want_x = torch.zeros(k, d, dtype=torch.float64).index_add_(
+        0, col, vals.double()[:, None] * G[rows].double())
+    for name, got, want in (("dvals", dv.cpu(), want_v), ("dX", dx.cpu(), want_x)):
+        assert torch.allclose(got.double(), want, rtol=1e-5, atol=1e-5, equal_nan=True), name
