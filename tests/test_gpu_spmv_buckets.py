@@ -141,3 +141,38 @@ def test_spmm_bucket_infinities(d):
         0, col, vals.double()[:, None] * G[rows].double())
     for name, got, want in (("dvals", dv.cpu(), want_v), ("dX", dx.cpu(), want_x)):
         assert torch.allclose(got.double(), want, rtol=1e-5, atol=1e-5, equal_nan=True), name
+
+
+@pytest.mark.parametrize("hub", [False, True])
+def test_spmm_bucket_backward_graph_replays_with_new_inputs(hub):
+    """The route captured once (counts cleared by a kernel, places reserved with
+    atomics) and replayed on new dY, with buckets of one part and of several:
+    every replay against float64 and an eager call, whose additions come in
+    another order."""
+    from test_gpu_graph_capture import _capture
+    from cases.spmv import op
+    m, k, d = 4000, 20000, 8
+    announce(f"spmm buckets graph capture, hub={hub}")
+    ptr, col = _csr(np.full(m, 20), k, 3, hub)
+    g = torch.Generator().manual_seed(3)
+    vals, X = torch.randn(20 * m, generator=g), torch.randn(k, d, generator=g)
+    args = [t.cuda() for t in (ptr.int(), col.int(), vals, X)]
+    dy = torch.zeros(m, d, device="cuda")
+    graph, (dv, dx) = _capture(lambda: op.spmv_backward(*args, dy))
+    rows = torch.repeat_interleave(torch.arange(m), 20)
+    tol = 2.0 ** -24 * (3 + math.sqrt(int(torch.bincount(col).max()) / 3))
+    for seed in range(4):
+        G = torch.randn(m, d, generator=g)
+        dy.copy_(G.cuda())
+        graph.replay()
+        torch.cuda.synchronize()
+        want = torch.zeros(k, d, dtype=torch.float64).index_add_(
+            0, col, vals.double()[:, None] * G[rows].double())
+        want_v = (G[rows].double() * X[col].double()).sum(1)
+        edv, edx = op.spmv_backward(*args, dy.clone())
+        torch.cuda.synchronize()
+        for name, a, b in (("dX", dx, want), ("eager dX", edx, want), ("dvals", dv, want_v)):
+            err = float((a.cpu().double() - b).norm() / b.norm())
+            print(f"  replay {seed} {name}: {err:.2e} of {tol:.2e}")
+            assert err <= tol, name
+        assert torch.equal(edv, dv)
