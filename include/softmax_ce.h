@@ -56,14 +56,16 @@ size_t softmax_ce_status_offset(void);
 
 /* loss [1] and lse [B] (softmax_ce_forward.cu:52-65, `softmax_ce_forward`;
  * lse is extra: the backward reuses it instead of recomputing each row's
- * max and sum).  The row-cached path runs for C % 4 == 0, C <= 8192 and a
- * 16-byte aligned `logits`; other shapes use a generic kernel. */
+ * max and sum).  Rows of at most 8192 classes are read once into registers, at
+ * any width and alignment, longer ones in one pass with a running maximum.  A
+ * row of -inf has lse = -inf and makes the loss NaN. */
 int softmax_ce_forward_f32(const float* logits, const int64_t* labels, float* loss, float* lse,
                            int64_t B, int64_t C, void* workspace, size_t workspace_bytes,
                            hipStream_t stream);
 
 /* dlogits [B, C] from the forward's lse and the upstream gradient gout [1]
- * (a device pointer, read by the kernel; softmax_ce_backward.cu:57-70). */
+ * (a device pointer, read by the kernel; softmax_ce_backward.cu:57-70).
+ * dlogits may be logits itself, and must not overlap it otherwise. */
 int softmax_ce_backward_f32(const float* logits, const int64_t* labels, const float* lse,
                             const float* gout, float* dlogits, int64_t B, int64_t C,
                             hipStream_t stream);

@@ -29,9 +29,9 @@
 //  * Backward: lse saved by the forward turns the gradient into a pure
 //    streaming pass (read logits, write dlogits, no reductions).  Aligned
 //    float4 rows of 1025 to 8192 classes are laid out like the forward, so
-//    each row's lse and label are read once; ragged rows of 512 classes
-//    or more go by segments of a row; the others stream flat, four floats a
-//    lane whatever the rows.
+//    each row's lse and label are read once; ragged rows of more than 512
+//    classes go by segments of a row; the others stream flat, four floats a
+//    lane where rows are aligned float4 and one where they are not.
 //  * A label outside [0, C) makes its row's loss term and gradient NaN (the
 //    reference would index out of the row; torch raises).
 //  * Unaligned rows (or C % 4 != 0) of at most 32 classes take a lane each
@@ -662,11 +662,14 @@ int softmax_ce_backward_f32(const float* logits, const int64_t* labels, const fl
 #undef SCE_BWD
     return nl2k::check_launch(who);
   }
-  // Ragged rows go by segments of a row while a launch holds them all.
+  // Ragged rows go by segments of a row, while a launch holds them all and the
+  // gradient does not take the logits' place (a segment reads columns that
+  // another may have written then).
   const int u = C > 2048 ? 4 : C > 1024 ? 2 : 1;
   const int64_t windows = nl2k::ceil_div(C, (int64_t)4);
   const int64_t segs = nl2k::ceil_div(windows, (int64_t)kBlock * u);
-  if (C > kLongClasses && !(aligned && C % 4 == 0) && B <= nl2k::max_blocks(kBlock) / segs) {
+  if (C > kLongClasses && !(aligned && C % 4 == 0) && B <= nl2k::max_blocks(kBlock) / segs &&
+      dlogits != logits) {
     auto* kernel = u == 4   ? &sce_bwd_long_kernel<4>
                    : u == 2 ? &sce_bwd_long_kernel<2>
                             : &sce_bwd_long_kernel<1>;

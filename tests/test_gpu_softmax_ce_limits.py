@@ -50,3 +50,22 @@ def test_rows_of_infinities(c, offset):
     want = torch.logsumexp(x.double(), 1)
     assert bool(torch.isnan(loss))
     assert torch.allclose(lse.cpu().double(), want, rtol=1e-6, atol=1e-6, equal_nan=True)
+
+
+@pytest.mark.parametrize("b,c", [(3000, 513), (700, 1029), (300, 2051), (64, 50257), (500, 4096),
+                                 (500, 100)])
+def test_backward_in_place(b, c):
+    """The gradient written over the logits, by whichever kernel."""
+    announce(f"softmax_ce backward in place [{b}, {c}]")
+    from cases.softmax_ce import op
+    from framework import capi
+    g = torch.Generator("cuda").manual_seed(c)
+    x = torch.randn(b, c, device="cuda", generator=g)
+    lab = torch.randint(0, c, (b,), device="cuda", generator=g)
+    _, lse = op.sce_forward(x, lab)
+    one = torch.ones(1, device="cuda")
+    want = op.sce_backward(x, lab, lse, one)
+    lib, P = op._lib(), capi.ptr
+    st = lib.softmax_ce_backward_f32(P(x), P(lab), P(lse), P(one), P(x), b, c, capi.stream_of(x))
+    capi.check(st, lib.softmax_ce_last_error, "sce_backward")
+    assert torch.allclose(x, want, rtol=1e-6, atol=1e-12)
