@@ -23,7 +23,7 @@
 //    rows scaled by inv_a / inv_b), on the bf16 splits or, for small shapes
 //    at D = 64, on fp32 MFMA (csrc/pairwise_d64.h); cos_bwd_reduce_kernel sums
 //    the partials and applies the projection.
-//  * Past those kernels' index ranges the tiled SIMT kernels of
+//  * Past those kernels' ranges the tiled SIMT kernels of
 //    csrc/pairwise_generic.h run (rows scaled by their inverse norms as they
 //    are staged), the backward's walks in slices whose partial rows the
 //    same reduce adds in order.
@@ -36,7 +36,6 @@
 #include "../../../csrc/pairwise_generic.h"
 #include "../../../csrc/pairwise_split.h"
 #include "cosine_sim.h"
-
 
 namespace {
 

@@ -20,7 +20,7 @@
 //    bf16 splits or, for small shapes at D = 64, on fp32 MFMA
 //    (csrc/pairwise_d64.h); rbf_bwd_reduce_kernel sums the slots and applies
 //    dX = -2 gamma (rowsum(W) X - W Y), dY = -2 gamma (colsum(W) Y - W^T X).
-//  * Without a workspace, or past the kernels' index ranges, tiled SIMT
+//  * Without a workspace, or past the kernels' ranges, tiled SIMT
 //    kernels run: W formed in LDS and walked in slices whose partial sums a
 //    reduce kernel adds in order (unsplit when the caller passes no workspace
 //    for them).

@@ -70,11 +70,6 @@ inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // along one dimension of the grid.
 constexpr int64_t max_blocks(int threads) { return UINT32_MAX / threads; }
 
-// Workgroups of `kernel` (launched with `threads` threads and no dynamic LDS)
-// that the current device holds at once: its CU count times the occupancy
-// the runtime computes from the kernel's registers, LDS and launch bounds.
-// Cached per (device, kernel), so instantiations with equal signatures but
-// different register counts keep their own figures.
 // Raises `kernel`'s dynamic LDS limit to at least `bytes` on the current
 // device.  The attribute call is made once per (device, kernel) and size
 // increase; later calls, captured into a graph or not, make none.
@@ -93,6 +88,11 @@ inline int raise_dynamic_lds(const void* kernel, int bytes) {
   return st;
 }
 
+// Workgroups of `kernel` (launched with `threads` threads and no dynamic LDS)
+// that the current device holds at once: its CU count times the occupancy
+// the runtime computes from the kernel's registers, LDS and launch bounds.
+// Cached per (device, kernel), so instantiations with equal signatures but
+// different register counts keep their own figures.
 inline int resident_blocks(const void* kernel, int threads, int* out) {
   static std::mutex mu;
   static std::map<std::pair<int, const void*>, int> cache;

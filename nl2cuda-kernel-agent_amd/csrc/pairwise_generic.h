@@ -1,7 +1,10 @@
 // Tiled SIMT kernels for pairwise row operations between X [N, D] and
-// Y [M, D] at any D and alignment: the shapes the fp32 MFMA tile engine
-// (pairwise_d64.h) does not take.  Shared by the RBF and cosine-similarity
-// cases through small policies.
+// Y [M, D] at any D, alignment and size, in 64-bit indices.  Shared by the RBF
+// and cosine-similarity cases through small policies, for what their matrix
+// kernels (pairwise_split.h, pairwise_d64.h, rbf.hip) do not take: the RBF
+// forward's tiles whose squared differences are summed directly, RBF backwards
+// without a workspace, M or D past 2^24 in a backward, and forwards of more
+// tiles than a launch holds.
 //
 //  * Forward: a 64 x 64 tile of outputs per step, 256 threads, a 4 x 4
 //    block per thread; features staged through LDS 16 at a time, k-major,

@@ -106,8 +106,8 @@ def test_rbf_workspace_plan():
     assert lib.rbf_backward_workspace_bytes(2048, 2048, 64) == 2 * 16 * 2048 * 65 * 4
     assert lib.rbf_backward_workspace_bytes(8192, 8192, 64) == 2 * 32 * 8192 * 65 * 4
     assert lib.rbf_backward_workspace_bytes(64, 64, 64) == 2 * 64 * 65 * 4
-    # other feature widths use the generic kernels: each side's walk in
-    # slices, 64-aligned, about 1024 workgroups a side.  4096^2, D = 32: 64
+    # other feature widths report what the general kernels' slices need, or
+    # the split kernels where that is more: each side's walk in slices, 64-aligned, about 1024 workgroups a side.  4096^2, D = 32: 64
     # row tiles x 1 feature pass -> 16 slices of 256, each a [rows, D]
     # partial plus a [rows] partial sum, for both sides
     assert lib.rbf_backward_workspace_bytes(4096, 4096, 32) == 2 * 16 * 4096 * 33 * 4
@@ -266,7 +266,7 @@ def test_cosine_sim_argument_validation_without_gpu():
     # D = 64 fast path: partial (dS . bh) [nRJ][N][64] + (dS^T . ah) [nRI][M][64], no sums;
     # 4096^2 -> 16 x 16 regions of 256
     assert lib.cosine_sim_backward_workspace_bytes(4096, 4096, 64) == 2 * 16 * 4096 * 64 * 4
-    assert lib.cosine_sim_backward_workspace_bytes(10, 20, 100) == (10 + 20) * 100 * 4  # generic
+    assert lib.cosine_sim_backward_workspace_bytes(10, 20, 100) == (10 + 20) * 100 * 4
     assert lib.cosine_sim_backward_workspace_bytes(0, 20, 64) == 0
     need = lib.cosine_sim_backward_workspace_bytes(64, 64, 64)
     st = lib.cosine_sim_backward_f32(fake, fake, fake, fake, fake, fake, fake, 64, 64, 64, fake,

@@ -4,8 +4,7 @@ atol = rtol = 1e-3.
 
 Workloads: A, B ~ N(0,1), dS ~ N(0,1); N = M = 2048 (the reference default)
 for two seeds and 4096 for one, forward S, the inverse norms and backward
-dA, dB; ragged shapes, the generic path (D != 64, misaligned rows), zero
-rows, a large eps, empty inputs, invariants (|S| <= 1, S(A, A) has a unit
+dA, dB; ragged shapes, other widths than 64, misaligned rows, zero rows, a large eps, empty inputs, invariants (|S| <= 1, S(A, A) has a unit
 diagonal), argument checks, and the framework's verify_all at the
 reference defaults.
 """
@@ -77,8 +76,7 @@ def test_cosine_square_vs_oracle(n, seed):
 
 @pytest.mark.parametrize("n,m,d", [(1000, 3000, 64), (1, 1, 64), (5, 7, 64), (300, 257, 64),
                                    (129, 65, 32), (200, 150, 100), (64, 64, 1), (3000, 3008, 64),
-                                   # tiled generic kernels: ragged tiles, feature chunks and
-                                   # passes, the backward's walks in several slices
+                                   # ragged tiles, feature chunks and passes
                                    (1000, 1000, 32), (257, 65, 128), (300, 129, 200), (70, 1500, 3)])
 def test_cosine_shapes(n, m, d):
     announce(f"cosine_sim N={n} M={m} D={d}")
@@ -86,8 +84,8 @@ def test_cosine_shapes(n, m, d):
     _check(A, B, dS)
 
 
-def test_cosine_generic_zero_rows():
-    announce("cosine_sim generic path, zero rows, D=48")
+def test_cosine_zero_rows_other_width():
+    announce("cosine_sim zero rows, D=48")
     A, B, dS = _inputs(500, 400, 48, 9)
     A[3] = 0.0
     B[17] = 0.0
@@ -104,7 +102,7 @@ def test_cosine_zero_rows_and_large_eps():
 
 
 def test_cosine_misaligned_rows():
-    announce("cosine_sim misaligned A (generic path)")
+    announce("cosine_sim misaligned A")
     A, B, dS = _inputs(130, 90, 64, 8)
     buf = torch.empty(A.numel() + 1, device="cuda")
     buf[1:].copy_(A.reshape(-1).cuda())

@@ -247,8 +247,8 @@ def test_rbf_graph_replays_with_new_inputs():
 
 @pytest.mark.parametrize("b,d", [(512, 4096), (300, 1000)])
 def test_layernorm_graph_replays_with_new_inputs(b, d):
-    """LayerNorm forward and backward (row kernels and the column sums; the
-    generic path at D = 1000) captured once and replayed on new inputs: every
+    """LayerNorm forward and backward (row kernels and the column sums; a
+    width of no whole wave at D = 1000) captured once and replayed on new inputs: every
     replay equals an eager call bit for bit and matches the float64 oracle."""
     announce(f"layernorm graph capture [{b},{d}]")
     from cases.layernorm import op

@@ -1,7 +1,7 @@
 """L2-norm-scale parity on the GPU (through the HIP library) against the
 float64 oracle at atol = rtol = 1e-3: the reference default [16384, 1024]
 and the LayerNorm acceptance shape [8192, 4096] (X, g, dY ~ N(0, 1)), every
-row-cached width class, the generic path (odd D, misaligned X, D > 8192),
+row-cached width class, odd D, misaligned X, D > 16384 (generic kernels),
 zero rows, a large eps, an empty batch, deterministic dg, and the
 framework's verify_all at the reference defaults."""
 

@@ -1,7 +1,7 @@
 """LayerNorm parity on the GPU (through the HIP library) against the float64
 oracle at atol = rtol = 1e-3: the acceptance workload x [8192, 4096]
-(gamma = 1 + 0.1 N, beta = 0.1 N), every row-cached width class, the generic
-path (odd D, misaligned pointers, D > 8192), empty batches, and the
+(gamma = 1 + 0.1 N, beta = 0.1 N), every row-cached width class, odd D,
+misaligned pointers, D > 16384 (generic kernels), empty batches, and the
 framework's verify_all against the case's reference."""
 
 import numpy as np

@@ -101,3 +101,49 @@ def test_cosine_forward_more_tiles_than_a_launch():
         ref = (b * inv[:, None]) @ (a[0].double() / (a.double().norm() + 1e-8))
         assert float((S[0, s].double() - ref).norm() / ref.norm()) <= 2.0 ** -21
         assert float((inv_b[s].double() - inv).norm() / inv.norm()) <= 2.0 ** -21
+
+
+# more columns than the split backwards take: the general kernels, one side's
+# walk in slices and the other's whole
+@pytest.mark.parametrize("n", [1, 70])
+def test_rbf_backward_many_columns(n):
+    m, d, gamma = (1 << 24) + 101, 2, 0.25
+    announce(f"rbf backward n={n} m={m} d={d}")
+    from cases.rbf import op
+    X, Y, G, K = _rows(n, d, 1), _rows(m, d, 2), _rows(n, m, 3), _rows(n, m, 4).sigmoid_()
+    dX, dY = op.rbf_backward(X, Y, G, K, gamma)
+    acc = torch.zeros(n, d + 1, dtype=torch.float64, device="cuda")
+    for c in range(0, m, 1 << 20):
+        s = slice(c, min(c + (1 << 20), m))
+        W, y = G[:, s].double() * K[:, s].double(), Y[s].double()
+        acc[:, d] += W.sum(1)
+        acc[:, :d] += W @ y
+        wt = W.t().contiguous()
+        ref = -2 * gamma * (W.sum(0)[:, None] * y - wt @ X.double())
+        assert float((dY[s].double() - ref).norm() / ref.norm()) <= 2.0 ** -24 * (4 + math.sqrt(n))
+    ref = -2 * gamma * (acc[:, d:] * X.double() - acc[:, :d])
+    # a slice is a sequential sum of 16400 columns, of which there are 1024
+    assert float((dX.double() - ref).norm() / ref.norm()) <= 2.0 ** -24 * (4 + math.sqrt(m / 1024))
+
+
+@pytest.mark.parametrize("n", [1, 70])
+def test_cosine_backward_many_columns(n):
+    m, d = (1 << 24) + 101, 2
+    announce(f"cosine backward n={n} m={m} d={d}")
+    from cases.cosine_sim import op
+    A, B, G = _rows(n, d, 1), _rows(m, d, 2), _rows(n, m, 3)
+    ia, ib = (1 / t.double().norm(dim=1) for t in (A, B))
+    dA, dB = op.cos_backward(A, B, ia.float(), ib.float(), G)
+    ah, acc = A.double() * ia[:, None], torch.zeros(n, d, dtype=torch.float64, device="cuda")
+    for c in range(0, m, 1 << 20):
+        s = slice(c, min(c + (1 << 20), m))
+        w, bh = G[:, s].double(), B[s].double() * ib[s, None]
+        acc += w @ bh
+        part = w.t().contiguous() @ ah
+        ref = ib[s, None] * (part - (bh * part).sum(1, keepdim=True) * bh)
+        # the projection leaves one of two dimensions: its error is the contraction's
+        scale = (ib[s, None] * part).norm()
+        assert float((dB[s].double() - ref).norm() / scale) <= 2.0 ** -24 * (8 + math.sqrt(n))
+    ref = ia[:, None] * (acc - (ah * acc).sum(1, keepdim=True) * ah)
+    assert float((dA.double() - ref).norm() / (ia[:, None] * acc).norm()) <= \
+        2.0 ** -24 * (8 + math.sqrt(m / 1024))

@@ -4,7 +4,7 @@ autograd op) against the float64 oracle, at atol = rtol = 1e-3.
 Workloads follow the acceptance configs (X, Y ~ N(0,1)/8, gamma = 0.5,
 dK ~ N(0,1)): N = M = 2048, 4096 and 8192 for seeds 0-4 (the reference
 protocol's seeds), with size-independent identities at 8192; then ragged and edge shapes, the
-generic (D != 64, misaligned) path, empty inputs, gamma = 0, NaN inputs, the committed
+other widths and misaligned rows, empty inputs, gamma = 0, NaN inputs, the committed
 fixtures written by the reference's own CPU loops, and the framework's
 verify_all against the case's reference.
 """
@@ -109,17 +109,17 @@ def test_rbf_ragged_shapes(n, m):
 
 
 @pytest.mark.parametrize("d", [1, 3, 32, 100])
-def test_rbf_generic_feature_dims(d):
-    announce(f"rbf generic D={d}")
+def test_rbf_feature_dims(d):
+    announce(f"rbf D={d}")
     _check_full(*_inputs(70, 45, d, d, scale=1.0 / np.sqrt(d)), 0.5)
 
 
-# the tiled generic kernels: ragged tile edges on both sides, feature chunks
-# of 16 (forward) and passes of 64 (backward) with ragged ends
+# D != 64: ragged tile edges on both sides, feature chunks of 16 (forward) and
+# passes of 64 (backward) with ragged ends
 @pytest.mark.parametrize("n,m,d", [(130, 200, 16), (257, 65, 128), (1000, 1000, 32),
                                    (64, 64, 65), (300, 129, 200)])
-def test_rbf_generic_tiled_shapes(n, m, d):
-    announce(f"rbf generic n={n} m={m} D={d}")
+def test_rbf_tiled_shapes(n, m, d):
+    announce(f"rbf n={n} m={m} D={d}")
     _check_full(*_inputs(n, m, d, n + m + d, scale=1.0 / np.sqrt(d)), 0.5)
 
 
@@ -178,7 +178,7 @@ def test_rbf_empty_inputs():
     assert torch.all(dX == 0) and dY.shape == (0, 64)
 
 
-def test_rbf_misaligned_inputs_use_generic_path():
+def test_rbf_misaligned_inputs():
     announce("rbf misaligned")
     X, Y, G = _inputs(40, 24, 64, 5)
     buf = torch.empty(40 * 64 + 1, device="cuda")
@@ -234,11 +234,10 @@ def test_rbf_c_abi_direct():
         assert st != 0 and b"workspace" in lib.rbf_last_error()
 
 
-def test_rbf_generic_backward_split_and_whole():
-    """D != 64: the generic backward cuts its walks into slices when the
-    workspace holds their partial sums, and runs them whole with no
-    workspace; both match the oracle."""
-    announce("rbf generic backward, sliced and whole, 1500 x 700, D=32")
+def test_rbf_backward_with_and_without_workspace():
+    """D != 64: the split kernels with their workspace, the general kernels'
+    whole walks with none; both match the oracle."""
+    announce("rbf backward with and without workspace, 1500 x 700, D=32")
     lib = _op()._lib()
     n, m, d = 1500, 700, 32
     X, Y, G = _inputs(n, m, d, 5, scale=1.0 / np.sqrt(d))
@@ -251,7 +250,7 @@ def test_rbf_generic_backward_split_and_whole():
     ws = torch.empty(ws_bytes // 4, device="cuda")
     Kr = orbf.forward_f64(X.numpy(), Y.numpy(), 0.5)
     dXr, dYr = orbf.backward_f64(X.numpy(), Y.numpy(), G.numpy(), Kr, 0.5)
-    for name, ptr, nbytes in (("sliced", capi.ptr(ws), ws_bytes), ("whole", None, 0)):
+    for name, ptr, nbytes in (("split", capi.ptr(ws), ws_bytes), ("whole", None, 0)):
         dX = torch.empty_like(Xd)
         dY = torch.empty_like(Yd)
         st = lib.rbf_backward_f32(capi.ptr(Xd), capi.ptr(Yd), capi.ptr(Gd), capi.ptr(K),
