@@ -12,8 +12,8 @@
 //    with kappa = gamma log2(e): at D = 64 on bf16 splits of the fp32 rows
 //    (csrc/pairwise_split.h), else in 64 bits (rbf_fwd_kernel), at any D and
 //    alignment.  Tiles whose distances that form would round too coarsely
-//    (split_norm_max, f64_norm_max) sum the squared differences directly, on
-//    SIMT tiles.
+//    (split_norm_max, f64_norm_max) go from the splits to 64 bits or to the
+//    squared differences summed directly on SIMT tiles, from 64 bits to those.
 //  * Backward: one pass over dK and K per 64 features.  Workgroups own
 //    regions of W = dK o K and write raw partial contractions W . Y and
 //    W^T . X and partial row and column sums of W to workspace slots, on the
@@ -56,24 +56,6 @@ struct RbfGenFwd {
   __device__ __forceinline__ float out(float s) const { return expf(-gamma * s); }
 };
 
-// Forward policy on the splits: the row term is -kappa |x|^2, the column term
-// |y|^2, and K = exp2(min(2 kappa x.y - kappa (|x|^2 + |y|^2), 0)); the clamp
-// keeps K <= 1 when the distance cancels to a tiny negative value.
-struct RbfFwdOp {
-  float neg_kappa;  // -gamma log2(e)
-  float gamma;
-  float norm_max;
-  static constexpr bool kScale = false, kDirect = true;
-  __device__ __forceinline__ float row(float sx) const { return neg_kappa * sx; }
-  __device__ __forceinline__ float col(float sy) const { return sy; }
-  __device__ __forceinline__ float out(float dot, float rt, float ct) const {
-    float t = fmaf(-2.f * neg_kappa, dot, fmaf(neg_kappa, ct, rt));
-    t = t > 0.f ? 0.f : t;  // squared distance >= 0; NaN passes through
-    return __builtin_amdgcn_exp2f(t);
-  }
-  __device__ __forceinline__ RbfGenFwd direct() const { return RbfGenFwd{gamma}; }
-};
-
 // Backward policy: W = dK o K, raw X / Y rows, row and column sums of W.
 struct RbfBwdOp {
   static constexpr bool kProduct = true, kScale = false, kSums = true;
@@ -93,6 +75,9 @@ typedef float f32x2_u __attribute__((ext_vector_type(2), aligned(4)));
 // features of a row, k + 4 h .. + 3, straight from global memory (the next 16
 // features are in flight while these are multiplied), and the norms are summed
 // from the same registers.
+// A tile with a norm past norm_max, or one that is not finite, sums the
+// squared differences directly; a wave that sees so in the first features
+// skips the rest.
 // Bound by the matrix instruction, which takes 120 cycles on a full chip (42
 // TFLOP/s).  Against the squared differences summed in fp32 on SIMT tiles:
 // 53 -> 39 us at 3000 x 2500 x 100, 20 -> 9.2 at 1000 x 1000 x 100, 39 -> 33
@@ -101,14 +86,19 @@ typedef float f32x2_u __attribute__((ext_vector_type(2), aligned(4)));
 // x 100, but a pair of rows 1 % apart is off by 7e-8 at gamma |x|^2 = 0.5 and
 // 6e-7 at 4 there, against 2e-8 directly.)
 constexpr int kFwdTile = 64;
-__global__ __launch_bounds__(256, 2) void rbf_fwd_kernel(
-    const float* __restrict__ X, const float* __restrict__ Y, float* __restrict__ K, int N, int M,
-    int D, double neg_kappa, double norm_max, float gamma, int n_jt) {
-  __shared__ __attribute__((aligned(16))) nl2k::pairwise::SimtTile simt;
+struct RbfF64 {
+  double neg_kappa;  // -gamma log2(e)
+  double norm_max;
+  float gamma;
+};
+__device__ __forceinline__ void rbf_f64_tile(nl2k::pairwise::SimtTile& simt,
+                                             const float* __restrict__ X,
+                                             const float* __restrict__ Y, float* __restrict__ K,
+                                             int N, int M, int D, int i0, int j0,
+                                             const RbfF64& op) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int n = lane & 15, h = lane >> 4;
-  const int i0 = (int)(blockIdx.x / n_jt) * kFwdTile, j0 = (int)(blockIdx.x % n_jt) * kFwdTile;
   const int ib = i0 + (wave >> 1) * 32, j = j0 + (wave & 1) * 32 + 2 * n;
   const float* src[4];  // rows ib + n, + 16 of X, rows j, j + 1 of Y
 #pragma unroll
@@ -142,6 +132,11 @@ __global__ __launch_bounds__(256, 2) void rbf_fwd_kernel(
 #pragma unroll
     for (int s = 0; s < 4; ++s) nxt[s] = nl2k::pairwise::load4_u(src[s] + k + 4 * h);
   };
+  bool direct = false;
+  auto check_norms = [&] {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) direct |= !(nsq[s] <= op.norm_max);
+  };
   const int whole = D & ~15;
   if (whole > 0) load(0);
   for (int k = 0; k < whole; k += 16) {
@@ -151,6 +146,10 @@ __global__ __launch_bounds__(256, 2) void rbf_fwd_kernel(
     if (k + 16 < whole) load(k + 16);
 #pragma unroll
     for (int u = 0; u < 4; ++u) step({cur[0][u], cur[1][u], cur[2][u], cur[3][u]});
+    if (k == 0) {
+      check_norms();
+      if (__any(direct)) break;
+    }
   }
   for (int k = whole; k < D; k += 4) {  // the last features, four at a time: zeros past D
     float x[4];
@@ -160,16 +159,15 @@ __global__ __launch_bounds__(256, 2) void rbf_fwd_kernel(
     for (int s = 0; s < 4; ++s) x[s] = k + h < D ? x[s] : 0.f;
     step(x);
   }
-  bool direct = false;
 #pragma unroll
   for (int s = 0; s < 4; ++s) {  // over the row's four lanes
     nsq[s] += __shfl_xor(nsq[s], 16, 64);
     nsq[s] += __shfl_xor(nsq[s], 32, 64);
-    direct |= !(nsq[s] <= norm_max);
   }
+  check_norms();
   if (__syncthreads_or(direct)) {
     nl2k::pairwise::simt_fwd_tile(simt, X, Y, K, (int64_t)N, (int64_t)M, (int64_t)D, (int64_t)i0,
-                                  (int64_t)j0, RbfGenFwd{gamma});
+                                  (int64_t)j0, RbfGenFwd{op.gamma});
     return;
   }
 #pragma unroll
@@ -182,7 +180,7 @@ __global__ __launch_bounds__(256, 2) void rbf_fwd_kernel(
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
         const double d2 = fma(-2., acc[a][b][r], nx + nsq[2 + b]);
-        o[b] = exp2f((float)(neg_kappa * fmax(d2, 0.)));
+        o[b] = exp2f((float)(op.neg_kappa * fmax(d2, 0.)));
       }
       if (i >= N) continue;
       float* p = K + (size_t)i * M + j;
@@ -192,6 +190,45 @@ __global__ __launch_bounds__(256, 2) void rbf_fwd_kernel(
         p[0] = o[0];
     }
 }
+
+__global__ __launch_bounds__(256, 2) void rbf_fwd_kernel(const float* __restrict__ X,
+                                                         const float* __restrict__ Y,
+                                                         float* __restrict__ K, int N, int M,
+                                                         int D, RbfF64 op, int n_jt) {
+  __shared__ __attribute__((aligned(16))) nl2k::pairwise::SimtTile simt;
+  rbf_f64_tile(simt, X, Y, K, N, M, D, (int)(blockIdx.x / n_jt) * kFwdTile,
+               (int)(blockIdx.x % n_jt) * kFwdTile, op);
+}
+
+// Forward policy on the splits: the row term is -kappa |x|^2, the column term
+// |y|^2, and K = exp2(min(2 kappa x.y - kappa (|x|^2 + |y|^2), 0)); the clamp
+// keeps K <= 1 when the distance cancels to a tiny negative value.
+struct RbfFwdOp {
+  float neg_kappa;  // -gamma log2(e)
+  float norm_max;
+  RbfF64 f64;  // for tiles with larger norms
+  static constexpr bool kScale = false, kDirect = true;
+  __device__ __forceinline__ float row(float sx) const { return neg_kappa * sx; }
+  __device__ __forceinline__ float col(float sy) const { return sy; }
+  __device__ __forceinline__ float out(float dot, float rt, float ct) const {
+    float t = fmaf(-2.f * neg_kappa, dot, fmaf(neg_kappa, ct, rt));
+    t = t > 0.f ? 0.f : t;  // squared distance >= 0; NaN passes through
+    return __builtin_amdgcn_exp2f(t);
+  }
+  // Workgroups of 128 x 128 have the registers for 64 bits (4096^2: 63-72 us, 87-99
+  // with the sum on SIMT tiles, two of them a CU); in those of 64 x 64 they cost
+  // the split itself (17.2 -> 18.1 us at 3000^2).
+  template <int TB>
+  __device__ __forceinline__ void direct(nl2k::pairwise::SimtTile& t, const float* X,
+                                         const float* Y, float* K, int N, int M, int D, int i0,
+                                         int j0) const {
+    if constexpr (TB == 128)
+      rbf_f64_tile(t, X, Y, K, N, M, D, i0, j0, f64);
+    else
+      nl2k::pairwise::simt_fwd_tile(t, X, Y, K, (int64_t)N, (int64_t)M, (int64_t)D, (int64_t)i0,
+                                    (int64_t)j0, RbfGenFwd{f64.gamma});
+  }
+};
 
 // ------------------------------------------------------------------ backward
 // One side of the backward: its own rows A and their gradient, the other
@@ -368,12 +405,13 @@ bool takes_split_forward(int64_t D, const float* X, const float* Y) {
 }
 
 // Largest squared row norm whose distances come from norms and products, |x|^2
-// + |y|^2 - 2 x.y; a tile with a larger one (or with a norm that is not
-// finite) sums the squared differences directly.  The former leaves an error
-// in the distance of about 2^-24 of |x|^2 + |y|^2 on the splits and 2^-52 in
-// 64 bits, whatever the distance is, and gamma carries it into K: a few 1e-7
-// at gamma |x|^2 = 4, and a quarter of K's last bit at gamma |x|^2 = 2^24.  A
-// negative or NaN gamma always sums directly.
+// + |y|^2 - 2 x.y.  That leaves an error in the distance of about 2^-24 of |x|^2
+// + |y|^2 on the splits and 2^-52 in 64 bits, whatever the distance is, and gamma
+// carries it into K: a few 1e-7 at gamma |x|^2 = 4, and a quarter of K's last
+// bit at gamma |x|^2 = 2^24.  A tile on the splits with a larger norm goes to 64
+// bits or to the direct sum (RbfFwdOp::direct), one in 64 bits with a larger
+// one, or one that is not finite, to the direct sum.
+// A negative or NaN gamma always sums directly.
 inline float split_norm_max(float gamma) {
   if (!(gamma >= 0.f)) return -1.f;
   return gamma <= 4e-30f ? 1e30f : 4.f / gamma;
@@ -555,19 +593,19 @@ int rbf_forward_f32(const float* X, const float* Y, float* K, int64_t N,
   if (!X || !Y || !K)
     return nl2k::fail(NL2K_ERR_NULL, "rbf_forward_f32: X, Y and K must be non-null");
 
+  const RbfF64 op = {-gamma * kLog2e, f64_norm_max(gamma), gamma};
   if (takes_split_forward(D, X, Y)) {
     const nl2k::pairwise::SplitFwdPlan fp = nl2k::pairwise::plan_split_forward(N, M, D);
     if (fp.n_jt > 0)
       return nl2k::pairwise::launch_fwd_split(
-          fp, X, Y, K, N, M, D, RbfFwdOp{(float)(-gamma * kLog2e), gamma, split_norm_max(gamma)},
-          nullptr, nullptr, stream, "rbf_forward_f32");
+          fp, X, Y, K, N, M, D, RbfFwdOp{(float)op.neg_kappa, split_norm_max(gamma), op}, nullptr,
+          nullptr, stream, "rbf_forward_f32");
   }
   const int64_t n_jt = nl2k::ceil_div(M, (int64_t)kFwdTile);
   const int64_t n_tiles = nl2k::ceil_div(N, (int64_t)kFwdTile) * n_jt;
   if (std::max(std::max(N, M), D) <= INT32_MAX - 1024 && n_tiles <= nl2k::max_blocks(256)) {
     hipLaunchKernelGGL(rbf_fwd_kernel, dim3((unsigned)n_tiles), dim3(256), 0, stream, X, Y, K,
-                       (int)N, (int)M, (int)D, -gamma * kLog2e, f64_norm_max(gamma), gamma,
-                       (int)n_jt);
+                       (int)N, (int)M, (int)D, op, (int)n_jt);
     return nl2k::check_launch("rbf_forward_f32");
   }
   const int64_t ntiles = nl2k::ceil_div(N, (int64_t)nl2k::pairwise::kGT) *

@@ -96,8 +96,8 @@ __device__ constexpr int kTermB[kProducts] = {0, 2, 1, 0, 1, 0};
 //                                   the contraction, and the scales written
 //                                   to rowv [N] / colv [M]
 //   static constexpr bool kDirect   a tile one of whose rows has a squared
-//                                   norm past Op::norm_max is summed directly
-//                                   (Op::Direct, the SIMT tile) instead
+//                                   norm past Op::norm_max is left to
+//                                   Op::direct<TB>, 64 x 64 outputs at a time
 //   float inv(float nsq)
 //   float row(float nsq) / col(float nsq)     epilogue terms
 //   float out(float dot, float rt, float ct)  the output entry
@@ -131,7 +131,7 @@ struct FwdLds {
 };
 
 template <class Op, int TB>
-__global__ __launch_bounds__(256, 2) void pair_fwd_split_kernel(
+__global__ __launch_bounds__(256, TB == 128 ? 2 : 4) void pair_fwd_split_kernel(
     const float* __restrict__ X, const float* __restrict__ Y, float* __restrict__ out, int N,
     int M, int D, Op op, int n_jt, float* __restrict__ rowv, float* __restrict__ colv) {
   __shared__ __attribute__((aligned(16))) FwdLds<TB> lds;
@@ -229,7 +229,7 @@ __global__ __launch_bounds__(256, 2) void pair_fwd_split_kernel(
     for (int b = 0; b < kWB; ++b) acc[a][b] = zero4();
 
   // Whether one of the tile's rows, as far as it has been summed, has too
-  // large a norm: the tile is then summed directly.
+  // large a norm: the tile is then left to Op::direct.
   auto too_large = [&] {
     bool big = false;
     if constexpr (Op::kDirect) {
@@ -245,8 +245,7 @@ __global__ __launch_bounds__(256, 2) void pair_fwd_split_kernel(
       for (int a = 0; a < TB; a += kGT)
         for (int b = 0; b < TB; b += kGT)
           if (i0 + a < N && j0 + b < M)
-            simt_fwd_tile(lds.simt, X, Y, out, (int64_t)N, (int64_t)M, (int64_t)D,
-                          (int64_t)i0 + a, (int64_t)j0 + b, op.direct());
+            op.template direct<TB>(lds.simt, X, Y, out, N, M, D, i0 + a, j0 + b);
     }
   };
   bool direct = false;  // workgroup-uniform
