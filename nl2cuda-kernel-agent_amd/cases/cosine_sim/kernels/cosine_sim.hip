@@ -65,30 +65,18 @@ struct CosBwdOp {
 // not finite.
 constexpr int kKeep = 4;
 
-// One side of the backward: its own rows A, their inverse norms and gradient,
-// the other side's rows B, entry (r, o) of dS at r own + o other.
-struct ReduceSide {
-  const float *P, *A, *inv, *B, *inv_b;
-  float* out;
-  int64_t rows, others;
-  size_t own, other;
-  int slots;
-};
-
 template <int V, int L, bool SPLIT>
-__device__ __forceinline__ void project_row(const ReduceSide& side, const float* __restrict__ dS,
-                                            int64_t r, int D, int lane) {
+__device__ __forceinline__ void project_row(
+    const float* __restrict__ P, const float* __restrict__ A, const float* __restrict__ inv,
+    float* __restrict__ out, int64_t rows, int64_t r, int D, int slots, int lane,
+    const float* __restrict__ dS, size_t own, size_t other,  // entry (r, o): r own + o other
+    const float* __restrict__ B, const float* __restrict__ inv_b, int64_t others) {
   typedef float vec __attribute__((ext_vector_type(V), aligned(4)));
-  const float* __restrict__ P = side.P;
-  const float* __restrict__ A = side.A;
-  float* out = side.out;
-  const int64_t rows = side.rows;
-  const int slots = side.slots;
   const int per = D / V;
   const int64_t stride = rows * (int64_t)D;
   const float* p = P + r * D;
   const float* a = A + r * D;
-  const float sc = side.inv[r];
+  const float sc = inv[r];
   auto partial = [&](int e) {
     auto at = [&](int s) { return *reinterpret_cast<const vec*>(p + s * stride + (int64_t)e * V); };
     vec a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
@@ -124,34 +112,38 @@ __device__ __forceinline__ void project_row(const ReduceSide& side, const float*
   }
   for (int e = lane + L * kKeep; e < per; e += L)
     add(partial(e), *reinterpret_cast<const vec*>(a + (int64_t)e * V));
-  auto over_row = [&](float v) {
+  auto over_row = [&] {
 #pragma unroll
-    for (int off = 1; off < L; off <<= 1) v += __shfl_xor(v, off, 64);
-    return v;
+    for (int off = 1; off < L; off <<= 1) {
+      dot += __shfl_xor(dot, off, 64);
+      nn += __shfl_xor(nn, off, 64);
+    }
   };
-  dot = over_row(dot);
-  const float nrm = sqrtf(over_row(nn));
+  over_row();
   auto store = [&](int e, const vec& acc, const vec& av, float coef) {
     *reinterpret_cast<vec*>(out + r * D + (int64_t)e * V) = sc * acc - coef * (av * sc);
   };
-  if (SPLIT && !(fabsf(dot) < INFINITY)) {  // a partial is not finite, or dot overflowed
-    dot = 0.f;
+  // a partial that is not finite, or a dot that overflowed
+  if (SPLIT && __builtin_expect(!(fabsf(dot) < INFINITY), 0)) {
+    dot = nn = 0.f;
+#pragma unroll 1
     for (int e = lane; e < per; e += L) {
       vec acc;
       float sum;
-      nl2k::pairwise::direct_sums<CosBwdOp>(dS, nullptr, (size_t)r * side.own, side.other,
-                                            side.B + (int64_t)e * V, side.inv_b, side.others, D,
-                                            acc, sum);
+      nl2k::pairwise::direct_sums<CosBwdOp>(dS, nullptr, (size_t)r * own, other,
+                                            B + (int64_t)e * V, inv_b, others, D, acc, sum);
       *reinterpret_cast<vec*>(out + r * D + (int64_t)e * V) = acc;  // read back below
       add(acc, *reinterpret_cast<const vec*>(a + (int64_t)e * V));
     }
-    dot = over_row(dot);
-    const float coef = nrm > 0.f ? dot / nrm : 0.f;
+    over_row();
+    const float nrm = sqrtf(nn), coef = nrm > 0.f ? dot / nrm : 0.f;
+#pragma unroll 1
     for (int e = lane; e < per; e += L)
       store(e, *reinterpret_cast<const vec*>(out + r * D + (int64_t)e * V),
             *reinterpret_cast<const vec*>(a + (int64_t)e * V), coef);
     return;
   }
+  const float nrm = sqrtf(nn);
   const float coef = nrm > 0.f ? dot / nrm : 0.f;
 #pragma unroll
   for (int k = 0; k < kKeep; ++k)
@@ -163,19 +155,22 @@ __device__ __forceinline__ void project_row(const ReduceSide& side, const float*
 // Both outputs in one launch: block b < bx handles dA, the rest dB.  A row's
 // lanes stay together: every lane of a group has the same row.
 template <int V, int L, bool SPLIT>
-__global__ __launch_bounds__(256) void cos_bwd_reduce_kernel(ReduceSide x, ReduceSide y,
-                                                             const float* __restrict__ dS, int D,
-                                                             int bx) {
+__global__ __launch_bounds__(256) void cos_bwd_reduce_kernel(
+    const float* __restrict__ Px, const float* __restrict__ A,
+    const float* __restrict__ inv_a, float* __restrict__ dA, int64_t N, int sx,
+    const float* __restrict__ Py, const float* __restrict__ B,
+    const float* __restrict__ inv_b, float* __restrict__ dB, int64_t M, int sy,
+    const float* __restrict__ dS, int D, int bx) {
   constexpr int kRows = 256 / L;
   const int b = (int)blockIdx.x;
   const int lane = threadIdx.x % L, g = threadIdx.x / L;
   if (b < bx) {
-    for (int64_t r = (int64_t)b * kRows + g; r < x.rows; r += (int64_t)bx * kRows)
-      project_row<V, L, SPLIT>(x, dS, r, D, lane);
+    for (int64_t r = (int64_t)b * kRows + g; r < N; r += (int64_t)bx * kRows)
+      project_row<V, L, SPLIT>(Px, A, inv_a, dA, N, r, D, sx, lane, dS, (size_t)M, 1, B, inv_b, M);
   } else {
     const int64_t nb = (int)gridDim.x - bx;
-    for (int64_t r = (int64_t)(b - bx) * kRows + g; r < y.rows; r += nb * kRows)
-      project_row<V, L, SPLIT>(y, dS, r, D, lane);
+    for (int64_t r = (int64_t)(b - bx) * kRows + g; r < M; r += nb * kRows)
+      project_row<V, L, SPLIT>(Py, B, inv_b, dB, M, r, D, sy, lane, dS, 1, (size_t)M, A, inv_a, N);
   }
 }
 
@@ -280,9 +275,8 @@ int reduce(const float* px, const float* py, int64_t sx, int64_t sy, const float
       vec ? (wide ? &cos_bwd_reduce_kernel<4, 64, SPLIT> : &cos_bwd_reduce_kernel<4, 16, SPLIT>)
           : (wide ? &cos_bwd_reduce_kernel<1, 64, SPLIT> : &cos_bwd_reduce_kernel<1, 16, SPLIT>);
   const int bx = grid_for(N, wide ? 4 : 16, 2048), by = grid_for(M, wide ? 4 : 16, 2048);
-  const ReduceSide x = {px, A, inv_a, B, inv_b, dA, N, M, (size_t)M, 1, (int)sx};
-  const ReduceSide y = {py, B, inv_b, A, inv_a, dB, M, N, 1, (size_t)M, (int)sy};
-  hipLaunchKernelGGL(kernel, dim3(bx + by), dim3(256), 0, stream, x, y, dS, (int)D, bx);
+  hipLaunchKernelGGL(kernel, dim3(bx + by), dim3(256), 0, stream, px, A, inv_a, dA, N, (int)sx,
+                     py, B, inv_b, dB, M, (int)sy, dS, (int)D, bx);
   return nl2k::check_launch(who);
 }
 

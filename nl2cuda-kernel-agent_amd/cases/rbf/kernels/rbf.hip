@@ -287,7 +287,7 @@ __device__ __forceinline__ void reduce_side(const ReduceSide& side, const float*
       for (int v = 0; v < V; ++v) finite &= fabsf(acc[v]) < INFINITY;
       sum *= nl2k::pairwise::kSumUnscale;
       acc *= nl2k::pairwise::kPartialUnscale;
-      if (!finite)
+      if (__builtin_expect(!finite, 0))
         nl2k::pairwise::direct_sums<RbfBwdOp>(dK, K, (size_t)r * side.own, side.other,
                                               side.B + (size_t)(e - r * per) * V, nullptr,
                                               side.others, D, acc, sum);

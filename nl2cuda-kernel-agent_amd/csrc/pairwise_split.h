@@ -801,6 +801,7 @@ __device__ __forceinline__ void direct_sums(const float* __restrict__ dK,
                                             int64_t D, Vec& acc, float& sum) {
   constexpr int V = sizeof(Vec) / sizeof(float);
   double a[V] = {}, s = 0.;
+#pragma unroll 1  // rarely taken: little code beside the callers' own
   for (int64_t o = 0; o < others; ++o) {
     float w = dK[at + o * step];
     if constexpr (Op::kProduct) w *= K[at + o * step];
